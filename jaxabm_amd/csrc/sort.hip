@@ -9,9 +9,10 @@
 // (birthday bound), so the sort must be stable: an LSD radix sort whose
 // per-tile ranks follow the input order is.
 //
-// Per 8-bit digit pass: (1) tile histograms, (2) one exclusive scan over
-// digit-major / tile-minor counts, (3) stable scatter, ranking within a
-// 64-wide wavefront by ballot matching on the digit bits.
+// Per 8-bit digit pass: (1) tile histograms, (2) per digit, an exclusive scan
+// of its tile counts and their total, (3) stable scatter: each tile scans the
+// 256 totals itself, and ranks within a 64-wide wavefront by ballot matching
+// on the digit bits.
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
@@ -20,7 +21,7 @@
 namespace abm {
 
 constexpr int kSortThreads = 256;
-constexpr int kSortRounds = 16;  // items per thread per tile, in rounds
+constexpr int kSortRounds = 8;  // items per thread per tile, in rounds
 constexpr int kTile = kSortThreads * kSortRounds;
 constexpr int kWaves = kSortThreads / 64;
 
@@ -42,36 +43,56 @@ __global__ void __launch_bounds__(kSortThreads)
   hist[(int64_t)threadIdx.x * tiles + blockIdx.x] = cnt[threadIdx.x];
 }
 
-// Exclusive scan of `len` counts by a single block per segment (blockIdx.y).
-__global__ void __launch_bounds__(1024)
-    k_scan_exclusive(uint32_t *__restrict__ data, int64_t len) {
-  data += (int64_t)blockIdx.y * len;
-  __shared__ uint32_t part[1024];
-  const int t = threadIdx.x;
-  int64_t per = (len + 1023) / 1024;
-  int64_t lo = t * per, hi = lo + per < len ? lo + per : len;
-  uint32_t s = 0;
-  for (int64_t i = lo; i < hi; ++i) s += data[i];
-  part[t] = s;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    uint32_t v = t >= off ? part[t - off] : 0u;
-    __syncthreads();
-    part[t] += v;
-    __syncthreads();
+// In place: digit row d = hist[d * tiles ..) becomes its exclusive scan, its
+// sum goes to totals[d]; one wavefront per digit, 64 x kScanLoads counts per
+// round.  The scan across digits is left to the scatter (256 values).  Bound
+// by the round's load latency.  One workgroup scanning all 256 * tiles counts
+// (each thread a contiguous, uncoalesced run) took 107 us a pass at 1,000,000
+// keys, five times the scatter; this takes 4.
+constexpr int kScanLoads = 4;
+
+__global__ void __launch_bounds__(kSortThreads)
+    k_digit_scan(uint32_t *__restrict__ hist, int tiles, uint32_t *__restrict__ totals) {
+  const int lane = threadIdx.x & 63;
+  const int d = blockIdx.x * kWaves + (threadIdx.x >> 6);
+  uint32_t *row = hist + ((int64_t)blockIdx.y * 256 + d) * tiles;
+  uint32_t run = 0;
+  for (int64_t b = 0; b < tiles; b += 64 * kScanLoads) {
+    uint32_t v[kScanLoads];
+#pragma unroll
+    for (int k = 0; k < kScanLoads; ++k) {
+      const int64_t i = b + k * 64 + lane;
+      v[k] = i < tiles ? row[i] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kScanLoads; ++k) {
+      const int64_t i = b + k * 64 + lane;
+      uint32_t inc = v[k];
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(inc, off);
+        if (lane >= off) inc += y;
+      }
+      if (i < tiles) row[i] = run + inc - v[k];
+      run += __shfl(inc, 63);
+    }
   }
-  uint32_t run = t ? part[t - 1] : 0u;
-  for (int64_t i = lo; i < hi; ++i) {
-    uint32_t v = data[i];
-    data[i] = run;
-    run += v;
-  }
+  if (lane == 0) totals[(int64_t)blockIdx.y * 256 + d] = run;
 }
 
+// Stable scatter of one digit.  Wave w of tile b owns items [b kTile + w 64
+// kSortRounds, ..) of the segment, 64 per round, so wave order and round order
+// are input order.  The loads of all rounds are issued together; each wave
+// counts its digits (LDS atomics), one pass over the waves turns the counts
+// into each wave's first position per digit, and from there a wave ranks and
+// stores its rounds alone: three barriers a tile instead of four a round, with
+// one load latency instead of one per round (1,000,000 pairs: 18.8 -> 16.7 us;
+// what is left is the scattered 4-byte stores).
 __global__ void __launch_bounds__(kSortThreads)
     k_digit_scatter(const uint32_t *__restrict__ keys_in,
                     const int32_t *__restrict__ vals_in, int64_t n, int shift,
-                    const uint32_t *__restrict__ offsets, int tiles,
+                    const uint32_t *__restrict__ offsets,
+                    const uint32_t *__restrict__ totals, int tiles,
                     uint32_t *__restrict__ keys_out,
                     int32_t *__restrict__ vals_out) {
   {
@@ -81,42 +102,72 @@ __global__ void __launch_bounds__(kSortThreads)
     keys_out += seg;
     vals_out += seg;
     offsets += (int64_t)blockIdx.y * 256 * tiles;
+    totals += (int64_t)blockIdx.y * 256;
   }
-  __shared__ uint32_t base[256];
-  __shared__ uint32_t wc[kWaves][256];
+  __shared__ uint32_t wpos[kWaves][256];
+  __shared__ uint32_t wsum[kWaves];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  base[t] = offsets[(int64_t)t * tiles + blockIdx.x];
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int64_t tile0 = (int64_t)blockIdx.x * kTile;
+  const int64_t first = (int64_t)blockIdx.x * kTile + (int64_t)wave * 64 * kSortRounds + lane;
+  uint32_t key[kSortRounds];
+  int32_t val[kSortRounds];
+#pragma unroll
   for (int r = 0; r < kSortRounds; ++r) {
-    for (int w = 0; w < kWaves; ++w) wc[w][t] = 0;
-    __syncthreads();
-    const int64_t i = tile0 + (int64_t)r * kSortThreads + t;
-    const bool valid = i < n;
-    uint32_t k = valid ? keys_in[i] : 0u;
-    int32_t v = valid ? vals_in[i] : 0;
-    uint32_t d = (k >> shift) & 255u;
+    const int64_t i = first + r * 64;
+    key[r] = i < n ? keys_in[i] : 0u;
+    val[r] = i < n ? vals_in[i] : 0;
+  }
+  const uint32_t own = offsets[(int64_t)t * tiles + blockIdx.x];
+  const uint32_t total = totals[t];
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) wpos[w][t] = 0;
+  uint32_t inc = total;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = __shfl_up(inc, off);
+    if (lane >= off) inc += y;
+  }
+  if (lane == 63) wsum[wave] = inc;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kSortRounds; ++r)
+    if (first + r * 64 < n) atomicAdd(&wpos[wave][(key[r] >> shift) & 255u], 1u);
+  // digit base: the keys of smaller digits, then this digit's earlier tiles
+  uint32_t pos = own + inc - total;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w)
+    if (w < wave) pos += wsum[w];
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const uint32_t c = wpos[w][t];
+    wpos[w][t] = pos;
+    pos += c;
+  }
+  __syncthreads();
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  volatile uint32_t *mine = wpos[wave];  // this wave's alone from here on
+#pragma unroll
+  for (int r = 0; r < kSortRounds; ++r) {
+    const bool valid = first + r * 64 < n;
+    const uint32_t d = (key[r] >> shift) & 255u;
     uint64_t peers = __ballot(valid);
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
       const bool bit = (d >> b) & 1u;
-      uint64_t m = __ballot(bit);
+      const uint64_t m = __ballot(bit);
       peers &= bit ? m : ~m;
     }
-    const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
-    if (valid && rank == 0) wc[wave][d] = (uint32_t)__popcll(peers);
-    __syncthreads();
     if (valid) {
-      uint32_t pos = base[d] + rank;
-      for (int w = 0; w < wave; ++w) pos += wc[w][d];
-      keys_out[pos] = k;
-      vals_out[pos] = v;
+      const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
+      const uint32_t at = mine[d];
+      // LDS operations of a wave complete in order: every lane has read the
+      // digit's position before its first lane moves it on
+      __builtin_amdgcn_wave_barrier();
+      if (rank == 0) mine[d] = at + (uint32_t)__popcll(peers);
+      keys_out[at + rank] = key[r];
+      vals_out[at + rank] = val[r];
     }
-    __syncthreads();
-    uint32_t add = 0;
-    for (int w = 0; w < kWaves; ++w) add += wc[w][t];
-    base[t] += add;
-    __syncthreads();
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -128,9 +179,10 @@ __global__ void k_iota(int32_t *__restrict__ out, int64_t n) {
 
 // Round r's sort keys: k_0 = key; k_{j+1}, sub_j = split(k_j); bits(sub_r).
 // Segment s = blockIdx.y takes its key at key[s * key_stride].
+// Round 0 also writes the identity the sorts permute, iota[s * n + i] = i.
 __global__ void k_perm_round_bits(const uint32_t *__restrict__ key, int64_t key_stride,
                                   int round, int64_t n, uint32_t *__restrict__ out,
-                                  int mode) {
+                                  int32_t *__restrict__ iota, int mode) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   key += (int64_t)blockIdx.y * key_stride;
@@ -142,14 +194,16 @@ __global__ void k_perm_round_bits(const uint32_t *__restrict__ key, int64_t key_
     k = nk;
   }
   out[i] = bits_at(sub, n, i, mode);
+  if (round == 0) iota[(int64_t)blockIdx.y * n + i] = (int32_t)i;
 }
 
 size_t sort_workspace_bytes(int64_t n, int64_t segs = 1) {
   int64_t tiles = (n + kTile - 1) / kTile;
-  // keys x2, vals x1 (the second value buffer is the caller's), hist
+  // the second key and value buffers, tile histograms, digit totals
   size_t b = 0;
-  b += (size_t)n * (size_t)segs * 4 * 3;
+  b += (size_t)n * (size_t)segs * 4 * 2;
   b += (size_t)tiles * 256 * 4 * (size_t)segs;
+  b += (size_t)256 * 4 * (size_t)segs;
   return (b + 255) & ~(size_t)255;
 }
 
@@ -165,18 +219,19 @@ int radix_sort_pairs(uint32_t *keys, int32_t *vals, int64_t n, void *ws,
   p += (size_t)total * 4;
   int32_t *v2 = (int32_t *)p;
   p += (size_t)total * 4;
-  p += (size_t)total * 4;  // reserved
   uint32_t *hist = (uint32_t *)p;
+  p += (size_t)tiles * 256 * 4 * (size_t)segs;
+  uint32_t *totals = (uint32_t *)p;
   uint32_t *ka = keys, *kb = k2;
   int32_t *va = vals, *vb = v2;
   const dim3 grid((unsigned)tiles, (unsigned)segs);
   for (int shift = 0; shift < 32; shift += 8) {
     hipLaunchKernelGGL(k_digit_hist, grid, dim3(kSortThreads), 0, s, ka, n, shift, hist,
                        tiles);
-    hipLaunchKernelGGL(k_scan_exclusive, dim3(1, (unsigned)segs), dim3(1024), 0, s, hist,
-                       (int64_t)tiles * 256);
+    hipLaunchKernelGGL(k_digit_scan, dim3(256 / kWaves, (unsigned)segs), dim3(kSortThreads), 0,
+                       s, hist, tiles, totals);
     hipLaunchKernelGGL(k_digit_scatter, grid, dim3(kSortThreads), 0, s, ka, va, n, shift,
-                       hist, tiles, kb, vb);
+                       hist, (const uint32_t *)totals, tiles, kb, vb);
     uint32_t *tk = ka;
     ka = kb;
     kb = tk;
@@ -194,13 +249,14 @@ int radix_sort_pairs(uint32_t *keys, int32_t *vals, int64_t n, void *ws,
 int permutation_segments(const uint32_t *keys, int64_t key_stride, int64_t segs, int64_t n,
                          int32_t *out, void *ws, int mode, hipStream_t s) {
   const dim3 g((unsigned)((n + 255) / 256), (unsigned)segs);
-  hipLaunchKernelGGL(k_iota, g, dim3(256), 0, s, out, n);
   uint32_t *bits = (uint32_t *)((char *)ws + sort_workspace_bytes(n, segs));
   const int rounds = (int)__builtin_ceil(3.0 * __builtin_log((double)(n > 1 ? n : 1)) /
                                          __builtin_log(4294967295.0));
+  if (rounds == 0)  // n == 1
+    hipLaunchKernelGGL(k_iota, g, dim3(256), 0, s, out, n);
   for (int r = 0; r < rounds; ++r) {
     hipLaunchKernelGGL(k_perm_round_bits, g, dim3(256), 0, s, keys, key_stride, r, n, bits,
-                       mode);
+                       out, mode);
     int rc = radix_sort_pairs(bits, out, n, ws, s, segs);
     if (rc) return rc;
   }
