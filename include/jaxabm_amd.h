@@ -246,13 +246,15 @@ typedef struct abm_wealth_inst {
 /* x, y, wealth from the collection's init key (device uint32[2]). */
 int abm_wealth_init(const uint32_t *init_key, int64_t n, float *x, float *y, int32_t *w,
                     int mode, void *stream);
-/* Runs every instance of the device array insts[count] for its steps, one
- * workgroup per instance.  max_n: the largest n in the table (0 if unknown).
- * With 0 < max_n <= 8000 every instance runs out of LDS (20 bytes per agent
- * of dynamic LDS per workgroup); otherwise, and for an instance above max_n,
- * on its global buffers.  With draws, every instance's draws are computed
- * first by a grid-wide kernel, and an instance of n < 1024 agents keeps its
- * state in registers.  Same results either way. */
+/* Runs every instance of the device array insts[count] for its steps (count
+ * <= 65,535).  max_n: the largest n in the table (0 if unknown).  With draws,
+ * an instance's draws are computed first by a grid-wide kernel; if n <= max_n
+ * <= 40,000 (or n <= 1,024), one workgroup then runs the exchange out of LDS
+ * (leaving each step's wealth in place of its targets in draws) while others
+ * walk the positions, and the records of all steps are taken at the end.
+ * Otherwise one workgroup runs the whole instance, out of LDS when 0 < n <=
+ * max_n <= 8000 (20 bytes per agent of dynamic LDS), else on its global
+ * buffers.  Same results either way. */
 int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t max_n, int mode,
                          void *stream);
 /* One instance across the whole GPU, for large n: two launches per step over

@@ -11,6 +11,18 @@
 
 namespace abm {
 
+// A pointer to global memory.  A pointer that a kernel reads from memory (an
+// instance table) has no known address space, and accesses through it compile
+// to flat instructions: those occupy the LDS counter too and make every wait
+// of a kernel with LDS traffic a full one, so loads in flight across an LDS
+// access are lost.  as_global(p) restores global loads and stores.
+template <class T>
+using GlobalPtr = T __attribute__((address_space(1))) *;
+template <class T>
+__device__ __forceinline__ GlobalPtr<T> as_global(T *p) {
+  return (GlobalPtr<T>)p;
+}
+
 // Integer threshold for `uniform < p` on [0,1): with m = bits >> 9,
 // u = m * 2^-23 exactly, so u < p  <=>  m < ceil(p * 2^23) (p in (0, 1]).
 // Computed on the host in double: exact for float p.

@@ -15,13 +15,21 @@
 // The sort is replaced by a histogram over wealth values: with c_w agents of
 // wealth w and b_w agents below, their ranks sum to c_w * b_w + c_w(c_w+1)/2,
 // so S = sum_w w * ranksum_w (mod 2^32, the int32 wrap of the reference).
-// Whole run in one launch: every phase boundary is a workgroup barrier.
-// Scatter-adds are integer atomics (exact, order-free); the histogram and
-// increments are cleared by the kernel after use.  An instance of up to
-// kWealthLdsAgents agents runs out of LDS (x, y, wealth, increments and
-// histogram, 20 bytes per agent, loaded at the start and x, y, wealth written
-// back at the end), so a step costs LDS latencies instead of global memory
-// round trips; larger instances run on their global buffers.
+// Scatter-adds are integer atomics (exact, order-free).
+//
+// A run with a draw buffer (abm_wealth_run_batch, draws != NULL) is split by
+// what depends on what.  The draws depend on nothing, so a grid-wide kernel
+// makes all of them first.  The walk depends on its own agent's draws only,
+// and a record only on its step's wealth.  What is left as a serial chain over
+// the steps is the exchange itself, and that alone runs step after step in
+// one workgroup (k_wealth_exchange), leaving every step's wealth in the draw
+// buffer; beside it other workgroups walk the positions, and after it the
+// records of all steps are taken at once, one workgroup per step
+// (k_wealth_records).
+// Without a draw buffer, or above the size the exchange keeps in LDS, one
+// workgroup runs everything: every phase boundary is a workgroup barrier, and
+// an instance of up to kWealthLdsAgents agents keeps its arrays in LDS
+// (20 bytes per agent), a larger one on its global buffers.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -52,8 +60,6 @@ __device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, uint32_t *red) {
   return s;  // valid in wave 0
 }
 
-// The whole run of one instance on the arrays x, y, w (state), inc and hist
-// (zero on entry, left zero) -- global buffers or their LDS copies.
 // The draws of agent i at one step: the position increments 0.01 * normal
 // (rounded as the reference's product) and the exchange target.
 struct WealthDraw {
@@ -78,26 +84,86 @@ __device__ __forceinline__ WealthDraw wealth_draw(const uint32_t *keys, int32_t 
 }
 
 // Every draw of a run, grid-wide, into draws[steps][3][n] (mdx, mdy bits,
-// target): none depends on the state, so the sequential run only applies
-// them.
-__global__ void __launch_bounds__(256)
+// target): none depends on the state.  Workgroups take tiles of one step and
+// kDrawThreads agents, so the step and its keys are uniform.
+constexpr int kDrawThreads = 256;
+
+__global__ void __launch_bounds__(kDrawThreads)
     k_wealth_draws(const abm_wealth_inst *__restrict__ insts, int mode) {
   const abm_wealth_inst in = insts[blockIdx.y];
   if (!in.draws) return;
   const int64_t n = in.n;
-  const int64_t total = (int64_t)in.steps * n;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += stride) {
-    const int32_t t = (int32_t)(e / n);
-    const int64_t i = e - (int64_t)t * n;
+  const int64_t per = (n + kDrawThreads - 1) / kDrawThreads;
+  for (int64_t q = blockIdx.x; q < (int64_t)in.steps * per; q += gridDim.x) {
+    const int32_t t = (int32_t)(q / per);
+    const int64_t i = (q - (int64_t)t * per) * kDrawThreads + threadIdx.x;
+    if (i >= n) continue;
     const WealthDraw d = wealth_draw(in.keys, t, n, i, mode);
-    uint32_t *row = in.draws + (int64_t)t * 3 * n;
+    const GlobalPtr<uint32_t> row = as_global(in.draws) + (int64_t)t * 3 * n;
     row[i] = __float_as_uint(d.mdx);
     row[n + i] = __float_as_uint(d.mdy);
     row[2 * n + i] = d.target;
   }
 }
 
+// Mean and Gini of a step from its total T and rank sum S.
+__device__ __forceinline__ void wealth_write_record(const abm_wealth_inst &in, int32_t t,
+                                                    uint32_t T, uint32_t S) {
+  const int64_t n = in.n;
+  in.mean_out[t] = (float)(int32_t)T / (float)n;
+  const int32_t Ti = (int32_t)T;
+  float g = 0.0f;
+  if ((float)Ti > 1e-6f) {
+    const int32_t num = (int32_t)(2u * S);
+    const int32_t den = (int32_t)((uint32_t)n * T);
+    const float q = (float)num / (float)den;
+    const float cst = (float)((double)(n + 1) / (double)n);
+    g = q - cst;
+  }
+  in.gini_out[t] = g;
+}
+
+// S = sum_w w * (c_w b_w + c_w (c_w + 1) / 2): chunked exclusive scan of the
+// histogram, one bin per thread per chunk, until all n agents are counted
+// (which covers every nonzero bin); the bins are cleared.  Valid in thread 0.
+__device__ __forceinline__ uint32_t wealth_rank_sum(int32_t *hist, int64_t n, uint32_t *red,
+                                                    uint32_t &carry) {
+  const int tid = threadIdx.x;
+  if (tid == 0) carry = 0;
+  __syncthreads();
+  uint32_t S_part = 0;
+  for (int64_t base = 0; base <= n; base += kWealthThreads) {
+    const int64_t w = base + tid;
+    const uint32_t c = w <= n ? (uint32_t)hist[w] : 0u;
+    // inclusive wave scan of c, then across waves
+    uint32_t inc = c;
+    const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(inc, off);
+      if (lane >= off) inc += y;
+    }
+    if (lane == 63) red[wave] = inc;
+    __syncthreads();
+    uint32_t wave_off = 0;
+    for (int q = 0; q < wave; ++q) wave_off += red[q];
+    const uint32_t before = carry + wave_off + inc - c;
+    if (c) {
+      const uint64_t ranksum = (uint64_t)c * before + (uint64_t)c * (c + 1) / 2;
+      S_part += (uint32_t)w * (uint32_t)ranksum;
+      hist[w] = 0;
+    }
+    __syncthreads();
+    if (tid == kWealthThreads - 1) carry = before + c;
+    __syncthreads();
+    if ((int64_t)carry >= n) break;  // block-uniform
+  }
+  return block_sum_u32(S_part, red);
+}
+
+// The whole run of one instance by one workgroup on the arrays x, y, w
+// (state), inc and hist (zero on entry, left zero) -- global buffers or their
+// LDS copies.
 __device__ __forceinline__ void wealth_steps(const abm_wealth_inst &in, float *gx, float *gy,
                                              int32_t *gw, int32_t *ginc, int32_t *ghist,
                                              uint32_t *red, uint32_t &carry, int mode) {
@@ -132,195 +198,215 @@ __device__ __forceinline__ void wealth_steps(const abm_wealth_inst &in, float *g
     }
     const uint32_t T = block_sum_u32(total, red);
     __syncthreads();
-    // S = sum_w w * (c_w b_w + c_w (c_w + 1) / 2): chunked exclusive scan of
-    // the histogram, one bin per thread per chunk
-    if (tid == 0) carry = 0;
-    __syncthreads();
-    uint32_t S_part = 0;
-    for (int64_t base = 0; base <= n; base += kWealthThreads) {
-      const int64_t w = base + tid;
-      const uint32_t c = w <= n ? (uint32_t)ghist[w] : 0u;
-      // inclusive wave scan of c, then across waves
-      uint32_t inc = c;
-      const int lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = __shfl_up(inc, off);
-        if (lane >= off) inc += y;
-      }
-      if (lane == 63) red[wave] = inc;
-      __syncthreads();
-      uint32_t wave_off = 0;
-      for (int q = 0; q < wave; ++q) wave_off += red[q];
-      const uint32_t before = carry + wave_off + inc - c;
-      if (c) {
-        const uint64_t ranksum = (uint64_t)c * before + (uint64_t)c * (c + 1) / 2;
-        S_part += (uint32_t)w * (uint32_t)ranksum;
-        ghist[w] = 0;
-      }
-      __syncthreads();
-      if (tid == kWealthThreads - 1) carry = before + c;
-      __syncthreads();
-    }
-    const uint32_t S = block_sum_u32(S_part, red);
-    if (tid == 0) {
-      in.mean_out[t] = (float)(int32_t)T / (float)n;
-      const int32_t Ti = (int32_t)T;
-      float g = 0.0f;
-      if ((float)Ti > 1e-6f) {
-        const int32_t num = (int32_t)(2u * S);
-        const int32_t den = (int32_t)((uint32_t)n * T);
-        const float q = (float)num / (float)den;
-        const float cst = (float)((double)(n + 1) / (double)n);
-        g = q - cst;
-      }
-      in.gini_out[t] = g;
-    }
+    const uint32_t S = wealth_rank_sum(ghist, n, red, carry);
+    if (tid == 0) wealth_write_record(in, t, T, S);
     __syncthreads();
   }
 }
 
-// n + 1 <= kWealthThreads with precomputed draws: one agent and one
-// histogram bin per thread, x, y and wealth in registers for the whole run,
-// increments and two histograms (steps alternate) in LDS; two barriers per
-// step.  Wealth is conserved, so the total T is summed once.  The rank sum S
-// of step t is taken by wave 0 alone from histogram t & 1 while the other
-// waves go on to step t + 1; that histogram's bins are cleared by their
-// owners after the next step's first barrier, when wave 0 has read them.
-__device__ __forceinline__ void wealth_steps_small(const abm_wealth_inst &in, int32_t *linc2,
-                                                   int32_t *lhist2, uint32_t *red_t) {
-  const int64_t n = in.n;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const bool agent = tid < n;
-  float x = agent ? in.x[tid] : 0.0f, y = agent ? in.y[tid] : 0.0f;
-  int32_t w = agent ? in.w[tid] : 0;
-  if (tid <= n) {
-    linc2[tid] = 0;
-    linc2[kWealthThreads + tid] = 0;
-    lhist2[tid] = 0;
-    lhist2[kWealthThreads + tid] = 0;
-  }
-  // T: the total wealth, the same at every step
-  uint32_t tw = agent ? (uint32_t)w : 0u;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) tw += __shfl_xor(tw, off);
-  if (lane == 0) red_t[wave] = tw;
-  __syncthreads();
-  uint32_t T = 0;
-  for (int q = 0; q < kWealthThreads / 64; ++q) T += red_t[q];
-  const float mean = (float)(int32_t)T / (float)n;
-  const float cst = (float)((double)(n + 1) / (double)n);
-  const int32_t steps = in.steps;
-  // Mean and Gini of step s from its histogram (wave 0), clearing the bins
-  // it reads: rank sum 64 bins a round until all n agents are counted (one
-  // round while every wealth is below 64); the nonzero bins all lie in the
-  // rounds read.
-  auto record = [&](int32_t s) {
-    int32_t *hist = lhist2 + (s & 1) * kWealthThreads;
-    uint32_t sp = 0, counted = 0;
-    for (int64_t b0 = 0; counted < (uint32_t)n && b0 <= n; b0 += 64) {
-      const int64_t wv = b0 + lane;
-      const uint32_t c = wv <= n ? (uint32_t)hist[wv] : 0u;
-      if (wv <= n) hist[wv] = 0;
-      uint32_t inc = c;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t v = __shfl_up(inc, off);
-        if (lane >= off) inc += v;
-      }
-      const uint32_t before = counted + inc - c;
-      if (c) {
-        const uint64_t ranksum = (uint64_t)c * before + (uint64_t)c * (c + 1) / 2;
-        sp += (uint32_t)wv * (uint32_t)ranksum;
-      }
-      counted += __shfl(inc, 63);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sp += __shfl_xor(sp, off);
-    if (lane == 0) {
-      in.mean_out[s] = mean;
-      const int32_t Ti = (int32_t)T;
-      float g = 0.0f;
-      if ((float)Ti > 1e-6f) {
-        const int32_t num = (int32_t)(2u * sp);
-        const int32_t den = (int32_t)((uint32_t)n * T);
-        const float q = (float)num / (float)den;
-        g = q - cst;
-      }
-      in.gini_out[s] = g;
-    }
-  };
-  // Step t's agent phase (walk, one exchange unit into linc[t & 1]) runs in
-  // the same phase as step t - 1's exchange (which reads and clears
-  // linc[(t - 1) & 1]), one barrier per step; wave 0 records step t - 1
-  // after the next barrier, while the others go on.  Each agent's own draw
-  // words of step t + 1 are loaded a step ahead.
-  uint32_t dx = 0u, dy = 0u, dt = 0u;
-  if (agent && steps > 0) {
-    dx = in.draws[tid];
-    dy = in.draws[n + tid];
-    dt = in.draws[2 * n + tid];
-  }
-  auto agent_phase = [&](int32_t t) {
-    const float mdx = __uint_as_float(dx), mdy = __uint_as_float(dy);
-    const uint32_t target = dt;
-    if (t + 1 < steps) {
-      const uint32_t *row = in.draws + (int64_t)(t + 1) * 3 * n;
-      dx = row[tid];
-      dy = row[n + tid];
-      dt = row[2 * n + tid];
-    }
-    x = mod1(x + mdx);
-    y = mod1(y + mdy);
-    if (w > 0) atomicAdd(&linc2[(t & 1) * kWealthThreads + target], 1);
-  };
-  if (agent && steps > 0) agent_phase(0);
-  for (int32_t t = 0; t < steps; ++t) {
-    __syncthreads();  // step t's exchange units are in; step t - 1's histogram is complete
-    if (wave == 0 && t > 0) record(t - 1);
-    if (agent) {
-      int32_t *linc = linc2 + (t & 1) * kWealthThreads;
-      w = w - (w > 0 ? 1 : 0) + linc[tid];
-      linc[tid] = 0;
-      atomicAdd(&lhist2[(t & 1) * kWealthThreads + w], 1);  // 0 <= w <= n: conserved
-      if (t + 1 < steps) agent_phase(t + 1);
-    }
-  }
-  if (steps > 0) {
-    __syncthreads();
-    if (wave == 0) record(steps - 1);
-  }
-  if (agent) {
-    in.x[tid] = x;
-    in.y[tid] = y;
-    in.w[tid] = w;
-  }
+// ---- runs with a draw buffer: exchange chain, walk and records apart
+
+// Instances the exchange kernel takes: two LDS arrays of increments, 32-bit up
+// to 20 agents a thread, and two agents per word above (a step gives an agent
+// at most n - 1 units, so neither half overflows), within 160 KB.
+constexpr int64_t kExchangeAgents = 40000;
+
+__host__ __device__ inline bool wealth_split_run(const abm_wealth_inst &in, int64_t cap) {
+  return in.draws != nullptr && in.n <= cap;
 }
 
-// kLds: the launch carries dynamic LDS for max_lds agents; instances with
-// n <= max_lds run out of it, others on their global buffers.
-template <bool kLds>
+// Barrier that orders LDS only: what a step reads back goes through LDS, so
+// the wealth rows in flight to memory need not have arrived.
+__device__ __forceinline__ void wealth_lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Words of one increment array: every thread's A agents, or pairs of them.
+constexpr int32_t exchange_words(int A, bool packed) {
+  return A * kWealthThreads / (packed ? 2 : 1);
+}
+
+// Steps ahead that a thread loads its A agents' targets: a step of few agents
+// takes less time than a memory round trip.
+constexpr int exchange_ahead(int A) { return A <= 2 ? 8 : A <= 8 ? 4 : A <= 16 ? 2 : 1; }
+
+// The exchange chain of one instance by one workgroup: thread t keeps the
+// wealth of agents t, t + 1024, .. (A of them) in registers, and a step is one
+// LDS atomic per giver, one barrier, and the increments read and cleared
+// (alternating arrays, so that one barrier a step is enough).  The wealth
+// after step t replaces the step's targets in the draw buffer.
+//
+// No global access of a step is in a branch: a wait for one load counts the
+// accesses issued after it, and a branch around any of them makes that a wait
+// for all, a memory round trip in every step (5,003 agents: 1.83 us a step,
+// 0.63 this way).  So the rows are accessed as raw buffers of n words, where
+// an absent agent's load gives 0 and its store is dropped by the bounds check.
+using RowBuffer = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ RowBuffer row_buffer(void *p, int32_t n) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, 4 * n, 0x00020000);
+}
+
+template <int A, bool kPacked>
+__device__ __forceinline__ void exchange_steps(const abm_wealth_inst &in, uint32_t *lds_inc) {
+  constexpr int P = exchange_ahead(A);
+  constexpr int32_t words = exchange_words(A, kPacked);
+  const uint32_t tid = threadIdx.x;
+  const int32_t n = (int32_t)in.n, steps = in.steps;
+  const int64_t row = 3 * (int64_t)n;
+  uint32_t *targets = in.draws + 2 * (int64_t)n;
+  auto load = [&](RowBuffer b, int a) {
+    return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(b, 4 * (tid + a * kWealthThreads), 0, 0);
+  };
+  auto store = [&](RowBuffer b, int a, uint32_t v) {
+    __builtin_amdgcn_raw_buffer_store_b32(v, b, 4 * (tid + a * kWealthThreads), 0, 0);
+  };
+  uint32_t w[A], target[P][A];
+  {
+    const RowBuffer wealth = row_buffer(in.w, n);
+#pragma unroll
+    for (int a = 0; a < A; ++a) w[a] = load(wealth, a);
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const RowBuffer b = row_buffer(targets + (p < steps ? p : 0) * row, n);
+#pragma unroll
+    for (int a = 0; a < A; ++a) target[p][a] = load(b, a);
+  }
+  for (int32_t t0 = 0; t0 < steps; t0 += P) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int32_t t = t0 + p;
+      if (t >= steps) break;
+      uint32_t *inc = lds_inc + ((t & 1) ? words : 0);
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        const uint32_t to = target[p][a];
+        if (w[a]) {
+          if constexpr (kPacked)
+            atomicAdd(&inc[to >> 1], 1u << ((to & 1u) << 4));
+          else
+            atomicAdd(&inc[to], 1u);
+        }
+      }
+      // rows past the end: the last one again, not used
+      const RowBuffer next = row_buffer(targets + (t + P < steps ? t + P : steps - 1) * row, n);
+#pragma unroll
+      for (int a = 0; a < A; ++a) target[p][a] = load(next, a);
+      wealth_lds_barrier();
+      const RowBuffer now = row_buffer(targets + t * row, n);
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        uint32_t got;
+        if constexpr (kPacked) {
+          uint16_t *mine = reinterpret_cast<uint16_t *>(inc) + a * kWealthThreads + tid;
+          got = *mine;
+          *mine = 0;
+        } else {
+          uint32_t *mine = inc + a * kWealthThreads + tid;
+          got = *mine;
+          *mine = 0;
+        }
+        w[a] = w[a] - (w[a] < 1u ? w[a] : 1u) + got;
+        store(now, a, w[a]);
+      }
+    }
+  }
+  const RowBuffer wealth = row_buffer(in.w, n);
+#pragma unroll
+  for (int a = 0; a < A; ++a) store(wealth, a, w[a]);
+}
+
+// Workgroups 0 .. count - 1 run the exchange chain of one instance each; the
+// workgroups after them walk the positions of 1024 agents each, which only
+// their own draws decide.  The chain is bound by its LDS latencies (atomic,
+// barrier, read) up to about 2,000 agents and by the LDS accesses of one CU
+// above.  1,000 agents x 100 steps: 25 us, where the workgroup that also
+// walked, counted and ranked took 141; 5,003 x 150: 94 us and 1,768.
+template <int A, bool kPacked>
 __global__ void __launch_bounds__(kWealthThreads)
-    k_wealth_run(const abm_wealth_inst *__restrict__ insts, int64_t max_lds, int mode) {
-  extern __shared__ int32_t lds_agents[];
+    k_wealth_exchange(const abm_wealth_inst *__restrict__ insts, int32_t count, int64_t cap) {
+  extern __shared__ uint32_t lds_inc[];
+  const int tid = threadIdx.x;
+  if ((int32_t)blockIdx.x >= count) {
+    const int32_t q = (int32_t)blockIdx.x - count;
+    const abm_wealth_inst in = insts[q % count];
+    const int64_t n = in.n, i = (int64_t)(q / count) * kWealthThreads + tid;
+    if (!wealth_split_run(in, cap) || i >= n) return;
+    constexpr int kAhead = 8;
+    const GlobalPtr<uint32_t> draws = as_global(in.draws) + i;
+    const GlobalPtr<float> gx = as_global(in.x) + i, gy = as_global(in.y) + i;
+    float x = *gx, y = *gy;
+    for (int32_t t0 = 0; t0 < in.steps; t0 += kAhead) {
+      float dx[kAhead], dy[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const int32_t t = t0 + k < in.steps ? t0 + k : in.steps - 1;
+        dx[k] = __uint_as_float(draws[(int64_t)t * 3 * n]);
+        dy[k] = __uint_as_float(draws[(int64_t)t * 3 * n + n]);
+      }
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k)
+        if (t0 + k < in.steps) {
+          x = mod1(x + dx[k]);
+          y = mod1(y + dy[k]);
+        }
+    }
+    *gx = x;
+    *gy = y;
+    return;
+  }
+  const abm_wealth_inst in = insts[blockIdx.x];
+  if (!wealth_split_run(in, cap)) return;
+  for (int32_t k = tid; k < 2 * exchange_words(A, kPacked); k += kWealthThreads) lds_inc[k] = 0;
+  __syncthreads();
+  exchange_steps<A, kPacked>(in, lds_inc);
+}
+
+// LDS limit of the records: n + 1 bins, or the state of kWealthLdsAgents.
+constexpr int64_t kRecordsLds = (kExchangeAgents + 1) * 4;
+static_assert(kRecordsLds >= kWealthLdsAgents * kWealthLdsBytesPerAgent + 4 &&
+                  kRecordsLds + 128 <= 160 * 1024,
+              "records LDS");
+
+// Workgroup (b, instance): the records of steps b, b + gridDim.x, .. of an
+// instance whose exchange has run, each from a histogram of the step's wealth
+// row in LDS (n + 1 bins).  Workgroup 0 of an instance that the exchange
+// kernel did not take runs it whole instead, in LDS where lds_bytes allow.
+__global__ void __launch_bounds__(kWealthThreads)
+    k_wealth_records(const abm_wealth_inst *__restrict__ insts, int64_t cap, int64_t lds_agents,
+                     int mode) {
+  extern __shared__ int32_t lds_agents_mem[];
   __shared__ uint32_t red[16];
   __shared__ uint32_t carry;
-  __shared__ uint32_t red_t[kWealthThreads / 64], red_s[kWealthThreads / 64];
-  const abm_wealth_inst in = insts[blockIdx.x];
+  const abm_wealth_inst in = insts[blockIdx.y];
   const int64_t n = in.n;
   const int tid = threadIdx.x;
-  if (in.draws && n + 1 <= kWealthThreads) {
-    // two increment arrays and two histograms: the dynamic LDS (at least 4 x
-    // kWealthThreads words in this launch), or a static array where the
-    // launch has none
-    if constexpr (kLds) {
-      wealth_steps_small(in, lds_agents, lds_agents + 2 * kWealthThreads, red_t);
-    } else {
-      __shared__ int32_t small_lds[4 * kWealthThreads];
-      wealth_steps_small(in, small_lds, small_lds + 2 * kWealthThreads, red_t);
+  if (wealth_split_run(in, cap)) {
+    int32_t *hist = lds_agents_mem;
+    if ((int32_t)blockIdx.x >= in.steps) return;
+    for (int64_t b = tid; b <= n; b += kWealthThreads) hist[b] = 0;
+    __syncthreads();
+    for (int32_t t = blockIdx.x; t < in.steps; t += gridDim.x) {
+      const GlobalPtr<const uint32_t> row =
+          as_global<const uint32_t>(in.draws) + (int64_t)t * 3 * n + 2 * n;
+      uint32_t total = 0;
+      for (int64_t i = tid; i < n; i += kWealthThreads) {
+        const uint32_t wi = row[i];
+        atomicAdd(&hist[wi], 1);  // 0 <= wi <= n: wealth is conserved
+        total += wi;
+      }
+      const uint32_t T = block_sum_u32(total, red);
+      const uint32_t S = wealth_rank_sum(hist, n, red, carry);
+      if (tid == 0) wealth_write_record(in, t, T, S);
+      __syncthreads();
     }
-  } else if (kLds && n <= max_lds) {
-    float *lx = reinterpret_cast<float *>(lds_agents);
+    return;
+  }
+  if (blockIdx.x != 0) return;
+  if (n <= lds_agents) {
+    float *lx = reinterpret_cast<float *>(lds_agents_mem);
     float *ly = lx + n;
     int32_t *lw = reinterpret_cast<int32_t *>(ly + n);
     int32_t *linc = lw + n;
@@ -498,7 +584,26 @@ __global__ void k_wealth_init(const uint32_t *__restrict__ init_key, int64_t n,
   w[i] = 1;
 }
 
-// The LDS-resident run needs more than 64 KB of dynamic LDS: the limit is
+using ExchangeKernel = void (*)(const abm_wealth_inst *, int32_t, int64_t);
+
+// One instantiation per number of agents a thread keeps.
+struct ExchangeVariant {
+  int agents;
+  size_t lds;
+  ExchangeKernel kernel;
+};
+template <int A, bool kPacked>
+constexpr ExchangeVariant exchange_variant() {
+  return ExchangeVariant{A, 8 * (size_t)exchange_words(A, kPacked), k_wealth_exchange<A, kPacked>};
+}
+const ExchangeVariant kExchange[] = {
+    exchange_variant<1, false>(),  exchange_variant<2, false>(),  exchange_variant<3, false>(),
+    exchange_variant<4, false>(),  exchange_variant<5, false>(),  exchange_variant<6, false>(),
+    exchange_variant<8, false>(),  exchange_variant<10, false>(), exchange_variant<12, false>(),
+    exchange_variant<16, false>(), exchange_variant<20, false>(), exchange_variant<24, true>(),
+    exchange_variant<32, true>(),  exchange_variant<40, true>()};
+
+// These kernels may need more than 64 KB of dynamic LDS: the limits are
 // raised once per device, under a lock.
 constexpr int kMaxDevices = 64;
 std::mutex g_wealth_attr_mu;
@@ -510,9 +615,13 @@ int wealth_lds_attr() {
   ABM_REQUIRE(dev >= 0 && dev < kMaxDevices, "wealth: device index out of range");
   std::lock_guard<std::mutex> lock(g_wealth_attr_mu);
   if (!g_wealth_attr_set[dev]) {
-    ABM_CHECK_HIP(hipFuncSetAttribute((const void *)k_wealth_run<true>,
+    for (const ExchangeVariant &v : kExchange)
+      ABM_CHECK_HIP(hipFuncSetAttribute((const void *)v.kernel,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)v.lds));
+    ABM_CHECK_HIP(hipFuncSetAttribute((const void *)k_wealth_records,
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)(kWealthLdsAgents * kWealthLdsBytesPerAgent + 4)));
+                                      (int)kRecordsLds));
     g_wealth_attr_set[dev] = true;
   }
   return kOk;
@@ -562,20 +671,27 @@ int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t ma
   ABM_REQUIRE(insts && count >= 0 && max_n >= 0 && (mode == 0 || mode == 1),
               "abm_wealth_run_batch: bad arguments");
   if (count == 0) return kOk;
-  hipLaunchKernelGGL(k_wealth_draws, dim3(512u, (unsigned)count), dim3(256), 0,
-                     (hipStream_t)stream, insts, mode);
-  if (max_n > 0 && max_n <= kWealthLdsAgents) {
-    if (int rc = wealth_lds_attr()) return rc;
-    size_t dyn = (size_t)(max_n * kWealthLdsBytesPerAgent + 4);
-    // an instance of n < kWealthThreads keeps its increments and two
-    // histograms there
-    if (dyn < 4 * kWealthThreads * sizeof(int32_t)) dyn = 4 * kWealthThreads * sizeof(int32_t);
-    hipLaunchKernelGGL(k_wealth_run<true>, dim3((unsigned)count), dim3(kWealthThreads), dyn,
-                       (hipStream_t)stream, insts, max_n, mode);
-  } else {
-    hipLaunchKernelGGL(k_wealth_run<false>, dim3((unsigned)count), dim3(kWealthThreads), 0,
-                       (hipStream_t)stream, insts, (int64_t)0, mode);
-  }
+  ABM_REQUIRE(count <= 65535, "abm_wealth_run_batch: at most 65,535 instances a call");
+  if (int rc = wealth_lds_attr()) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  // the exchange kernel takes instances of up to `cap` agents: the table's
+  // largest, and always those of one agent per thread
+  const int64_t known = max_n <= kExchangeAgents ? max_n : 0;
+  const int64_t cap = known > kWealthThreads ? known : kWealthThreads;
+  const int per = (int)((cap + kWealthThreads - 1) / kWealthThreads);
+  const ExchangeVariant *v = kExchange;
+  while (v->agents < per) ++v;
+  // LDS of the records: the histogram of `cap` agents, or the whole state of
+  // an instance that runs in one workgroup (no draw buffer)
+  const int64_t lds_agents = max_n > 0 && max_n <= kWealthLdsAgents ? max_n : 0;
+  size_t dyn = (size_t)(lds_agents * kWealthLdsBytesPerAgent + 4);
+  if (dyn < (size_t)(cap + 1) * 4) dyn = (size_t)(cap + 1) * 4;
+  hipLaunchKernelGGL(k_wealth_draws, dim3(512u, (unsigned)count), dim3(kDrawThreads), 0, s,
+                     insts, mode);
+  hipLaunchKernelGGL(v->kernel, dim3((unsigned)(count * (1 + per))), dim3(kWealthThreads),
+                     v->lds, s, insts, count, cap);
+  hipLaunchKernelGGL(k_wealth_records, dim3(256u, (unsigned)count), dim3(kWealthThreads), dyn, s,
+                     insts, cap, lds_agents, mode);
   ABM_LAUNCH_CHECK("abm_wealth_run_batch");
   return kOk;
 }

@@ -146,3 +146,56 @@ def test_grid_path_wealth_above_the_lds_bins(wealth):
     np.testing.assert_array_equal(mean, om)
     np.testing.assert_array_equal(gini, og)
     np.testing.assert_array_equal(eng.w.cpu().numpy(), w)
+
+
+# one agent more or less than a thread's share, the widest 32-bit and the
+# packed increment arrays, the largest instance the exchange kernel takes;
+# step counts around the load-ahead distances and the 256 record workgroups
+@pytest.mark.parametrize("n,steps", [(2, 1), (63, 2), (64, 7), (65, 8), (1023, 9), (1024, 17),
+                                     (1025, 300), (2049, 3), (6145, 5), (10241, 4), (20480, 6),
+                                     (20481, 6), (39999, 3), (40000, 4), (40001, 2)])
+def test_exchange_run_matches_oracle_at_its_edges(wealth, n, steps):
+    import os
+
+    for mode in (O.MODE_PARTITIONABLE, O.MODE_ORIGINAL):
+        eng = wealth.WealthEngine(n, seed=n, mode=mode)
+        mean, gini = _run_raw(wealth, eng, steps, n, draws=True)
+        x, y, w, rng = O.wealth_init(n, n, mode)
+        om, og = O.wealth_run_threads(x, y, w, rng, steps,
+                                      max(1, min(16, os.cpu_count() or 1)), mode)
+        np.testing.assert_array_equal(mean, om)
+        np.testing.assert_array_equal(gini, og)
+        np.testing.assert_array_equal(eng.w.cpu().numpy(), w)
+        np.testing.assert_array_equal(eng.x.cpu().numpy(), x)
+        np.testing.assert_array_equal(eng.y.cpu().numpy(), y)
+
+
+def test_batch_of_split_and_whole_runs(wealth):
+    """One table with instances of uneven sizes, with and without a draw
+    buffer, and steps 0: each as its own run."""
+    import torch
+
+    from jaxabm_amd._lib import check, lib, ptr, stream_handle
+
+    sizes = [(3000, 12, True), (900, 30, False), (1, 0, None), (40, 5, True), (2999, 12, False)]
+    sizes = [(max(n, 2), s, d) for n, s, d in sizes]
+    engs = [wealth.WealthEngine(n, seed=i) for i, (n, _, _) in enumerate(sizes)]
+    keep, descs, outs = [], [], []
+    for e, (n, s, d) in zip(engs, sizes):
+        keys = e.key_table(s)
+        mean = torch.empty(max(s, 1), dtype=torch.float32, device=e.device)
+        gini = torch.empty(max(s, 1), dtype=torch.float32, device=e.device)
+        buf = e.draw_buffer(s) if d or d is None else None
+        keep += [keys, buf]
+        descs.append(e.descriptor(keys, s, mean, gini, buf))
+        outs.append((mean, gini))
+    table = torch.from_numpy(np.concatenate(descs).view(np.uint8)).cuda()
+    check(lib().abm_wealth_run_batch(ptr(table), len(engs), 3000, engs[0].mode, stream_handle()),
+          "run")
+    for i, (e, (n, s, _), (mean, gini)) in enumerate(zip(engs, sizes, outs)):
+        x, y, w, rng = O.wealth_init(n, i, e.mode)
+        om, og = O.wealth_run(x, y, w, rng, s, e.mode)
+        np.testing.assert_array_equal(mean.cpu().numpy()[:s], om[:s])
+        np.testing.assert_array_equal(gini.cpu().numpy()[:s], og[:s])
+        for a, b in ((e.w, w), (e.x, x), (e.y, y)):
+            np.testing.assert_array_equal(a.cpu().numpy(), b)
