@@ -257,12 +257,13 @@ int abm_wealth_init(const uint32_t *init_key, int64_t n, float *x, float *y, int
  * buffers.  Same results either way. */
 int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t max_n, int mode,
                          void *stream);
-/* One instance across the whole GPU, for large n: two launches per step over
- * all workgroups (each agent's draws computed and applied, exchange atomics,
- * with the previous step's mean and Gini recorded by workgroup 0; then the
- * exchange applied, the wealth histogram, total and maximum).  inst: the
- * descriptor in host memory (passed to the kernels by value); its draws
- * field is not used.  acc: device scratch uint32[ABM_WEALTH_GRID_ACC_WORDS]
+/* One instance across the whole GPU, for large n.  inst: the descriptor in
+ * host memory (passed to the kernels by value).  With draws != NULL (at least
+ * 3 n words of scratch) and n >= 1033, one launch per step: every workgroup
+ * applies the previous step's exchange to its agents, then draws and applies
+ * this step's walk and gives its units, while one workgroup records the step
+ * before.  Otherwise two launches per step (draws, walk and exchange atomics
+ * with the previous step recorded; then the exchange applied and counted).  acc: device scratch uint32[ABM_WEALTH_GRID_ACC_WORDS]
  * (the total and 16 copies of the 64 smallest histogram bins, so that no
  * word takes an atomic from every workgroup).  Same results as
  * abm_wealth_run_batch. */

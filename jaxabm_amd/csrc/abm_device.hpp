@@ -28,6 +28,19 @@ struct Key {
 
 ABM_HD uint32_t rotl(uint32_t v, int r) { return (v << r) | (v >> (32 - r)); }
 
+// A source that draws in one straight run (a compile-time stream mode) defines
+// ABM_STRAIGHT_DRAWS before it includes this: the compiler must then not
+// reassociate integer sums across a threefry block's key injections.  It would
+// rewrite the round sums x0 + x1 + x1' + .. in terms of one another, with
+// twice the operations and 229 registers (seven blocks and two normals: 1,750
+// operations a thread instead of 850).  Where the mode is decided at run time,
+// branches keep the blocks apart, and the barriers only cost registers.
+#if defined(__HIP_DEVICE_COMPILE__) && defined(ABM_STRAIGHT_DRAWS)
+#define ABM_KEEP_ORDER(a, b) asm("" : "+v"(a), "+v"(b));
+#else
+#define ABM_KEEP_ORDER(a, b)
+#endif
+
 // One threefry2x32-20 block.
 ABM_HD void threefry(uint32_t k0, uint32_t k1, uint32_t x0, uint32_t x1,
                      uint32_t &y0, uint32_t &y1) {
@@ -37,11 +50,11 @@ ABM_HD void threefry(uint32_t k0, uint32_t k1, uint32_t x0, uint32_t x1,
 #define ABM_R(r) \
   x0 += x1;      \
   x1 = rotl(x1, r) ^ x0;
-  ABM_R(13) ABM_R(15) ABM_R(26) ABM_R(6) x0 += k1; x1 += k2 + 1u;
-  ABM_R(17) ABM_R(29) ABM_R(16) ABM_R(24) x0 += k2; x1 += k0 + 2u;
-  ABM_R(13) ABM_R(15) ABM_R(26) ABM_R(6) x0 += k0; x1 += k1 + 3u;
-  ABM_R(17) ABM_R(29) ABM_R(16) ABM_R(24) x0 += k1; x1 += k2 + 4u;
-  ABM_R(13) ABM_R(15) ABM_R(26) ABM_R(6) x0 += k2; x1 += k0 + 5u;
+  ABM_R(13) ABM_R(15) ABM_R(26) ABM_R(6) ABM_KEEP_ORDER(x0, x1) x0 += k1; x1 += k2 + 1u;
+  ABM_R(17) ABM_R(29) ABM_R(16) ABM_R(24) ABM_KEEP_ORDER(x0, x1) x0 += k2; x1 += k0 + 2u;
+  ABM_R(13) ABM_R(15) ABM_R(26) ABM_R(6) ABM_KEEP_ORDER(x0, x1) x0 += k0; x1 += k1 + 3u;
+  ABM_R(17) ABM_R(29) ABM_R(16) ABM_R(24) ABM_KEEP_ORDER(x0, x1) x0 += k1; x1 += k2 + 4u;
+  ABM_R(13) ABM_R(15) ABM_R(26) ABM_R(6) ABM_KEEP_ORDER(x0, x1) x0 += k2; x1 += k0 + 5u;
 #undef ABM_R
   y0 = x0;
   y1 = x1;

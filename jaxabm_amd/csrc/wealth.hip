@@ -34,6 +34,7 @@
 
 #include <mutex>
 
+#define ABM_STRAIGHT_DRAWS
 #include "common.hpp"
 #include "jaxabm_amd.h"
 
@@ -67,12 +68,10 @@ struct WealthDraw {
   uint32_t target;
 };
 
-__device__ __forceinline__ WealthDraw wealth_draw(const uint32_t *keys, int32_t t, int64_t n,
-                                                  int64_t i, int mode) {
-  const Key ck{keys[4 * t + 0], keys[4 * t + 1]};
-  const Key uk{keys[4 * t + 2], keys[4 * t + 3]};
-  Key kk1, kk2, k1, k2;
-  split2(uk, kk1, kk2, mode);
+// (ck: the collection key; kk1, kk2 = split(uk), the same for every agent).
+__device__ __forceinline__ WealthDraw wealth_draw(Key ck, Key kk1, Key kk2, int64_t n, int64_t i,
+                                                  int mode) {
+  Key k1, k2;
   split2(split_at(ck, n, i, mode), k1, k2, mode);
   WealthDraw d;
   d.mdx = 0.01f * normal_from_bits(bits_scalar(k1, mode));
@@ -83,13 +82,23 @@ __device__ __forceinline__ WealthDraw wealth_draw(const uint32_t *keys, int32_t 
   return d;
 }
 
+__device__ __forceinline__ WealthDraw wealth_draw(const uint32_t *keys, int32_t t, int64_t n,
+                                                  int64_t i, int mode) {
+  const Key ck{keys[4 * t + 0], keys[4 * t + 1]};
+  const Key uk{keys[4 * t + 2], keys[4 * t + 3]};
+  Key kk1, kk2;
+  split2(uk, kk1, kk2, mode);
+  return wealth_draw(ck, kk1, kk2, n, i, mode);
+}
+
 // Every draw of a run, grid-wide, into draws[steps][3][n] (mdx, mdy bits,
 // target): none depends on the state.  Workgroups take tiles of one step and
 // kDrawThreads agents, so the step and its keys are uniform.
 constexpr int kDrawThreads = 256;
 
+template <int kMode>
 __global__ void __launch_bounds__(kDrawThreads)
-    k_wealth_draws(const abm_wealth_inst *__restrict__ insts, int mode) {
+    k_wealth_draws(const abm_wealth_inst *__restrict__ insts) {
   const abm_wealth_inst in = insts[blockIdx.y];
   if (!in.draws) return;
   const int64_t n = in.n;
@@ -98,7 +107,7 @@ __global__ void __launch_bounds__(kDrawThreads)
     const int32_t t = (int32_t)(q / per);
     const int64_t i = (q - (int64_t)t * per) * kDrawThreads + threadIdx.x;
     if (i >= n) continue;
-    const WealthDraw d = wealth_draw(in.keys, t, n, i, mode);
+    const WealthDraw d = wealth_draw(in.keys, t, n, i, kMode);
     const GlobalPtr<uint32_t> row = as_global(in.draws) + (int64_t)t * 3 * n;
     row[i] = __float_as_uint(d.mdx);
     row[n + i] = __float_as_uint(d.mdy);
@@ -446,6 +455,11 @@ __global__ void __launch_bounds__(kWealthThreads)
 constexpr int kGridThreads = 256;
 constexpr int kGridBins = 1024;     // LDS histogram bins per workgroup
 constexpr int64_t kGridMaxBlocks = 1024;
+// workgroups of a one-launch step, beside the recording one (each flushes its
+// bins, so a large instance gives them several tiles of agents)
+constexpr int64_t kGridStepBlocks = 4096;
+// a one-launch step's scratch, 2 n + 1 + 1024 + 8 words, is within 3 n from here
+constexpr int64_t kGridOneLaunch = 1033;
 constexpr int kGridHot = 64;        // values with their own histogram copies
 constexpr int kGridCopies = 16;
 static_assert(ABM_WEALTH_GRID_ACC_WORDS == 2 + kGridCopies * kGridHot,
@@ -568,6 +582,149 @@ __global__ void __launch_bounds__(kGridThreads)
   }
 }
 
+// One launch per step, with scratch for a second increment array, histogram
+// and set of hot bins: launch t applies step t - 1's exchange to its agents
+// (own reads and writes only) and counts their wealth, then gives step t's
+// units and walks, and workgroup 0 records step t - 2.  What a launch adds to
+// (increments of step t, bins of step t - 1) and what it reads and clears
+// (increments of step t - 1, bins of step t - 2) alternate between the two
+// copies, so no launch reads what another workgroup of it writes.  Launch
+// `steps` only applies, launch steps + 1 only records.  Of a step of 247,720
+// agents 6.4 us are its seven threefry blocks and two erf_inv an agent (1,020
+// operations, VALU); the rest is the launch, the loads before and the bins
+// after them.  Two launches a step, with the record in front of workgroup 0's
+// agents, took 14.0 us a step; this takes 11.8.
+// The keys that all agents share (split(uk) of the step) are made by workgroup
+// 0 of the launch before; in every thread they were 137 of 990 operations.
+struct WealthGrid {
+  uint32_t *inc[2], *hist[2], *hot[2], *total;
+  uint32_t *shared_keys;  // [2][4]: kk1, kk2 of even and odd steps
+};
+
+// split(uk) of step t into the shared keys (one thread).
+__device__ __forceinline__ void wealth_shared_keys(const abm_wealth_inst &in, uint32_t *shared,
+                                                   int32_t t, int mode) {
+  Key kk1, kk2;
+  split2(Key{in.keys[4 * t + 2], in.keys[4 * t + 3]}, kk1, kk2, mode);
+  uint32_t *out = shared + 4 * (t & 1);
+  out[0] = kk1.k0;
+  out[1] = kk1.k1;
+  out[2] = kk2.k0;
+  out[3] = kk2.k1;
+}
+
+// Mean and Gini of step t from a histogram set; clears the bins it reads.
+__device__ void wealth_grid_rank(const abm_wealth_inst &in, int32_t t, uint32_t T, uint32_t *hot,
+                                 uint32_t *hist, uint32_t *red) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t n = in.n;
+  uint32_t S_part = 0, counted = 0;
+  for (int64_t base = 0; base <= n; base += kGridThreads) {
+    const int64_t w = base + tid;
+    uint32_t c = 0;
+    if (w < kGridHot) {
+      uint32_t v[kGridCopies];
+#pragma unroll
+      for (int k = 0; k < kGridCopies; ++k) v[k] = hot[k * kGridHot + w];
+#pragma unroll
+      for (int k = 0; k < kGridCopies; ++k) {
+        c += v[k];
+        if (v[k]) hot[k * kGridHot + w] = 0;
+      }
+    } else if (w <= n) {
+      c = hist[w];
+      if (c) hist[w] = 0;
+    }
+    uint32_t inc = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(inc, off);
+      if (lane >= off) inc += y;
+    }
+    if (lane == 63) red[wave] = inc;
+    __syncthreads();
+    uint32_t before = counted + inc - c;
+    for (int q = 0; q < kGridThreads / 64; ++q) {
+      if (q < wave) before += red[q];
+      counted += red[q];
+    }
+    if (c) {
+      const uint64_t ranksum = (uint64_t)c * before + (uint64_t)c * (c + 1) / 2;
+      S_part += (uint32_t)w * (uint32_t)ranksum;
+    }
+    __syncthreads();  // red is rewritten
+    if ((int64_t)counted >= n) break;  // block-uniform
+  }
+  const uint32_t S = block_sum_u32(S_part, red);
+  if (tid == 0) wealth_write_record(in, t, T, S);
+}
+
+template <int kMode>
+__global__ void __launch_bounds__(kGridThreads)
+    k_wealth_grid_step(abm_wealth_inst in, WealthGrid g, int32_t t) {
+  __shared__ uint32_t red[kGridThreads / 64];
+  __shared__ uint32_t bins[kGridBins];
+  const int64_t n = in.n;
+  const int cur = t & 1, prev = cur ^ 1;
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0 && t + 1 < in.steps)
+      wealth_shared_keys(in, g.shared_keys, t + 1, kMode);
+    if (t > 1) wealth_grid_rank(in, t - 2, *g.total, g.hot[cur], g.hist[cur], red);
+    return;
+  }
+  if (t > in.steps) return;
+  for (int b = threadIdx.x; b < kGridBins; b += kGridThreads) bins[b] = 0;
+  __syncthreads();
+  uint32_t total = 0;
+  const int32_t tk = t < in.steps ? t : 0;  // the last launch draws nothing
+  const Key ck{in.keys[4 * tk], in.keys[4 * tk + 1]};
+  const uint32_t *sk = g.shared_keys + 4 * (tk & 1);
+  const Key kk1{sk[0], sk[1]}, kk2{sk[2], sk[3]};
+  const int64_t stride = (int64_t)(gridDim.x - 1) * kGridThreads;
+#pragma unroll 1
+  for (int64_t i = (int64_t)(blockIdx.x - 1) * kGridThreads + threadIdx.x; i < n; i += stride) {
+    int32_t wi = in.w[i];
+    if (t > 0) {
+      wi = wi - (wi > 0 ? 1 : 0) + (int32_t)g.inc[prev][i];
+      g.inc[prev][i] = 0;
+      in.w[i] = wi;
+      // 0 <= wi <= n: wealth is conserved
+      if (wi < kGridBins)
+        atomicAdd(&bins[wi], 1u);
+      else
+        atomicAdd(&g.hist[prev][wi], 1u);
+      total += (uint32_t)wi;
+    }
+    if (t < in.steps) {
+      const WealthDraw d = wealth_draw(ck, kk1, kk2, n, i, kMode);
+      if (wi > 0) atomicAdd(&g.inc[cur][d.target], 1u);
+      in.x[i] = mod1(in.x[i] + d.mdx);
+      in.y[i] = mod1(in.y[i] + d.mdy);
+    }
+  }
+  if (t == 0) return;
+  __syncthreads();
+  uint32_t *hot = g.hot[prev] + (int64_t)(blockIdx.x % kGridCopies) * kGridHot;
+  for (int b = threadIdx.x; b < kGridBins; b += kGridThreads) {
+    const uint32_t c = bins[b];
+    if (!c) continue;
+    atomicAdd(b < kGridHot ? &hot[b] : &g.hist[prev][b], c);
+  }
+  if (t == 1) {  // the total, conserved from here on
+    const uint32_t T = block_sum_u32(total, red);
+    if (threadIdx.x == 0) atomicAdd(g.total, T);
+  }
+}
+
+// Clears a run's scratch and makes step 0's shared keys.
+__global__ void k_wealth_grid_begin(abm_wealth_inst in, WealthGrid g, uint32_t *acc, int64_t used,
+                                    int mode) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < used) in.draws[i] = 0;
+  if (i < ABM_WEALTH_GRID_ACC_WORDS) acc[i] = 0;
+  if (i == used) wealth_shared_keys(in, g.shared_keys, 0, mode);
+}
+
 __global__ void k_wealth_zero_acc(uint32_t *acc) {
   for (int i = threadIdx.x; i < ABM_WEALTH_GRID_ACC_WORDS; i += blockDim.x) acc[i] = 0;
 }
@@ -652,6 +809,30 @@ int abm_wealth_run_grid(const abm_wealth_inst *inst, uint32_t *acc, int mode, vo
               "abm_wealth_run_grid: incomplete instance");
   hipStream_t s = (hipStream_t)stream;
   if (in.steps == 0) return kOk;
+  if (in.draws && in.n >= kGridOneLaunch) {
+    WealthGrid g;
+    g.total = acc;
+    g.inc[0] = (uint32_t *)in.inc;
+    g.hist[0] = (uint32_t *)in.hist;
+    g.hot[0] = acc + 2;
+    g.inc[1] = in.draws;
+    g.hist[1] = in.draws + in.n;
+    g.hot[1] = in.draws + 2 * in.n + 1;
+    const int64_t used = 2 * in.n + 1 + kGridCopies * kGridHot;
+    g.shared_keys = in.draws + used;
+    hipLaunchKernelGGL(k_wealth_grid_begin, dim3((unsigned)(used / 256 + 1)), dim3(256), 0, s, in,
+                       g, acc, used, mode);
+    const int64_t tiles = (in.n + kGridThreads - 1) / kGridThreads;
+    const int64_t per = (tiles + kGridStepBlocks - 1) / kGridStepBlocks;  // tiles a workgroup
+    const unsigned blocks = (unsigned)(1 + (tiles + per - 1) / per);
+    auto *step = mode == kModePartitionable ? k_wealth_grid_step<kModePartitionable>
+                                            : k_wealth_grid_step<kModeOriginal>;
+    for (int32_t t = 0; t <= in.steps + 1; ++t)  // the last one only records
+      hipLaunchKernelGGL(step, dim3(t <= in.steps ? blocks : 1), dim3(kGridThreads), 0, s, in, g,
+                         t);
+    ABM_LAUNCH_CHECK("abm_wealth_run_grid");
+    return kOk;
+  }
   hipLaunchKernelGGL(k_wealth_zero_acc, dim3(1), dim3(256), 0, s, acc);
   int64_t blocks = (in.n + kGridThreads - 1) / kGridThreads;
   if (blocks > kGridMaxBlocks) blocks = kGridMaxBlocks;
@@ -686,8 +867,9 @@ int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t ma
   const int64_t lds_agents = max_n > 0 && max_n <= kWealthLdsAgents ? max_n : 0;
   size_t dyn = (size_t)(lds_agents * kWealthLdsBytesPerAgent + 4);
   if (dyn < (size_t)(cap + 1) * 4) dyn = (size_t)(cap + 1) * 4;
-  hipLaunchKernelGGL(k_wealth_draws, dim3(512u, (unsigned)count), dim3(kDrawThreads), 0, s,
-                     insts, mode);
+  hipLaunchKernelGGL(mode == kModePartitionable ? k_wealth_draws<kModePartitionable>
+                                                : k_wealth_draws<kModeOriginal>,
+                     dim3(512u, (unsigned)count), dim3(kDrawThreads), 0, s, insts);
   hipLaunchKernelGGL(v->kernel, dim3((unsigned)(count * (1 + per))), dim3(kWealthThreads),
                      v->lds, s, insts, count, cap);
   hipLaunchKernelGGL(k_wealth_records, dim3(256u, (unsigned)count), dim3(kWealthThreads), dyn, s,

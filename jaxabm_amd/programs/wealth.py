@@ -23,9 +23,15 @@ from .._lib import (WEALTH_GRID_ACC_WORDS, WEALTH_INST, check, lib, ptr, require
                     stream_handle)
 
 
-# above the LDS capacity of one workgroup (8,000 agents), a run spreads over
-# the whole GPU
+# up to here one workgroup can run a whole simulation out of LDS, whatever the
+# number of steps
 GRID_MIN_AGENTS = 8000
+# up to here the exchange of a run with a draw buffer fits one workgroup's LDS.
+# 100 steps of 8,000 / 20,000 / 40,000 agents: 259 / 437 / 717 us, and 673 /
+# 680 / 732 us spread over the GPU, where a step costs a launch
+EXCHANGE_MAX_AGENTS = 40_000
+# largest draw buffer a run above GRID_MIN_AGENTS takes for that
+DRAW_BUFFER_MAX_BYTES = 1 << 30
 
 
 class WealthEngine:
@@ -76,15 +82,20 @@ class WealthEngine:
 
     def run(self, steps: int):
         """Run ``steps`` steps; returns host (mean, gini) float32 arrays.
-        Up to GRID_MIN_AGENTS agents one workgroup runs the whole simulation
-        out of LDS; larger instances spread every step over the whole GPU
+        Up to EXCHANGE_MAX_AGENTS agents every draw of the run is made first
+        and one workgroup runs the exchange out of LDS; larger instances (and
+        runs above GRID_MIN_AGENTS whose draws would take more than
+        DRAW_BUFFER_MAX_BYTES) spread every step over the whole GPU
         (abm_wealth_run_grid).  Same results either way."""
         keys = self.key_table(steps)
         mean = torch.empty(max(steps, 1), dtype=torch.float32, device=self.device)
         gini = torch.empty(max(steps, 1), dtype=torch.float32, device=self.device)
-        if self.n > GRID_MIN_AGENTS:
-            # draws computed inline by the step kernels: no draw buffer
-            host = self.descriptor(keys, steps, mean, gini)
+        if self.n > GRID_MIN_AGENTS and (self.n > EXCHANGE_MAX_AGENTS or
+                                         12 * self.n * steps > DRAW_BUFFER_MAX_BYTES):
+            # draws computed inline by the step kernels; scratch for the
+            # second copies of what one launch per step reads and adds to
+            scratch = self.draw_buffer(1)
+            host = self.descriptor(keys, steps, mean, gini, scratch)
             acc = torch.empty(WEALTH_GRID_ACC_WORDS, dtype=torch.int32, device=self.device)
             check(lib().abm_wealth_run_grid(host.ctypes.data, ptr(acc), self.mode,
                                             stream_handle()), "wealth_run_grid")

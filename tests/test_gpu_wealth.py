@@ -199,3 +199,60 @@ def test_batch_of_split_and_whole_runs(wealth):
         np.testing.assert_array_equal(gini.cpu().numpy()[:s], og[:s])
         for a, b in ((e.w, w), (e.x, x), (e.y, y)):
             np.testing.assert_array_equal(a.cpu().numpy(), b)
+
+
+def _run_grid(eng, steps, scratch):
+    import torch
+
+    from jaxabm_amd._lib import WEALTH_GRID_ACC_WORDS, check, lib, ptr, stream_handle
+
+    keys = eng.key_table(steps)
+    mean = torch.empty(steps, dtype=torch.float32, device=eng.device)
+    gini = torch.empty(steps, dtype=torch.float32, device=eng.device)
+    acc = torch.empty(WEALTH_GRID_ACC_WORDS, dtype=torch.int32, device=eng.device)
+    buf = eng.draw_buffer(1).fill_(-1) if scratch else None
+    host = eng.descriptor(keys, steps, mean, gini, buf)
+    check(lib().abm_wealth_run_grid(host.ctypes.data, ptr(acc), eng.mode, stream_handle()), "run")
+    return mean.cpu().numpy(), gini.cpu().numpy()
+
+
+# below, at and above the smallest instance that takes one launch per step, one
+# and two tiles of agents a workgroup; wealth above the LDS bins
+@pytest.mark.parametrize("n,steps,rich", [(1032, 5, 0), (1033, 6, 0), (1280, 1, 0), (20_000, 25, 5000),
+                                          (2 * 256 * 4096 + 3, 3, 0)])
+@pytest.mark.parametrize("scratch", [False, True])
+def test_grid_run_one_and_two_launches_match_oracle(wealth, n, steps, rich, scratch):
+    import os
+
+    import torch
+
+    for mode in (O.MODE_PARTITIONABLE, O.MODE_ORIGINAL):
+        eng = wealth.WealthEngine(n, seed=9, mode=mode)
+        x, y, w, rng = O.wealth_init(n, 9, mode)
+        if rich:
+            w[:] = 0
+            w[20:10020] = 1
+            w[7] = rich
+            eng.w.copy_(torch.from_numpy(w.copy()).to(eng.w.device))
+        mean, gini = _run_grid(eng, steps, scratch)
+        om, og = O.wealth_run_threads(x, y, w, rng, steps,
+                                      max(1, min(16, os.cpu_count() or 1)), mode)
+        assert not rich or w.max() > 1024
+        np.testing.assert_array_equal(mean, om)
+        np.testing.assert_array_equal(gini, og)
+        for a, b in ((eng.w, w), (eng.x, x), (eng.y, y)):
+            np.testing.assert_array_equal(a.cpu().numpy(), b)
+        assert not eng.inc.any() and not eng.hist.any()   # left zero for the next run
+
+
+def test_engine_routes_give_the_same_bits(wealth, monkeypatch):
+    """The exchange run and the run over the whole GPU of one engine size."""
+    n, steps = 12_001, 9
+    a, b = wealth.WealthEngine(n, seed=4), wealth.WealthEngine(n, seed=4)
+    ra = a.run(steps)
+    monkeypatch.setattr(wealth, "DRAW_BUFFER_MAX_BYTES", 12 * n * steps - 1)
+    rb = b.run(steps)
+    for u, v in zip(ra, rb):
+        np.testing.assert_array_equal(u, v)
+    for t in ("w", "x", "y"):
+        np.testing.assert_array_equal(getattr(a, t).cpu().numpy(), getattr(b, t).cpu().numpy())
