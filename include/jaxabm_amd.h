@@ -369,6 +369,11 @@ typedef struct abm_deffuant_problem {
  * this descriptor, so that segment is not recomputed.  A second backward of
  * the same forward must clear it (the first one overwrites traj). */
 #define ABM_DEFFUANT_TAPE_LAST 1
+/* flags bit, the same in the forward and the backward of a descriptor: ckpt[j]
+ * for j >= 1, traj and lam are the library's own (no layout promised), which
+ * lets a run keep each instance's opinions on chip where that is faster.
+ * ckpt[0], work and every result are as without it. */
+#define ABM_DEFFUANT_COLUMNS 2
 /* x[i][b] = uniform(split(init_key, n)[i]) for every instance b. */
 int abm_deffuant_init(const uint32_t *init_key, int64_t n, int32_t batch, float *x, int mode,
                       void *stream);

@@ -62,7 +62,8 @@ class SchellingGrid(C.Structure):
     ]
 
 
-DEFFUANT_TAPE_LAST = 1  # abm_deffuant_problem.flags bit
+DEFFUANT_TAPE_LAST = 1  # abm_deffuant_problem.flags bits
+DEFFUANT_COLUMNS = 2
 
 
 class DeffuantProblem(C.Structure):

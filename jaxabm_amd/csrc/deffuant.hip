@@ -31,7 +31,14 @@
 // Checkpoints: the forward keeps the state at every ckpt_every-th step; the
 // backward recomputes each segment's states from its checkpoint, then sweeps
 // the segment in reverse.
+//
+// Column runs (ABM_DEFFUANT_COLUMNS): the instances never meet, so one
+// workgroup can keep the opinions of one instance in LDS and run all its
+// steps in one launch, where the step kernels above read and write the whole
+// batch once per step.  See "column runs" below.
 #include <hip/hip_runtime.h>
+
+#include <mutex>
 
 #include "common.hpp"
 #include "jaxabm_amd.h"
@@ -312,14 +319,11 @@ __global__ void k_deffuant_loss(const double *__restrict__ sums, int64_t n, int3
   loss[b] = L;
 }
 
-// lam[i][b] = dL/dx_i for instance b from the final state.
-__global__ void k_deffuant_lambda(const float *__restrict__ x, int64_t n, int32_t B,
-                                  const double *__restrict__ stats,
-                                  const double *__restrict__ coef, float *__restrict__ lam) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n * B) return;
-  const int b = (int)(idx % B);
-  const double xi = (double)x[idx];
+// dL/dx for the final opinion x of an agent of instance b.
+__device__ __forceinline__ float lambda_at(float x, int b, int32_t B,
+                                           const double *__restrict__ stats,
+                                           const double *__restrict__ coef) {
+  const double xi = (double)x;
   const double e4 = exp(4.0);
   double g = coef[b] + coef[B + b] * (xi - stats[(int64_t)b * kStatLen]);
   double t = exp(-kHistSlope * xi);
@@ -332,7 +336,352 @@ __global__ void k_deffuant_lambda(const float *__restrict__ x, int64_t n, int32_
     g += coef[(int64_t)(2 + k) * B + b] * kHistSlope * (ds_prev - ds);
     ds_prev = ds;
   }
-  lam[idx] = (float)g;
+  return (float)g;
+}
+
+// lam[i][b] = dL/dx_i for instance b from the final state.
+__global__ void k_deffuant_lambda(const float *__restrict__ x, int64_t n, int32_t B,
+                                  const double *__restrict__ stats,
+                                  const double *__restrict__ coef, float *__restrict__ lam) {
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= n * B) return;
+  lam[idx] = lambda_at(x[idx], (int)(idx % B), B, stats, coef);
+}
+
+// ---- column runs: one workgroup, one instance, all steps in one launch
+//
+// The opinions x (and in the backward the adjoints lam) of one instance live
+// in LDS, indexed by agent; a step is, per pair, two LDS reads, the gate, two
+// LDS writes, and one barrier.  HBM sees the pairings (shared by all
+// instances, so mostly L2), the checkpoints, and a tape of the pairs'
+// differences d = x_c - x_a: a step's adjoint needs nothing else of the
+// state, and in pair order the tape is written and read coalesced, at 2 bytes
+// an agent and step where a step kernel moves 8 (forward) or 12 (adjoint).
+// What bounds a step is then the gate's arithmetic (VALU).
+//
+// Layouts: ckpt[0] and work as ever ([n][B]); ckpt[j], j >= 1, and lam as
+// [B][n]; tape of one step [B][n / 2], a segment's steps in traj (k n / 2 <=
+// (k - 1) n floats an instance for k >= 2).  With k = 1 there are no
+// checkpoints to recompute from: step t's tape takes the first half of
+// ckpt[t] (step 0's the second half of ckpt[1]), and every backward sweeps it.
+constexpr int kColLds = 160 * 1024;
+constexpr int kColStatic = 512;                          // reduction scratch
+constexpr int64_t kColAgents = (kColLds - kColStatic) / 4;  // n floats in LDS
+constexpr int kColThreads = 1024;
+// P, the pairs a thread holds per iteration: 1 while a thread has no more than
+// one pair (a step is then one chain of latencies), 4 where it has several.
+
+struct ColumnRun {
+  int32_t n, B, steps, k;
+  const int32_t *perms;
+  const float *eps, *mu;
+  float *work, *ckpt, *traj, *lam;
+  double *grads;
+  int32_t tape_last;  // traj holds (forward: receives) the last segment's tape
+};
+
+// Instance of workgroup blk.  Workgroups go to the 8 XCDs in turn; within 256
+// of them each XCD gets 32 neighbouring instances, one 128-byte line of a row
+// of [n][B], so that its L2 reads and writes those rows whole.
+__device__ __forceinline__ int32_t column_of(int32_t blk, int32_t B) {
+  const int32_t base = blk & ~255, r = blk & 255;
+  return base + 256 <= B ? base + (r & 7) * 32 + (r >> 3) : blk;
+}
+
+__device__ __forceinline__ void column_barrier() {
+  // orders LDS only: the tape and the next pairings may stay in flight
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// x / kGateScale rounded once, in three operations: with y = 50 the rounded
+// reciprocal, q + (x - q c) y corrects q = x y to the rounded quotient
+// (Markstein, IBM J. Res. Dev. 34(1), 1990).  Equal to the IEEE division for
+// every float32 of [2^-60, 1.6] (all tested); below, the gate is 1 / 2 either
+// way.
+__device__ __forceinline__ float div_gate_scale(float x) {
+  const float q = x * 50.0f;
+  return fmaf(fmaf(-q, kGateScale, x), 50.0f, q);
+}
+
+// 1 / d rounded once for 1 <= d < 2^120: the hardware estimate (1 ulp) and two
+// corrections (the second exact, Markstein as above).
+__device__ __forceinline__ float inv_rounded(float d) {
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
+
+// The gates of P differences, the same bits as gate(): its quotients
+// by div_gate_scale and inv_rounded, and abm_expf without its range branches,
+// for |eps - |d|| <= 1.6 (|z| <= 80); any other argument of the wavefront, NaN
+// included, sends it through gate().  34 operations a gate instead of about 58.
+template <int P>
+__device__ __forceinline__ void gates(float eps, const float (&d)[P], float (&g)[P]) {
+  bool odd = false;
+#pragma unroll
+  for (int u = 0; u < P; ++u) {
+    const float num = eps - fabsf(d[u]);
+    odd |= !(fabsf(num) <= 1.6f);
+    const float x = -div_gate_scale(num);
+    const float m = __builtin_rintf(x * 0x1.715476p0f);
+    const float r = (x - m * 0x1.62e4p-1f) - m * 0x1.7f7d1cp-20f;
+    float q = 0x1.a01a02p-13f;
+    q = 0x1.6c16c2p-10f + q * r;
+    q = 0x1.111112p-7f + q * r;
+    q = 0x1.555556p-5f + q * r;
+    q = 0x1.555556p-3f + q * r;
+    q = 0.5f + q * r;
+    const float p = 1.0f + (r + (r * r) * q);
+    g[u] = inv_rounded(1.0f + __builtin_ldexpf(p, (int)m));  // exact: no subnormal here
+  }
+  if (__ballot(odd)) {
+#pragma unroll
+    for (int u = 0; u < P; ++u) g[u] = gate(eps, d[u]);
+  }
+}
+
+// Accesses below go through raw buffers of one row: a pair past the end loads
+// pair (0, 0) and stores nothing, without a branch around the access (which
+// would make every later wait a full one).
+using ColBuffer = __amdgpu_buffer_rsrc_t;
+using ColPair = unsigned __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ ColBuffer col_buffer(const void *p, int32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000);
+}
+
+// Threads of the workgroup: with P > 1 always kColThreads.
+template <int P>
+__device__ __forceinline__ int32_t col_threads() {
+  return P > 1 ? kColThreads : (int32_t)__builtin_amdgcn_readfirstlane(blockDim.x);
+}
+
+// A step's pairs in rounds of P x kColThreads (P = 1: one round).
+template <int P>
+__device__ __forceinline__ int32_t col_rounds(int32_t npairs) {
+  return P > 1 ? (npairs + P * kColThreads - 1) / (P * kColThreads) : 1;
+}
+
+// Pair u of a thread in round r.
+template <int P>
+__device__ __forceinline__ int32_t col_pair(int32_t r, int u) {
+  return (r * P + u) * kColThreads + (int32_t)threadIdx.x;
+}
+
+template <int P>
+struct ColPairs {
+  ColPair p[P];
+};
+template <int P>
+__device__ __forceinline__ ColPairs<P> load_pairs(const ColumnRun &a, int32_t t, int32_t r) {
+  ColPairs<P> v;
+  const ColBuffer b = col_buffer(a.perms + (int64_t)t * a.n, 8 * (a.n >> 1));
+#pragma unroll
+  for (int u = 0; u < P; ++u)
+    v.p[u] = __builtin_amdgcn_raw_buffer_load_b64(b, 8 * col_pair<P>(r, u), 0, 0);
+  return v;
+}
+
+// Steps t0 .. t1 - 1 on the opinions x; step t's differences go to tape(t)
+// where that is not null; after(t) runs with every thread past step t.
+template <int P, class Tape, class After>
+__device__ __forceinline__ void column_steps(const ColumnRun &a, float *x, int32_t t0, int32_t t1,
+                                             float eps, float mu, Tape tape, After after) {
+  const int32_t npairs = a.n >> 1, rounds = col_rounds<P>(npairs);
+  ColPairs<P> pr = load_pairs<P>(a, t0, 0);
+  for (int32_t t = t0; t < t1; ++t) {
+    float *out = tape(t);
+    const ColBuffer tb = col_buffer(out, out ? 4 * npairs : 0);
+    for (int32_t r = 0; r < rounds; ++r) {
+      // the next pairs, of this step or the next (after the last: its own)
+      const bool more = r + 1 < rounds;
+      const ColPairs<P> nx =
+          load_pairs<P>(a, more || t + 1 == t1 ? t : t + 1, more ? r + 1 : 0);
+      float xa[P], xc[P], d[P], g[P];
+#pragma unroll
+      for (int u = 0; u < P; ++u) {
+        xa[u] = x[pr.p[u].x];
+        xc[u] = x[pr.p[u].y];
+        d[u] = xc[u] - xa[u];
+      }
+      gates<P>(eps, d, g);
+#pragma unroll
+      for (int u = 0; u < P; ++u) {
+        const float delta = (mu * g[u]) * d[u];
+        if (col_pair<P>(r, u) < npairs) {
+          x[pr.p[u].x] = xa[u] + delta;
+          x[pr.p[u].y] = xc[u] - delta;
+        }
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(d[u]), tb, 4 * col_pair<P>(r, u), 0,
+                                              0);
+      }
+      pr = nx;
+    }
+    column_barrier();
+    after(t);
+  }
+}
+
+// Row of step t's tape in the k = 1 layout.
+__device__ __forceinline__ float *column_full_tape(const ColumnRun &a, int32_t t, int32_t b) {
+  const int64_t nB = (int64_t)a.n * a.B, half = a.n >> 1;
+  return a.ckpt + (t ? t * nB : nB + half * a.B) + half * b;
+}
+
+template <int P>
+__global__ void __launch_bounds__(kColThreads) k_deffuant_column_forward(ColumnRun a) {
+  extern __shared__ float col_x[];
+  const int32_t b = column_of(blockIdx.x, a.B), tid = threadIdx.x, T = col_threads<P>();
+  const int64_t nB = (int64_t)a.n * a.B, half = a.n >> 1;
+  for (int32_t i = tid; i < a.n; i += T) col_x[i] = a.ckpt[(int64_t)i * a.B + b];
+  column_barrier();
+  const int32_t t_last = (a.steps - 1) / a.k * a.k;
+  int32_t next = a.k;  // steps done at the next checkpoint
+  auto tape = [&](int32_t t) -> float * {
+    if (a.k == 1) return column_full_tape(a, t, b);
+    return a.tape_last && t >= t_last ? a.traj + (t - t_last) * half * a.B + half * b : nullptr;
+  };
+  auto after = [&](int32_t t) {
+    if (a.k == 1 || t + 1 != next || t + 1 == a.steps) return;
+    float *c = a.ckpt + (int64_t)((t + 1) / a.k) * nB + (int64_t)b * a.n;
+    for (int32_t i = tid; i < a.n; i += T) c[i] = col_x[i];
+    next += a.k;
+    column_barrier();  // before the next step writes
+  };
+  column_steps<P>(a, col_x, 0, a.steps, a.eps[b], a.mu[b], tape, after);
+  for (int32_t i = tid; i < a.n; i += T) a.work[(int64_t)i * a.B + b] = col_x[i];
+}
+
+// Reverse sweep of steps t1 - 1 .. t0 on the adjoints l.
+template <int P, class Tape>
+__device__ __forceinline__ void column_sweep(const ColumnRun &a, float *l, int32_t t0, int32_t t1,
+                                             float eps, float mu, Tape tape, double &ge,
+                                             double &gm) {
+  const int32_t npairs = a.n >> 1, rounds = col_rounds<P>(npairs);
+  auto load_d = [&](int32_t t, int32_t r, float (&d)[P]) {
+    const ColBuffer tb = col_buffer(tape(t), 4 * npairs);
+#pragma unroll
+    for (int u = 0; u < P; ++u)
+      d[u] = __uint_as_float(
+          __builtin_amdgcn_raw_buffer_load_b32(tb, 4 * col_pair<P>(r, u), 0, 0));
+  };
+  ColPairs<P> pr = load_pairs<P>(a, t1 - 1, 0);
+  float d[P];
+  load_d(t1 - 1, 0, d);
+  for (int32_t t = t1 - 1; t >= t0; --t) {
+    for (int32_t r = 0; r < rounds; ++r) {
+      const bool more = r + 1 < rounds;
+      const int32_t tn = more || t == t0 ? t : t - 1, rn = more ? r + 1 : 0;
+      const ColPairs<P> nx = load_pairs<P>(a, tn, rn);
+      float dn[P], la[P], lc[P], g[P];
+      load_d(tn, rn, dn);
+#pragma unroll
+      for (int u = 0; u < P; ++u) {
+        la[u] = l[pr.p[u].x];
+        lc[u] = l[pr.p[u].y];
+      }
+      gates<P>(eps, d, g);
+#pragma unroll
+      for (int u = 0; u < P; ++u) {
+        const float gp = div_gate_scale(g[u] * (1.0f - g[u]));
+        const float fd = mu * (g[u] - fabsf(d[u]) * gp);
+        const float fe = mu * d[u] * gp;
+        const float fm = g[u] * d[u];
+        const bool pair = col_pair<P>(r, u) < npairs;
+        const float w = pair ? la[u] - lc[u] : 0.0f;
+        if (pair) {
+          l[pr.p[u].x] = la[u] - w * fd;
+          l[pr.p[u].y] = lc[u] + w * fd;
+        }
+        ge += (double)(w * fe);
+        gm += (double)(w * fm);
+        d[u] = dn[u];
+      }
+      pr = nx;
+    }
+    column_barrier();
+  }
+}
+
+// The whole backward of one instance: per segment from the last, the steps
+// again from its checkpoint with their tape (unless the forward left it),
+// then the sweep.  kBoth: x and lam both fit LDS; otherwise they take turns,
+// lam waiting in its global column meanwhile.
+template <bool kBoth, int P>
+__global__ void __launch_bounds__(kColThreads) k_deffuant_column_backward(ColumnRun a) {
+  extern __shared__ float col_mem[];
+  __shared__ double red[2][kColThreads / 64];
+  const int32_t b = column_of(blockIdx.x, a.B), tid = threadIdx.x, T = col_threads<P>();
+  const int64_t nB = (int64_t)a.n * a.B, half = a.n >> 1;
+  float *x = col_mem, *l = kBoth ? col_mem + a.n : col_mem;
+  float *column = a.lam + (int64_t)b * a.n;
+  const float eps = a.eps[b], mu = a.mu[b];
+  double ge = 0.0, gm = 0.0;
+  const int32_t len = a.k == 1 ? a.steps : a.k;  // steps a segment
+  const int32_t nseg = (a.steps + len - 1) / len;
+  for (int32_t j = nseg - 1; j >= 0; --j) {
+    const int32_t t0 = j * len, t1 = t0 + len < a.steps ? t0 + len : a.steps;
+    auto tape = [&](int32_t t) -> float * {
+      return a.k == 1 ? column_full_tape(a, t, b) : a.traj + (t - t0) * half * a.B + half * b;
+    };
+    if (a.k > 1 && !(a.tape_last && j == nseg - 1)) {
+      if (j == 0) {
+        for (int32_t i = tid; i < a.n; i += T) x[i] = a.ckpt[(int64_t)i * a.B + b];
+      } else {
+        const float *c = a.ckpt + j * nB + (int64_t)b * a.n;
+        for (int32_t i = tid; i < a.n; i += T) x[i] = c[i];
+      }
+      column_barrier();
+      column_steps<P>(a, x, t0, t1, eps, mu, tape, [](int32_t) {});
+    }
+    if (!kBoth || j == nseg - 1) {
+      for (int32_t i = tid; i < a.n; i += T) l[i] = column[i];
+      column_barrier();
+    }
+    column_sweep<P>(a, l, t0, t1, eps, mu, tape, ge, gm);
+    if (!kBoth && j > 0) {
+      for (int32_t i = tid; i < a.n; i += T) column[i] = l[i];
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    ge += __shfl_xor(ge, off);
+    gm += __shfl_xor(gm, off);
+  }
+  if ((tid & 63) == 0) {
+    red[0][tid >> 6] = ge;
+    red[1][tid >> 6] = gm;
+  }
+  __syncthreads();
+  if (tid < 2) {
+    double s = 0.0;
+    for (int w = 0; w < (T >> 6); ++w) s += red[tid][w];
+    a.grads[(int64_t)tid * a.B + b] = s;
+  }
+}
+
+// k_deffuant_lambda into columns: lam[b][i], tiles of 64 agents x 16 instances
+// turned in LDS.
+__global__ void __launch_bounds__(256)
+    k_deffuant_lambda_columns(const float *__restrict__ x, int64_t n, int32_t B,
+                              const double *__restrict__ stats, const double *__restrict__ coef,
+                              float *__restrict__ lam) {
+  __shared__ float tile[16][65];
+  const int64_t i0 = (int64_t)blockIdx.x * 64;
+  const int32_t b0 = blockIdx.y * 16;
+#pragma unroll 1
+  for (int r = threadIdx.x >> 4; r < 64; r += 16) {
+    const int c = threadIdx.x & 15;
+    const int64_t i = i0 + r;
+    if (i < n && b0 + c < B) tile[c][r] = lambda_at(x[i * B + b0 + c], b0 + c, B, stats, coef);
+  }
+  __syncthreads();
+  for (int c = threadIdx.x >> 6; c < 16; c += 4) {
+    const int r = threadIdx.x & 63;
+    if (i0 + r < n && b0 + c < B) lam[(int64_t)(b0 + c) * n + i0 + r] = tile[c][r];
+  }
 }
 
 __global__ void k_deffuant_init(const uint32_t *__restrict__ init_key, int64_t n, int32_t B,
@@ -396,6 +745,75 @@ void launch_loss(const abm_deffuant_problem *p, const float *x, hipStream_t s) {
                      p->loss, p->coef);
 }
 
+// Whether a flagged descriptor takes the column run; the same answer in the
+// forward and the backward of one descriptor.
+bool column_run(const abm_deffuant_problem *p) {
+  if (!(p->flags & ABM_DEFFUANT_COLUMNS) || p->n > kColAgents || p->steps < 1) return false;
+  if (p->ckpt_every == 1 ? p->steps < 2 : !p->traj) return false;
+  return true;
+}
+
+ColumnRun column_args(const abm_deffuant_problem *p) {
+  ColumnRun a;
+  a.n = (int32_t)p->n;
+  a.B = p->batch;
+  a.steps = p->steps;
+  a.k = p->ckpt_every;
+  a.perms = p->perms;
+  a.eps = p->eps;
+  a.mu = p->mu;
+  a.work = p->work;
+  a.ckpt = p->ckpt;
+  a.traj = p->traj;
+  a.lam = p->lam;
+  a.grads = p->grads;
+  a.tape_last = (p->flags & ABM_DEFFUANT_TAPE_LAST) != 0;
+  return a;
+}
+
+// One pair a thread, whole wavefronts, up to a full workgroup.
+unsigned column_threads(int64_t n) {
+  const int64_t t = ((n >> 1) + 63) / 64 * 64;
+  return (unsigned)(t < kColThreads ? t : kColThreads);
+}
+
+using ColumnKernel = void (*)(ColumnRun);
+
+ColumnKernel column_forward(int64_t n) {
+  return (n >> 1) <= kColThreads ? k_deffuant_column_forward<1> : k_deffuant_column_forward<4>;
+}
+
+bool column_both(int64_t n) { return 2 * n <= kColAgents; }
+
+ColumnKernel column_backward(int64_t n) {
+  if ((n >> 1) <= kColThreads) return k_deffuant_column_backward<true, 1>;
+  return column_both(n) ? k_deffuant_column_backward<true, 4>
+                        : k_deffuant_column_backward<false, 4>;
+}
+
+constexpr int kMaxDevices = 64;
+std::mutex g_column_attr_mu;
+bool g_column_attr_set[kMaxDevices];
+
+// The column kernels need more than 64 KB of dynamic LDS: the limit is raised
+// once per device, under a lock.
+int column_lds_attr() {
+  int dev = -1;
+  ABM_CHECK_HIP(hipGetDevice(&dev));
+  ABM_REQUIRE(dev >= 0 && dev < kMaxDevices, "deffuant: device index out of range");
+  std::lock_guard<std::mutex> lock(g_column_attr_mu);
+  if (!g_column_attr_set[dev]) {
+    for (const ColumnKernel k :
+         {k_deffuant_column_forward<1>, k_deffuant_column_forward<4>,
+          k_deffuant_column_backward<true, 1>, k_deffuant_column_backward<true, 4>,
+          k_deffuant_column_backward<false, 4>})
+      ABM_CHECK_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)(kColAgents * 4)));
+    g_column_attr_set[dev] = true;
+  }
+  return kOk;
+}
+
 int check_problem(const abm_deffuant_problem *p, const char *who, bool backward) {
   bool ok = p && p->n >= 2 && p->n < (1ll << 31) && p->batch >= 1 && p->steps >= 0 &&
             p->ckpt_every >= 1 && p->pair_blocks >= 1 && p->pair_blocks <= 65535 &&
@@ -442,6 +860,14 @@ int abm_deffuant_step(const float *src, float *dst, int64_t n, int32_t batch,
 int abm_deffuant_forward(const abm_deffuant_problem *p, void *stream) {
   if (int rc = check_problem(p, "abm_deffuant_forward", false)) return rc;
   hipStream_t s = (hipStream_t)stream;
+  if (column_run(p)) {
+    if (int rc = column_lds_attr()) return rc;
+    hipLaunchKernelGGL(column_forward(p->n), dim3((unsigned)p->batch),
+                       dim3(column_threads(p->n)), (size_t)p->n * 4, s, column_args(p));
+    launch_loss(p, p->work, s);
+    ABM_LAUNCH_CHECK("abm_deffuant_forward");
+    return kOk;
+  }
   const int64_t nB = p->n * (int64_t)p->batch;
   const int32_t k = p->ckpt_every;
   // first step of the last segment; with the tape flag its steps write traj
@@ -471,6 +897,16 @@ int abm_deffuant_backward(const abm_deffuant_problem *p, void *stream) {
   const int64_t n = p->n, nB = n * (int64_t)p->batch;
   const int32_t k = p->ckpt_every;
   const float *final_x = p->steps > 0 ? p->work : p->ckpt;
+  if (column_run(p)) {
+    if (int rc = column_lds_attr()) return rc;
+    hipLaunchKernelGGL(k_deffuant_lambda_columns, dim3(nblocks(n, 64), nblocks(p->batch, 16)),
+                       dim3(256), 0, s, final_x, n, p->batch, (const double *)p->stats,
+                       (const double *)p->coef, p->lam);
+    hipLaunchKernelGGL(column_backward(n), dim3((unsigned)p->batch), dim3(column_threads(n)),
+                       (size_t)n * (column_both(n) ? 8 : 4), s, column_args(p));
+    ABM_LAUNCH_CHECK("abm_deffuant_backward");
+    return kOk;
+  }
   hipLaunchKernelGGL(k_deffuant_lambda, dim3(nblocks(nB, 256)), dim3(256), 0, s, final_x, n,
                      p->batch, (const double *)p->stats, (const double *)p->coef, p->lam);
   const int64_t acc_len = (int64_t)p->pair_blocks * 2 * p->batch;

@@ -27,8 +27,8 @@ import numpy as np
 import torch
 
 from .. import random as jr
-from .._lib import (DEFFUANT_TAPE_LAST, DeffuantProblem, check, lib, ptr, require_gpu,
-                    stream_handle)
+from .._lib import (DEFFUANT_COLUMNS, DEFFUANT_TAPE_LAST, DeffuantProblem, check, lib, ptr,
+                    require_gpu, stream_handle)
 
 STATS_LEN = 34
 HIST_BINS = 32
@@ -107,7 +107,8 @@ class DeffuantModel:
 
     def _problem(self, flags: int = 0) -> DeffuantProblem:
         p = DeffuantProblem()
-        p.n, p.batch, p.steps, p.flags = self.n, self.batch, self.steps, flags
+        p.n, p.batch, p.steps = self.n, self.batch, self.steps
+        p.flags = flags | DEFFUANT_COLUMNS
         p.ckpt_every, p.pair_blocks, p.stat_chunks = (self.ckpt_every, self.pair_blocks,
                                                       self.stat_chunks)
         for name in ("perms", "eps", "mu", "work", "ckpt", "traj", "lam", "acc", "partial",

@@ -244,3 +244,46 @@ def test_batch_size_does_not_change_an_instance(dm):
         out.append((loss[:41], ge[:41], gm[:41]))
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+# Column runs against the step kernels: pairs per thread 1 and 4 (1,024 and
+# 1,025 pairs), opinions and adjoints both in LDS or in turn (20,416 agents and
+# above), the largest column and the next size (step kernels on both sides),
+# whole lines of instances and a rest, every tape layout (k = 1, 2, one
+# segment, a last segment of one step), one step.
+@pytest.mark.parametrize("n,B,steps,k", [(2, 1, 5, 2), (3, 2, 4, 1), (65, 5, 7, 3),
+                                         (2048, 3, 6, 2), (2049, 3, 6, 6), (2050, 2, 5, 1),
+                                         (2051, 257, 4, 3), (8191, 4, 5, 4), (20416, 2, 5, 2),
+                                         (20417, 3, 7, 3), (20418, 2, 4, 1), (40832, 2, 5, 2),
+                                         (40833, 2, 3, 2), (1000, 2, 1, 2), (1000, 2, 1, 1)])
+def test_column_run_equals_step_kernels(dm, monkeypatch, n, B, steps, k):
+    rs = np.random.default_rng(n + B)
+    eps = rs.uniform(0.05, 0.5, B).astype(np.float32)
+    mu = rs.uniform(0.05, 0.5, B).astype(np.float32)
+    # confidence bounds whose gate argument leaves the short form of the gate
+    eps[0] = 2.5
+    if B > 3:
+        eps[1], eps[2], eps[3] = -3.0, np.inf, 1.6
+    target = rs.uniform(0.0, 0.1, 34)
+    got = []
+    for flag in (0, 2):
+        monkeypatch.setattr(dm, "DEFFUANT_COLUMNS", flag)
+        m = dm.DeffuantModel(n, B, steps, seed=2, ckpt_every=k)
+        loss = m.forward(eps, mu, target).cpu().numpy()
+        first = [g.cpu().numpy() for g in m.backward()]
+        again = [g.cpu().numpy() for g in m.backward()]   # every segment recomputed
+        for a, b in zip(first, again):
+            np.testing.assert_array_equal(a, b)
+        got.append((m.final_state().cpu().numpy(), m.x0.cpu().numpy(), loss, *first))
+    (x, x0, loss, ge, gm), (cx, cx0, closs, cge, cgm) = got
+    np.testing.assert_array_equal(cx, x)
+    np.testing.assert_array_equal(cx0, x0)
+    np.testing.assert_array_equal(closs, loss)
+    # the same float32 terms, summed in float64 in another order: n / 2 * steps
+    # terms of size up to the largest gradient's, each rounding below 2^-53
+    tol = n * steps * 2.0 ** -53
+    for a, b in ((cge, ge), (cgm, gm)):
+        fin = np.isfinite(b)
+        np.testing.assert_array_equal(np.isfinite(a), fin)
+        scale = np.abs(b[fin]).max() if fin.any() else 0.0
+        np.testing.assert_allclose(a[fin], b[fin], rtol=max(tol, 1e-12) * 100, atol=scale * tol * 100)
