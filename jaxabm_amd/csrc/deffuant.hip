@@ -48,6 +48,9 @@ namespace abm {
 constexpr float kGateScale = 0.02f;
 constexpr int kDefThreads = 256;
 constexpr int kDefWaves = kDefThreads / 64;
+// most row chunks of the statistics: two wavefronts per SIMD at 256 columns,
+// and eight rounds of loads to sum them
+constexpr int64_t kStatChunks = 512;
 constexpr int kStatLen = 2 + 32;
 constexpr int kHistBins = 32;
 constexpr double kHistSlope = 128.0;
@@ -233,15 +236,21 @@ __device__ __forceinline__ double inv_one_plus(double t) {
   return r;
 }
 
-// Per-chunk float64 partial sums of one instance column:
+// Per-chunk float64 partial sums of the instance columns:
 // [sum x, sum (x - 1/2)^2, hist_0 .. hist_31] -> partial[chunk][34][B].
 // sigmoid(128 (x - k/32)) = 1 / (1 + t e^(4k)) with t = e^(-128 x).
+// A workgroup is `cols` columns (a power of two, up to its threads) by
+// kDefThreads / cols chunks, so that a small batch fills its lanes too.  What
+// a chunk is and how the chunks are summed depends on n alone: an instance's
+// statistics do not depend on the batch it runs in.  Bound by the 33
+// reciprocals an opinion (float64 VALU).
 __global__ void __launch_bounds__(kDefThreads)
-    k_deffuant_stats(const float *__restrict__ x, int64_t n, int32_t B, int64_t rows,
-                     double *__restrict__ partial) {
-  const int b = blockIdx.x * kDefThreads + threadIdx.x;
-  if (b >= B) return;
-  const int64_t i0 = (int64_t)blockIdx.y * rows;
+    k_deffuant_stats(const float *__restrict__ x, int64_t n, int32_t B, int32_t cols,
+                     int64_t rows, int64_t chunks, double *__restrict__ partial) {
+  const int b = blockIdx.x * cols + (threadIdx.x & (cols - 1));
+  const int64_t chunk = (int64_t)blockIdx.y * (kDefThreads / cols) + threadIdx.x / cols;
+  if (b >= B || chunk >= chunks) return;
+  const int64_t i0 = chunk * rows;
   const int64_t i1 = i0 + rows < n ? i0 + rows : n;
   const double e4 = exp(4.0);
   double s1 = 0.0, s2 = 0.0, h[kHistBins];
@@ -261,7 +270,7 @@ __global__ void __launch_bounds__(kDefThreads)
       prev = cur;
     }
   }
-  double *out = partial + (int64_t)blockIdx.y * kStatLen * B + b;
+  double *out = partial + chunk * kStatLen * B + b;
   out[0] = s1;
   out[B] = s2;
 #pragma unroll
@@ -269,26 +278,36 @@ __global__ void __launch_bounds__(kDefThreads)
 }
 
 // out[j][b] = sum over r of in[r][j][b], for j = blockIdx.y; 64 columns per
-// block, 4 row groups combined in a fixed order.
-__global__ void __launch_bounds__(256)
+// block, kSumGroups row groups of four loads in flight, combined in a fixed
+// order.
+constexpr int kSumGroups = 16;
+
+__global__ void __launch_bounds__(64 * kSumGroups)
     k_sum_rows(const double *__restrict__ in, int64_t rows, int32_t J, int32_t B,
                double *__restrict__ out) {
-  __shared__ double red[4][64];
+  __shared__ double red[kSumGroups][64];
   const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
   const int b = blockIdx.x * 64 + lane;
   const int j = blockIdx.y;
-  double s0 = 0.0, s1 = 0.0;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
   if (b < B) {
-    int64_t r = g;
-    for (; r + 4 < rows; r += 8) {
-      s0 += in[(r * J + j) * B + b];
-      s1 += in[((r + 4) * J + j) * B + b];
+    for (int64_t r = g; r < rows; r += 4 * kSumGroups) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[u] = r + u * kSumGroups < rows ? in[((r + u * kSumGroups) * J + j) * B + b] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s[u] += v[u];
     }
-    for (; r < rows; r += 4) s0 += in[(r * J + j) * B + b];
   }
-  red[g][lane] = s0 + s1;
+  red[g][lane] = (s[0] + s[1]) + (s[2] + s[3]);
   __syncthreads();
-  if (g == 0 && b < B) out[(int64_t)j * B + b] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+  if (g == 0 && b < B) {
+    double t = 0.0;
+#pragma unroll
+    for (int q = 0; q < kSumGroups; ++q) t += red[q][lane];
+    out[(int64_t)j * B + b] = t;
+  }
 }
 
 // stats[b][34], loss[b] and the coefficients of dL/dx (coef[34][B]:
@@ -301,20 +320,28 @@ __global__ void k_deffuant_loss(const double *__restrict__ sums, int64_t n, int3
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= B) return;
   const double dn = (double)n;
-  const double m = sums[b] / dn;
-  const double v = sums[B + b] / dn - (m - 0.5) * (m - 0.5);
-  const double w0 = weights ? weights[0] : 1.0, w1 = weights ? weights[1] : 1.0;
-  double L = w0 * (m - target[0]) * (m - target[0]) + w1 * (v - target[1]) * (v - target[1]);
+  double sum[kStatLen], aim[kStatLen], wt[kStatLen];  // all loads in flight at once
+#pragma unroll
+  for (int k = 0; k < kStatLen; ++k) {
+    sum[k] = sums[(int64_t)k * B + b];
+    aim[k] = target[k];
+    wt[k] = weights ? weights[k] : 1.0;
+  }
+  const double m = sum[0] / dn;
+  const double v = sum[1] / dn - (m - 0.5) * (m - 0.5);
+  const double w0 = wt[0], w1 = wt[1];
+  double L = w0 * (m - aim[0]) * (m - aim[0]) + w1 * (v - aim[1]) * (v - aim[1]);
   stats[(int64_t)b * kStatLen] = m;
   stats[(int64_t)b * kStatLen + 1] = v;
-  coef[b] = w0 * 2.0 * (m - target[0]) / dn;
-  coef[B + b] = w1 * 2.0 * (v - target[1]) * 2.0 / dn;
+  coef[b] = w0 * 2.0 * (m - aim[0]) / dn;
+  coef[B + b] = w1 * 2.0 * (v - aim[1]) * 2.0 / dn;
+#pragma unroll
   for (int k = 0; k < kHistBins; ++k) {
-    const double hk = sums[(int64_t)(2 + k) * B + b] / dn;
-    const double wk = weights ? weights[2 + k] : 1.0;
+    const double hk = sum[2 + k] / dn;
+    const double wk = wt[2 + k];
     stats[(int64_t)b * kStatLen + 2 + k] = hk;
-    L += wk * (hk - target[2 + k]) * (hk - target[2 + k]);
-    coef[(int64_t)(2 + k) * B + b] = wk * 2.0 * (hk - target[2 + k]) / dn;
+    L += wk * (hk - aim[2 + k]) * (hk - aim[2 + k]);
+    coef[(int64_t)(2 + k) * B + b] = wk * 2.0 * (hk - aim[2 + k]) / dn;
   }
   loss[b] = L;
 }
@@ -662,24 +689,26 @@ __global__ void __launch_bounds__(kColThreads) k_deffuant_column_backward(Column
   }
 }
 
-// k_deffuant_lambda into columns: lam[b][i], tiles of 64 agents x 16 instances
-// turned in LDS.
+// k_deffuant_lambda into columns: lam[b][i], tiles of R agents x 16 instances
+// turned in LDS; R = 64 writes whole lines, R = 16 spreads a small batch over
+// more workgroups (1,001 x 12: 18 us with 64, 8 with 16).
+template <int R>
 __global__ void __launch_bounds__(256)
     k_deffuant_lambda_columns(const float *__restrict__ x, int64_t n, int32_t B,
                               const double *__restrict__ stats, const double *__restrict__ coef,
                               float *__restrict__ lam) {
-  __shared__ float tile[16][65];
-  const int64_t i0 = (int64_t)blockIdx.x * 64;
+  __shared__ float tile[16][R + 1];
+  const int64_t i0 = (int64_t)blockIdx.x * R;
   const int32_t b0 = blockIdx.y * 16;
 #pragma unroll 1
-  for (int r = threadIdx.x >> 4; r < 64; r += 16) {
+  for (int r = threadIdx.x >> 4; r < R; r += 16) {
     const int c = threadIdx.x & 15;
     const int64_t i = i0 + r;
     if (i < n && b0 + c < B) tile[c][r] = lambda_at(x[i * B + b0 + c], b0 + c, B, stats, coef);
   }
   __syncthreads();
-  for (int c = threadIdx.x >> 6; c < 16; c += 4) {
-    const int r = threadIdx.x & 63;
+  for (int c = threadIdx.x / R; c < 16; c += 256 / R) {
+    const int r = threadIdx.x & (R - 1);
     if (i0 + r < n && b0 + c < B) lam[(int64_t)(b0 + c) * n + i0 + r] = tile[c][r];
   }
 }
@@ -734,13 +763,17 @@ void launch_adjoint(const float *x_pre, float *lam, int64_t n, int32_t B, const 
 }
 
 void launch_loss(const abm_deffuant_problem *p, const float *x, hipStream_t s) {
-  const int64_t rows = (p->n + p->stat_chunks - 1) / p->stat_chunks;
+  int32_t cols = 1;
+  while (cols < p->batch && cols < kDefThreads) cols *= 2;
+  const int64_t most = p->stat_chunks < kStatChunks ? p->stat_chunks : kStatChunks;
+  const int64_t rows = (p->n + most - 1) / most;
   const int64_t chunks = (p->n + rows - 1) / rows;
-  hipLaunchKernelGGL(k_deffuant_stats, dim3(nblocks(p->batch, kDefThreads), (unsigned)chunks),
-                     dim3(kDefThreads), 0, s, x, p->n, p->batch, rows, p->partial);
-  hipLaunchKernelGGL(k_sum_rows, dim3(nblocks(p->batch, 64), (unsigned)kStatLen), dim3(256), 0,
-                     s, (const double *)p->partial, chunks, kStatLen, p->batch, p->sums);
-  hipLaunchKernelGGL(k_deffuant_loss, dim3(nblocks(p->batch, 256)), dim3(256), 0, s,
+  hipLaunchKernelGGL(k_deffuant_stats,
+                     dim3(nblocks(p->batch, cols), nblocks(chunks, kDefThreads / cols)),
+                     dim3(kDefThreads), 0, s, x, p->n, p->batch, cols, rows, chunks, p->partial);
+  hipLaunchKernelGGL(k_sum_rows, dim3(nblocks(p->batch, 64), (unsigned)kStatLen),
+                     dim3(64 * kSumGroups), 0, s, (const double *)p->partial, chunks, kStatLen, p->batch, p->sums);
+  hipLaunchKernelGGL(k_deffuant_loss, dim3(nblocks(p->batch, 64)), dim3(64), 0, s,
                      (const double *)p->sums, p->n, p->batch, p->target, p->weights, p->stats,
                      p->loss, p->coef);
 }
@@ -899,8 +932,9 @@ int abm_deffuant_backward(const abm_deffuant_problem *p, void *stream) {
   const float *final_x = p->steps > 0 ? p->work : p->ckpt;
   if (column_run(p)) {
     if (int rc = column_lds_attr()) return rc;
-    hipLaunchKernelGGL(k_deffuant_lambda_columns, dim3(nblocks(n, 64), nblocks(p->batch, 16)),
-                       dim3(256), 0, s, final_x, n, p->batch, (const double *)p->stats,
+    const bool wide = nblocks(n, 64) * (int64_t)nblocks(p->batch, 16) >= 1024;
+    hipLaunchKernelGGL(wide ? k_deffuant_lambda_columns<64> : k_deffuant_lambda_columns<16>,
+                       dim3(nblocks(n, wide ? 64 : 16), nblocks(p->batch, 16)), dim3(256), 0, s, final_x, n, p->batch, (const double *)p->stats,
                        (const double *)p->coef, p->lam);
     hipLaunchKernelGGL(column_backward(n), dim3((unsigned)p->batch), dim3(column_threads(n)),
                        (size_t)n * (column_both(n) ? 8 : 4), s, column_args(p));
@@ -930,7 +964,7 @@ int abm_deffuant_backward(const abm_deffuant_problem *p, void *stream) {
                      p->pair_blocks, p->acc, s);
     }
   }
-  hipLaunchKernelGGL(k_sum_rows, dim3(nblocks(p->batch, 64), 2u), dim3(256), 0, s,
+  hipLaunchKernelGGL(k_sum_rows, dim3(nblocks(p->batch, 64), 2u), dim3(64 * kSumGroups), 0, s,
                      (const double *)p->acc, (int64_t)p->pair_blocks, 2, p->batch, p->grads);
   ABM_LAUNCH_CHECK("abm_deffuant_backward");
   return kOk;
