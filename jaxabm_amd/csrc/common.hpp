@@ -22,6 +22,17 @@ template <class T>
 __device__ __forceinline__ GlobalPtr<T> as_global(T *p) {
   return (GlobalPtr<T>)p;
 }
+// The same for code that takes plain pointers: the compiler follows the
+// address space from the cast on, past a barrier that keeps it from cancelling
+// the two casts.  p must be the same for the whole wavefront.
+template <class T>
+__device__ __forceinline__ T *in_global(T *p) {
+  GlobalPtr<T> g = (GlobalPtr<T>)p;
+#ifdef __HIP_DEVICE_COMPILE__
+  asm("" : "+s"(g));
+#endif
+  return (T *)g;
+}
 
 // Integer threshold for `uniform < p` on [0,1): with m = bits >> 9,
 // u = m * 2^-23 exactly, so u < p  <=>  m < ceil(p * 2^23) (p in (0, 1]).

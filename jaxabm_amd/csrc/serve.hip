@@ -45,6 +45,7 @@
 #include <unordered_map>
 #include <vector>
 
+#define ABM_STRAIGHT_DRAWS
 #include "common.hpp"
 #include "jaxabm_amd.h"
 
@@ -94,6 +95,27 @@ struct Inst {
 struct Range {
   int32_t inst, begin, end, kind;
 };
+
+// An instance as a kernel uses it: every array is global memory.
+__device__ __forceinline__ Inst load_inst(const Inst *p) {
+  Inst in = *p;
+  in.keys = in_global(in.keys);
+  in.row_ptr = in_global(in.row_ptr);
+  in.col = in_global(in.col);
+  in.state0 = in_global(in.state0);
+  in.state1 = in_global(in.state1);
+  in.mark = in_global(in.mark);
+  in.counts = in_global(in.counts);
+  in.x = in_global(in.x);
+  in.y = in_global(in.y);
+  in.w = in_global(in.w);
+  in.inc = in_global(in.inc);
+  in.hist = in_global(in.hist);
+  in.acc = in_global(in.acc);
+  in.mean = in_global(in.mean);
+  in.gini = in_global(in.gini);
+  return in;
+}
 
 // ---------------------------------------------------------------- block helpers
 template <int THREADS>
@@ -204,9 +226,15 @@ __device__ void wealth_record(int64_t n, uint32_t T, uint32_t S, float *mean, fl
   gini[t] = g;
 }
 
-// Agent phase of one wealth agent; returns the exchange target or -1.
-__device__ __forceinline__ int32_t wealth_agent(const Inst &in, int64_t i, Key ck, Key kk1,
-                                                Key kk2, uint32_t span, int mode) {
+// Exchange target of a wealth agent.
+__device__ __forceinline__ uint32_t wealth_target(const Inst &in, int64_t i, Key kk1, Key kk2,
+                                                  uint32_t span, int mode) {
+  uint32_t ti = randint_offset(bits_at(kk1, in.n, i, mode), bits_at(kk2, in.n, i, mode), span);
+  return ti + (ti >= (uint32_t)i ? 1u : 0u);
+}
+
+// Position walk of a wealth agent.
+__device__ __forceinline__ void wealth_walk(const Inst &in, int64_t i, Key ck, int mode) {
   Key k1, k2;
   split2(split_at(ck, in.n, i, mode), k1, k2, mode);
   const float dx = normal_from_bits(bits_scalar(k1, mode));
@@ -215,10 +243,32 @@ __device__ __forceinline__ int32_t wealth_agent(const Inst &in, int64_t i, Key c
   const float sy = in.y[i] + 0.01f * dy;
   in.x[i] = mod1(sx);
   in.y[i] = mod1(sy);
-  if (in.w[i] <= 0) return -1;
-  uint32_t ti = randint_offset(bits_at(kk1, in.n, i, mode), bits_at(kk2, in.n, i, mode), span);
-  ti += ti >= (uint32_t)i ? 1u : 0u;
-  return (int32_t)ti;
+}
+
+// Entries of a row that a thread (a lane of a wavefront) has in flight: a row
+// scanned entry by entry costs two dependent memory round trips an entry, and
+// a step waits for its longest row (48 requests: 47 us a step, 31 with eight
+// in flight).
+constexpr int kRowLoads = 8;
+
+// Bit k: entry e + k * stride of the row (below e1) has an infected neighbour.
+__device__ __forceinline__ uint32_t infected_entries(const Inst &in, const uint8_t *old, int32_t e,
+                                                     int32_t e1, int32_t stride) {
+  int32_t c[kRowLoads];
+  uint8_t st[kRowLoads];
+#pragma unroll
+  for (int k = 0; k < kRowLoads; ++k) {
+    // past the end: the last entry again, left out below
+    const int32_t at = e + k * stride;
+    c[k] = in.col[at < e1 ? at : e1 - 1];
+  }
+#pragma unroll
+  for (int k = 0; k < kRowLoads; ++k) st[k] = old[c[k]];
+  uint32_t m = 0;
+#pragma unroll
+  for (int k = 0; k < kRowLoads; ++k)
+    if (e + k * stride < e1 && st[k] == 1) m |= 1u << k;
+  return m;
 }
 
 // Next SIR state of a light row (scanned by one thread).
@@ -226,8 +276,10 @@ __device__ __forceinline__ uint8_t sir_light(const Inst &in, const uint8_t *old,
                                              uint8_t s, int32_t e0, int32_t e1, Key kinf,
                                              Key krec, int mode) {
   if (s == 0) {
-    for (int32_t e = e0; e < e1; ++e)
-      if (old[in.col[e]] == 1 && (bits_at(kinf, in.nnz, e, mode) >> 9) < in.thr_beta) return 1;
+    for (int32_t e = e0; e < e1; e += kRowLoads) {
+      for (uint32_t m = infected_entries(in, old, e, e1, 1); m; m &= m - 1)
+        if ((bits_at(kinf, in.nnz, e + __builtin_ctz(m), mode) >> 9) < in.thr_beta) return 1;
+    }
     return 0;
   }
   if (s == 1) return (bits_at(krec, in.n, v, mode) >> 9) < in.thr_gamma ? 2 : 1;
@@ -239,13 +291,29 @@ __device__ __forceinline__ uint8_t sir_light(const Inst &in, const uint8_t *old,
 __device__ __forceinline__ bool sir_heavy_hit(const Inst &in, const uint8_t *old, int32_t e0,
                                               int32_t e1, Key kinf, int mode) {
   const int lane = threadIdx.x & 63;
-  for (int32_t base = e0; base < e1; base += 64) {
-    const int32_t e = base + lane;
-    const bool mine = e < e1 && old[in.col[e]] == 1 &&
-                      (bits_at(kinf, in.nnz, e, mode) >> 9) < in.thr_beta;
+  for (int32_t base = e0; base < e1; base += 64 * kRowLoads) {
+    bool mine = false;
+    for (uint32_t m = infected_entries(in, old, base + lane, e1, 64); m && !mine; m &= m - 1)
+      mine = (bits_at(kinf, in.nnz, base + lane + 64 * __builtin_ctz(m), mode) >> 9) < in.thr_beta;
     if (__ballot(mine)) return true;
   }
   return false;
+}
+
+// mark[u] = m for the neighbours u of a row: its entries e, e + stride, ..
+__device__ __forceinline__ void mark_row(const Inst &in, int32_t e, int32_t e1, int32_t stride,
+                                         uint16_t m) {
+  for (; e < e1; e += kRowLoads * stride) {
+    int32_t c[kRowLoads];
+#pragma unroll
+    for (int k = 0; k < kRowLoads; ++k) {
+      const int32_t at = e + k * stride;
+      c[k] = in.col[at < e1 ? at : e1 - 1];
+    }
+#pragma unroll
+    for (int k = 0; k < kRowLoads; ++k)
+      if (e + k * stride < e1) in.mark[c[k]] = m;
+  }
 }
 
 // ---------------------------------------------------------------- resident path
@@ -253,7 +321,7 @@ __device__ __forceinline__ bool sir_heavy_hit(const Inst &in, const uint8_t *old
 // after the heavy rows and the counts.  The S/I/R counts and the heavy-row
 // count live in LDS, double-buffered by step parity: a step's buffer is
 // reset during the step before it, after every thread has read it.
-__device__ void sir_resident(const Inst &in, int32_t t_end, int mode, uint8_t *lds,
+__device__ __forceinline__ void sir_resident(const Inst &in, int32_t t_end, int mode, uint8_t *lds,
                              int32_t *heavy, int32_t *nheavy2, uint32_t *cnt2) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t n = in.n;
@@ -345,7 +413,7 @@ __device__ void sir_resident(const Inst &in, int32_t t_end, int mode, uint8_t *l
 // instance's global bins, which wave 0 clears as it reads them.  The packed
 // increments of agents 2j and 2j + 1 are read and cleared by one thread
 // before the second barrier.
-__device__ void wealth_resident(const Inst &in, int32_t t_end, int mode, uint8_t *lds,
+__device__ __forceinline__ void wealth_resident(const Inst &in, int32_t t_end, int mode, uint8_t *lds,
                                 uint32_t *red) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t n = in.n;
@@ -366,9 +434,10 @@ __device__ void wealth_resident(const Inst &in, int32_t t_end, int mode, uint8_t
     Key kk1, kk2;
     split2(uk, kk1, kk2, mode);
     for (int64_t i = tid; i < n; i += kResThreads) {
-      const int32_t ti = wealth_agent(in, i, ck, kk1, kk2, span, mode);
+      const uint32_t ti = wealth_target(in, i, kk1, kk2, span, mode);
       // an agent receives at most n - 1 < 2^16 units per step: no carry
-      if (ti >= 0) atomicAdd(&inc2[ti >> 1], 1u << ((ti & 1) * 16));
+      if (in.w[i] > 0) atomicAdd(&inc2[ti >> 1], 1u << ((ti & 1) * 16));
+      wealth_walk(in, i, ck, mode);
     }
     __syncthreads();
     for (int b = tid; b < kHistLds; b += kResThreads) prev[b] = 0;
@@ -423,21 +492,21 @@ __device__ void wealth_resident(const Inst &in, int32_t t_end, int mode, uint8_t
   }
 }
 
+template <int kMode>
 __global__ void __launch_bounds__(kResThreads)
-    k_serve_resident(const Inst *__restrict__ insts, const int32_t *__restrict__ list, int32_t K,
-                     int mode) {
+    k_serve_resident(const Inst *__restrict__ insts, const int32_t *__restrict__ list, int32_t K) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ int32_t heavy[kResHeavyCap];
   __shared__ int32_t nheavy2[2];
   __shared__ uint32_t cnt2[6];
   __shared__ uint32_t red[kResWaves];
-  const Inst in = insts[list[blockIdx.x]];
+  const Inst in = load_inst(insts + list[blockIdx.x]);
   const int32_t t_end = min(in.t0 + K, in.steps);
   if (in.t0 >= t_end) return;
   if (in.kind == kSir)
-    sir_resident(in, t_end, mode, lds, heavy, nheavy2, cnt2);
+    sir_resident(in, t_end, kMode, lds, heavy, nheavy2, cnt2);
   else
-    wealth_resident(in, t_end, mode, lds, red);
+    wealth_resident(in, t_end, kMode, lds, red);
 }
 
 // ---------------------------------------------------------------- stepwise path
@@ -457,11 +526,14 @@ __device__ void wealth_stepwise_record(const Inst &in, int32_t t, uint32_t *red,
 // t - 1 and the agent phase of step t touch each agent from the same thread;
 // step t's increments go to the other inc copy, so no agent reads an
 // increment of the step being drawn.
-__device__ void wealth_stepwise(const Inst &in, const Range &r, int32_t t, int mode,
+__device__ __forceinline__ void wealth_stepwise(const Inst &in, const Range &r, int32_t t, int mode,
                                 uint32_t *red, uint32_t *carry, uint32_t *bins) {
   const int tid = threadIdx.x;
   const int64_t n = in.n;
-  if (r.begin == 0 && t >= 2) wealth_stepwise_record(in, t - 2, red, carry);  // block-uniform
+  if (r.begin < 0) {  // block-uniform
+    if (t >= 2) wealth_stepwise_record(in, t - 2, red, carry);
+    return;
+  }
   const bool apply = t >= 1 && t - 1 < in.steps;  // block-uniform
   const bool draw = t < in.steps;
   int32_t *inc_old = in.inc + (int64_t)((t + 1) & 1) * n;  // step t - 1's increments
@@ -478,10 +550,11 @@ __device__ void wealth_stepwise(const Inst &in, const Range &r, int32_t t, int m
   }
   const uint32_t span = (uint32_t)(n - 1);
   uint32_t total = 0;
+#pragma unroll 1
   for (int64_t i = r.begin + tid; i < r.end; i += kStepThreads) {
+    int32_t wi = in.w[i];
     if (apply) {
-      const int32_t w0 = in.w[i];
-      const int32_t wi = w0 - (w0 > 0 ? 1 : 0) + inc_old[i];
+      wi = wi - (wi > 0 ? 1 : 0) + inc_old[i];
       in.w[i] = wi;
       inc_old[i] = 0;
       total += (uint32_t)wi;
@@ -491,8 +564,11 @@ __device__ void wealth_stepwise(const Inst &in, const Range &r, int32_t t, int m
         atomicAdd(&hist[wi], 1);  // 0 <= wi <= n: wealth is conserved
     }
     if (draw) {
-      const int32_t ti = wealth_agent(in, i, ck, kk1, kk2, span, mode);
-      if (ti >= 0) atomicAdd(&inc_new[ti], 1);
+      // the unit first, so that its atomic (device-wide these run at 26 per
+      // ns) goes on beside the walk's draws instead of after them
+      const uint32_t ti = wealth_target(in, i, kk1, kk2, span, mode);
+      if (wi > 0) atomicAdd(&inc_new[ti], 1);
+      wealth_walk(in, i, ck, mode);
     }
   }
   if (apply) {
@@ -506,14 +582,15 @@ __device__ void wealth_stepwise(const Inst &in, const Range &r, int32_t t, int m
 }
 
 // Phase 1 of sub-step s, the one launch per step: SIR step of the range, or
-// for wealth (t = t0 + s): the record of step t - 2 (by the block of the
-// instance's first range), the exchange of step t - 1 applied to the range's
-// agents (wealth, histogram, total and maximum), then step t's agent phase
+// for wealth (t = t0 + s): the record of step t - 2 (by a workgroup of its
+// own, a range that begins at -1), the exchange of step t - 1 applied to the
+// range's agents (wealth, histogram, total and maximum), then step t's agent phase
 // (positions and exchange increments).  A wealth instance runs two sub-steps
 // past its last step to apply and record it.
+template <int kMode>
 __global__ void __launch_bounds__(kStepThreads)
-    k_serve_phase1(const Inst *__restrict__ insts, const Range *__restrict__ ranges, int32_t s,
-                   int mode) {
+    k_serve_phase1(const Inst *__restrict__ insts, const Range *__restrict__ ranges, int32_t s) {
+  constexpr int mode = kMode;
   __shared__ int32_t heavy[kStepHeavyCap];
   __shared__ int32_t marking[kStepHeavyCap];
   __shared__ int32_t nheavy, nmark;
@@ -521,7 +598,7 @@ __global__ void __launch_bounds__(kStepThreads)
   __shared__ uint32_t carry;
   __shared__ uint32_t bins[kStepBins];
   const Range r = ranges[blockIdx.x];
-  const Inst in = insts[r.inst];
+  const Inst in = load_inst(insts + r.inst);
   const int32_t t = in.t0 + s;
   if (in.kind == kWealth) {
     if (t >= in.steps + 2) return;  // block-uniform
@@ -584,7 +661,7 @@ __global__ void __launch_bounds__(kStepThreads)
           continue;
         }
       }
-      for (int32_t e = e0; e < e1; ++e) in.mark[in.col[e]] = new_mark;
+      mark_row(in, e0, e1, 1, new_mark);
     }
   }
   __syncthreads();
@@ -599,13 +676,12 @@ __global__ void __launch_bounds__(kStepThreads)
       cs += !hit;
     }
     if (hit)  // wave-uniform: the newly infected hub marks its neighbours
-      for (int32_t e = e0 + lane; e < e1; e += 64) in.mark[in.col[e]] = new_mark;
+      mark_row(in, e0 + lane, e1, 64, new_mark);
   }
   const int32_t nm = min(nmark, kStepHeavyCap);
   for (int32_t h = wave; h < nm; h += kStepWaves) {
     const int32_t v = marking[h];
-    for (int32_t e = in.row_ptr[v] + lane; e < in.row_ptr[v + 1]; e += 64)
-      in.mark[in.col[e]] = new_mark;
+    mark_row(in, in.row_ptr[v] + lane, in.row_ptr[v + 1], 64, new_mark);
   }
   cs = block_sum<kStepThreads>(cs, red);
   ci = block_sum<kStepThreads>(ci, red);
@@ -652,8 +728,7 @@ __global__ void k_serve_seed_sir(Inst in, const int32_t *__restrict__ infected, 
   if (i < n0) {
     const int32_t v = infected[i];
     in.state0[v] = 1;
-    for (int32_t e = in.row_ptr[v]; e < in.row_ptr[v + 1]; ++e)
-      in.mark[in.col[e]] = (uint16_t)kMarkHorizon;
+    mark_row(in, in.row_ptr[v], in.row_ptr[v + 1], 1, (uint16_t)kMarkHorizon);
   }
 }
 
@@ -809,6 +884,14 @@ class Server {
   void sched_loop();
   bool sched_once();
   int launch_tick();
+  auto *resident_kernel() const {
+    return cfg_.mode == kModePartitionable ? k_serve_resident<kModePartitionable>
+                                           : k_serve_resident<kModeOriginal>;
+  }
+  auto *phase1_kernel() const {
+    return cfg_.mode == kModePartitionable ? k_serve_phase1<kModePartitionable>
+                                           : k_serve_phase1<kModeOriginal>;
+  }
   bool retire_tick(bool block);
   void admit();
   void activate_uploads();
@@ -866,7 +949,7 @@ int Server::start() {
   ABM_CHECK_HIP(hipMalloc(&base, cfg_.hbm_budget));
   dev_base_ = (char *)base;
   arena_.init(cfg_.hbm_budget);
-  ABM_CHECK_HIP(hipFuncSetAttribute((const void *)k_serve_resident,
+  ABM_CHECK_HIP(hipFuncSetAttribute((const void *)resident_kernel(),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResLds));
   if (int rc = ensure_tables(cfg_.max_active, 4096)) return rc;
   for (int i = 0; i < cfg_.prep_threads; ++i) workers_.emplace_back([this] { prep_loop(); });
@@ -1229,7 +1312,7 @@ int Server::launch_tick() {
   const int32_t K = cfg_.steps_per_tick;
   size_t n1 = 0;
   for (Req *r : active_)
-    if (!r->resident) n1 += r->ranges.size() - 1;
+    if (!r->resident) n1 += r->ranges.size() - (r->d.kind == kWealth ? 0 : 1);
   if (int rc = ensure_tables(active_.size(), n1)) return rc;
   TableSet &ts = sets_[tick_idx_ % kSets];
   const size_t o1 = align256(sizeof(Inst) * active_.size());
@@ -1246,6 +1329,11 @@ int Server::launch_tick() {
   int32_t nres = 0;
   size_t i1 = 0;
   Tick tick;
+  // the wealth instances' records first: a workgroup each, so that none of
+  // them delays the agents of a range
+  for (size_t i = 0; i < active_.size(); ++i)
+    if (!active_[i]->resident && active_[i]->d.kind == kWealth)
+      h1[i1++] = Range{(int32_t)i, -1, -1, kWealth};
   for (size_t i = 0; i < active_.size(); ++i) {
     Req *r = active_[i];
     hi[i] = r->d;
@@ -1268,11 +1356,11 @@ int Server::launch_tick() {
   ABM_CHECK_HIP(hipEventRecord(ev_tab_, sW_));
   ABM_CHECK_HIP(hipStreamWaitEvent(sR_, ev_tab_, 0));
   if (nres)
-    hipLaunchKernelGGL(k_serve_resident, dim3((unsigned)nres), dim3(kResThreads), kResLds, sR_,
-                       di, dres, K, cfg_.mode);
+    hipLaunchKernelGGL(resident_kernel(), dim3((unsigned)nres), dim3(kResThreads), kResLds, sR_,
+                       di, dres, K);
   for (int32_t s = 0; i1 && s < K; ++s)
-    hipLaunchKernelGGL(k_serve_phase1, dim3((unsigned)i1), dim3(kStepThreads), 0, sW_, di, d1, s,
-                       cfg_.mode);
+    hipLaunchKernelGGL(phase1_kernel(), dim3((unsigned)i1), dim3(kStepThreads), 0, sW_, di, d1,
+                       s);
   ABM_LAUNCH_CHECK("serve tick");
   auto take = [this]() {
     if (!free_events_.empty()) {

@@ -61,34 +61,36 @@ __device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, uint32_t *red) {
   return s;  // valid in wave 0
 }
 
-// The draws of agent i at one step: the position increments 0.01 * normal
-// (rounded as the reference's product) and the exchange target.
-struct WealthDraw {
+// The draws of agent i at one step (ck: the collection key; kk1, kk2 =
+// split(uk), the same for every agent): the position increments 0.01 * normal
+// (rounded as the reference's product), and the exchange target.
+struct WealthWalk {
   float mdx, mdy;
-  uint32_t target;
 };
 
-// (ck: the collection key; kk1, kk2 = split(uk), the same for every agent).
-__device__ __forceinline__ WealthDraw wealth_draw(Key ck, Key kk1, Key kk2, int64_t n, int64_t i,
-                                                  int mode) {
+__device__ __forceinline__ WealthWalk wealth_walk(Key ck, int64_t n, int64_t i, int mode) {
   Key k1, k2;
   split2(split_at(ck, n, i, mode), k1, k2, mode);
-  WealthDraw d;
+  WealthWalk d;
   d.mdx = 0.01f * normal_from_bits(bits_scalar(k1, mode));
   d.mdy = 0.01f * normal_from_bits(bits_scalar(k2, mode));
-  const uint32_t span = n > 1 ? (uint32_t)(n - 1) : 1u;
-  uint32_t ti = randint_offset(bits_at(kk1, n, i, mode), bits_at(kk2, n, i, mode), span);
-  d.target = ti + (ti >= (uint32_t)i ? 1u : 0u);
   return d;
 }
 
-__device__ __forceinline__ WealthDraw wealth_draw(const uint32_t *keys, int32_t t, int64_t n,
-                                                  int64_t i, int mode) {
-  const Key ck{keys[4 * t + 0], keys[4 * t + 1]};
-  const Key uk{keys[4 * t + 2], keys[4 * t + 3]};
-  Key kk1, kk2;
-  split2(uk, kk1, kk2, mode);
-  return wealth_draw(ck, kk1, kk2, n, i, mode);
+__device__ __forceinline__ uint32_t wealth_target(Key kk1, Key kk2, int64_t n, int64_t i,
+                                                  int mode) {
+  const uint32_t span = n > 1 ? (uint32_t)(n - 1) : 1u;
+  uint32_t ti = randint_offset(bits_at(kk1, n, i, mode), bits_at(kk2, n, i, mode), span);
+  return ti + (ti >= (uint32_t)i ? 1u : 0u);
+}
+
+__device__ __forceinline__ Key collection_key(const uint32_t *keys, int32_t t) {
+  return Key{keys[4 * t + 0], keys[4 * t + 1]};
+}
+
+__device__ __forceinline__ void target_keys(const uint32_t *keys, int32_t t, Key &kk1, Key &kk2,
+                                            int mode) {
+  split2(Key{keys[4 * t + 2], keys[4 * t + 3]}, kk1, kk2, mode);
 }
 
 // Every draw of a run, grid-wide, into draws[steps][3][n] (mdx, mdy bits,
@@ -107,11 +109,13 @@ __global__ void __launch_bounds__(kDrawThreads)
     const int32_t t = (int32_t)(q / per);
     const int64_t i = (q - (int64_t)t * per) * kDrawThreads + threadIdx.x;
     if (i >= n) continue;
-    const WealthDraw d = wealth_draw(in.keys, t, n, i, kMode);
+    Key kk1, kk2;
+    target_keys(in.keys, t, kk1, kk2, kMode);
+    const WealthWalk d = wealth_walk(collection_key(in.keys, t), n, i, kMode);
     const GlobalPtr<uint32_t> row = as_global(in.draws) + (int64_t)t * 3 * n;
     row[i] = __float_as_uint(d.mdx);
     row[n + i] = __float_as_uint(d.mdy);
-    row[2 * n + i] = d.target;
+    row[2 * n + i] = wealth_target(kk1, kk2, n, i, kMode);
   }
 }
 
@@ -181,18 +185,22 @@ __device__ __forceinline__ void wealth_steps(const abm_wealth_inst &in, float *g
   for (int32_t t = 0; t < in.steps; ++t) {
     // agent phase + exchange targets
     for (int64_t i = tid; i < n; i += kWealthThreads) {
-      WealthDraw d;
+      WealthWalk d;
+      uint32_t target;
       if (in.draws) {
         const uint32_t *row = in.draws + (int64_t)t * 3 * n;
         d.mdx = __uint_as_float(row[i]);
         d.mdy = __uint_as_float(row[n + i]);
-        d.target = row[2 * n + i];
+        target = row[2 * n + i];
       } else {
-        d = wealth_draw(in.keys, t, n, i, mode);
+        Key kk1, kk2;
+        target_keys(in.keys, t, kk1, kk2, mode);
+        target = wealth_target(kk1, kk2, n, i, mode);
+        d = wealth_walk(collection_key(in.keys, t), n, i, mode);
       }
       gx[i] = mod1(gx[i] + d.mdx);
       gy[i] = mod1(gy[i] + d.mdy);
-      if (gw[i] > 0) atomicAdd(&ginc[d.target], 1);
+      if (gw[i] > 0) atomicAdd(&ginc[target], 1);
     }
     __syncthreads();
     // apply the exchange, histogram of wealth values
@@ -538,10 +546,14 @@ __global__ void __launch_bounds__(kGridThreads)
   const int64_t n = in.n;
   const int64_t stride = (int64_t)gridDim.x * kGridThreads;
   for (int64_t i = (int64_t)blockIdx.x * kGridThreads + threadIdx.x; i < n; i += stride) {
-    const WealthDraw d = wealth_draw(in.keys, t, n, i, mode);
+    // the unit first: see k_wealth_grid_step
+    Key kk1, kk2;
+    target_keys(in.keys, t, kk1, kk2, mode);
+    const uint32_t target = wealth_target(kk1, kk2, n, i, mode);
+    if (in.w[i] > 0) atomicAdd(&in.inc[target], 1);
+    const WealthWalk d = wealth_walk(collection_key(in.keys, t), n, i, mode);
     in.x[i] = mod1(in.x[i] + d.mdx);
     in.y[i] = mod1(in.y[i] + d.mdy);
-    if (in.w[i] > 0) atomicAdd(&in.inc[d.target], 1);
   }
 }
 
@@ -589,11 +601,11 @@ __global__ void __launch_bounds__(kGridThreads)
 // (increments of step t, bins of step t - 1) and what it reads and clears
 // (increments of step t - 1, bins of step t - 2) alternate between the two
 // copies, so no launch reads what another workgroup of it writes.  Launch
-// `steps` only applies, launch steps + 1 only records.  Of a step of 247,720
-// agents 6.4 us are its seven threefry blocks and two erf_inv an agent (1,020
-// operations, VALU); the rest is the launch, the loads before and the bins
-// after them.  Two launches a step, with the record in front of workgroup 0's
-// agents, took 14.0 us a step; this takes 11.8.
+// `steps` only applies, launch steps + 1 only records.  A step of 247,720
+// agents takes 11.0 us: 5.0 without the walk and the exchange's atomics, of
+// which the 156,000 (26 per ns, whatever their scope) take 5.9 and the walk's
+// five threefry blocks and two erf_inv 4.8 beside them.  Two launches a step,
+// with the record in front of workgroup 0's agents, took 14.0.
 // The keys that all agents share (split(uk) of the step) are made by workgroup
 // 0 of the launch before; in every thread they were 137 of 990 operations.
 struct WealthGrid {
@@ -696,8 +708,10 @@ __global__ void __launch_bounds__(kGridThreads)
       total += (uint32_t)wi;
     }
     if (t < in.steps) {
-      const WealthDraw d = wealth_draw(ck, kk1, kk2, n, i, kMode);
-      if (wi > 0) atomicAdd(&g.inc[cur][d.target], 1u);
+      // the unit first, so that its atomic runs beside the walk's draws
+      const uint32_t target = wealth_target(kk1, kk2, n, i, kMode);
+      if (wi > 0) atomicAdd(&g.inc[cur][target], 1u);
+      const WealthWalk d = wealth_walk(ck, n, i, kMode);
       in.x[i] = mod1(in.x[i] + d.mdx);
       in.y[i] = mod1(in.y[i] + d.mdy);
     }
