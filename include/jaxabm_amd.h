@@ -210,6 +210,17 @@ int abm_sir_seed(const abm_sir_graph *g, const int32_t *perm, int64_t n0, uint8_
 int abm_sir_run(const abm_sir_graph *g, uint8_t *state, uint16_t *mark, uint32_t *bitmaps,
                 uint32_t t0, const uint32_t *keys, int32_t steps, float beta, float gamma,
                 int mode, int32_t *slots, int32_t *counts, void *stream);
+/* abm_sir_run for a caller that waits for the counts anyway: the same results,
+ * but the host keeps only a few steps launched ahead and launches no more once
+ * one has begun without an infected agent (it and the steps after it are the
+ * identity; the step loop of jaxabm/model.py:146-216 has no such exit).
+ * watch: two words of pinned host memory, not in use by another run; *launched
+ * receives the number of steps launched.  Not for stream capture: the call
+ * returns when the last of them is launched. */
+int abm_sir_run_watched(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
+                        uint32_t *bitmaps, uint32_t t0, const uint32_t *keys, int32_t steps,
+                        float beta, float gamma, int mode, int32_t *slots, int32_t *counts,
+                        int32_t *watch, int32_t *launched, void *stream);
 /* One step: reads bitmap bm_in, writes bm_out, updates state in place;
  * accumulates into a zeroed slots[abm_sir_slots()][3].  prev_slots: the
  * previous step's slots (lets a step with no infected agent skip its work),

@@ -170,6 +170,8 @@ SIGNATURES = {
     "abm_sir_seed": (_int, [C.POINTER(SirGraph), _p, _i64, _p, _p, _p, _u32, _p]),
     "abm_sir_run": (_int, [C.POINTER(SirGraph), _p, _p, _p, _u32, _p, _i32, _f32, _f32,
                            _int, _p, _p, _p]),
+    "abm_sir_run_watched": (_int, [C.POINTER(SirGraph), _p, _p, _p, _u32, _p, _i32, _f32, _f32,
+                                   _int, _p, _p, _p, C.POINTER(_i32), _p]),
     "abm_sir_step": (_int, [C.POINTER(SirGraph), _p, _p, _p, _p, _u32, _p, _f32, _f32,
                             _int, _p, _p, _p]),
     "abm_sir_reduce_counts": (_int, [_p, _i32, _p, _p]),

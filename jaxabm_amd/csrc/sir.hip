@@ -98,7 +98,13 @@ struct SirStep {
   uint32_t thr_beta, thr_gamma;
   int mode;
   int32_t *slots;
+  int32_t *watch;  // host memory, or null: [0] steps begun, [1] 1 once one was the identity
+  int32_t begun;   // value for watch[0], or 0: this step does not tell
 };
+
+__device__ __forceinline__ void tell_host(int32_t *p, int32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Workgroup barrier that orders LDS only.  Every intra-block exchange in the
 // step kernel goes through LDS (state, marks and bitmaps are never read back
@@ -118,54 +124,44 @@ __device__ __forceinline__ bool at_risk(uint16_t m, uint32_t t) {
   return (uint16_t)(m - (uint16_t)t) <= kMarkHorizon;
 }
 
-// Rows of degree <= 32 are scanned by one lane, kScanGroup rows at a time:
-// the group's row bounds load together, then each round loads the next four
-// entries of every row still scanning together.  The S-I candidates of a
-// round are drawn in order (one draw site); a row stops at its first
-// infecting entry.  hitm bit g: row g of the group is infected.  One row per
-// group is the fastest on MI355X (1M-agent BA run: 8.44 us per step against
-// 9.07 with two rows and 10.15 with four): a busy step's scans are bound by
-// the draws and the slowest lane, not by the lanes' memory round trips.
-constexpr int kScanGroup = 1;
+// Entries of a row that one lane loads per round, as two 16-byte loads: a
+// lane's rows are scattered, so every load instruction of a wavefront touches
+// 64 lines, and entry by entry the same lines were fetched again and again
+// (they do not stay in the 32 KB L1).
+constexpr int kRowRound = 8;
 
-__device__ __forceinline__ uint32_t scan_light_group(const int32_t *__restrict__ col,
-                                                     const uint32_t *__restrict__ bm,
-                                                     int32_t (&e)[kScanGroup],
-                                                     const int32_t (&hi)[kScanGroup], Key kinf,
-                                                     int64_t nnz, uint32_t thr, int mode) {
-  uint32_t hitm = 0;
-  for (;;) {
-    uint32_t live = 0;
+// c[k] = col[e + k] for e + k < hi, else -1.
+__device__ __forceinline__ void load_row_round(const int32_t *__restrict__ col, int32_t e,
+                                               int32_t hi, int64_t nnz, int32_t (&c)[kRowRound]) {
+  if (e + kRowRound <= nnz) {
+    int32_t v[kRowRound];
+    __builtin_memcpy(v, col + e, 16);
+    __builtin_memcpy(v + 4, col + e + 4, 16);
 #pragma unroll
-    for (int g = 0; g < kScanGroup; ++g) live |= (uint32_t)(e[g] < hi[g]) << g;
-    if (!live) break;
-    int32_t c[kScanGroup][4];
+    for (int k = 0; k < kRowRound; ++k) c[k] = e + k < hi ? v[k] : -1;
+  } else {  // the last entries of the array
 #pragma unroll
-    for (int g = 0; g < kScanGroup; ++g)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) c[g][k] = e[g] + k < hi[g] ? col[e[g] + k] : -1;
-    uint32_t cm = 0;  // bit 4g + k: entry e[g] + k is an S-I candidate
-#pragma unroll
-    for (int g = 0; g < kScanGroup; ++g)
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (c[g][k] >= 0 && infected(bm, c[g][k])) cm |= 1u << (4 * g + k);
-    while (cm) {
-      const int bit = __builtin_ctz(cm);
-      cm &= cm - 1;
-      const int g = bit >> 2;
-      int32_t base = e[0];
-#pragma unroll
-      for (int q = 1; q < kScanGroup; ++q) base = g == q ? e[q] : base;
-      if ((bits_at(kinf, nnz, base + (bit & 3), mode) >> 9) < thr) {
-        hitm |= 1u << g;
-        cm &= ~(0xFu << (4 * g));
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < kScanGroup; ++g) e[g] = (hitm >> g) & 1u ? hi[g] : e[g] + 4;
+    for (int k = 0; k < kRowRound; ++k) c[k] = e + k < hi ? col[e + k] : -1;
   }
-  return hitm;
+}
+
+// A row of degree <= 32 scanned by one lane: each round tests kRowRound
+// entries and draws its S-I candidates in order, stopping at the first
+// infecting one.
+__device__ __forceinline__ bool scan_light(const int32_t *__restrict__ col,
+                                           const uint32_t *__restrict__ bm, int32_t e, int32_t hi,
+                                           Key kinf, int64_t nnz, uint32_t thr, int mode) {
+  for (; e < hi; e += kRowRound) {
+    int32_t c[kRowRound];
+    load_row_round(col, e, hi, nnz, c);
+    uint32_t cm = 0;
+#pragma unroll
+    for (int k = 0; k < kRowRound; ++k)
+      if (c[k] >= 0 && infected(bm, c[k])) cm |= 1u << k;
+    for (; cm; cm &= cm - 1)
+      if ((bits_at(kinf, nnz, e + __builtin_ctz(cm), mode) >> 9) < thr) return true;
+  }
+  return false;
 }
 
 // Scan of a long row by a whole wavefront (wave-uniform result): 8 x 64
@@ -197,54 +193,24 @@ __device__ __forceinline__ bool scan_heavy(const int32_t *__restrict__ col,
   return false;
 }
 
-// Marks of the rows of degree <= 32 of a group (as scan_light_group: the
-// next four entries of every row per round, loaded together).
-__device__ __forceinline__ void mark_light_group(const int32_t *__restrict__ col,
-                                                 uint16_t *__restrict__ mark,
-                                                 int32_t (&e)[kScanGroup],
-                                                 const int32_t (&hi)[kScanGroup], uint16_t m) {
-  for (;;) {
-    uint32_t live = 0;
+// Marks of a row of degree <= 32 by one lane.
+__device__ __forceinline__ void mark_light(const int32_t *__restrict__ col,
+                                           uint16_t *__restrict__ mark, int32_t e, int32_t hi,
+                                           int64_t nnz, uint16_t m) {
+  for (; e < hi; e += kRowRound) {
+    int32_t c[kRowRound];
+    load_row_round(col, e, hi, nnz, c);
 #pragma unroll
-    for (int g = 0; g < kScanGroup; ++g) live |= (uint32_t)(e[g] < hi[g]) << g;
-    if (!live) break;
-    int32_t c[kScanGroup][4];
-#pragma unroll
-    for (int g = 0; g < kScanGroup; ++g)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) c[g][k] = e[g] + k < hi[g] ? col[e[g] + k] : -1;
-#pragma unroll
-    for (int g = 0; g < kScanGroup; ++g) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (c[g][k] >= 0) mark[c[g][k]] = m;
-      e[g] += 4;
-    }
+    for (int k = 0; k < kRowRound; ++k)
+      if (c[k] >= 0) mark[c[k]] = m;
   }
 }
 
-// Row bounds of this lane's group of light items items[k0 + g * kSirThreads]
-// (g < kScanGroup, k < nl), loaded together; rows past nl are empty.
-__device__ __forceinline__ void light_group_rows(const SirStep &a, int64_t sub, int32_t k0,
-                                                 int32_t nl, const uint16_t *items,
-                                                 int (&loc)[kScanGroup],
-                                                 int32_t (&e)[kScanGroup],
-                                                 int32_t (&hi)[kScanGroup]) {
-#pragma unroll
-  for (int g = 0; g < kScanGroup; ++g) {
-    const int32_t k = k0 + g * kSirThreads;
-    loc[g] = k < nl ? (int)items[k] : -1;
-  }
-#pragma unroll
-  for (int g = 0; g < kScanGroup; ++g) {
-    e[g] = 0;
-    hi[g] = 0;
-    if (loc[g] >= 0) {
-      const int64_t u = sub + loc[g];
-      e[g] = a.row_ptr[u];
-      hi[g] = a.row_ptr[u + 1];
-    }
-  }
+// Row bounds of item k of a worklist (empty when k is past its end).
+__device__ __forceinline__ int2 item_bounds(const SirStep &a, int64_t sub, bool valid, int loc) {
+  if (!valid) return make_int2(0, 0);
+  const int64_t u = sub + loc;
+  return make_int2(a.row_ptr[u], a.row_ptr[u + 1]);
 }
 
 __device__ __forceinline__ void mark_heavy(const int32_t *__restrict__ col,
@@ -303,28 +269,34 @@ __device__ __forceinline__ void push_items(uint32_t lmask, uint32_t hmask, uint1
 template <int kMode>
 __device__ __forceinline__ void scan_items(const SirStep &a, const uint32_t *__restrict__ bm,
                                            int64_t sub, int32_t nl, int32_t nh,
-                                           const uint16_t *items, uint8_t *outb, Key kinf,
-                                           int32_t *next_heavy) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  for (;;) {
-    int32_t k = 0;
-    if (lane == 0) k = atomicAdd(next_heavy, 1);
-    k = __shfl(k, 0);
-    if (k >= nh) break;
-    const int loc = items[kTile - 1 - k];
-    const int64_t u = sub + loc;
-    const bool hit = scan_heavy(a.col, bm, a.row_ptr[u], a.row_ptr[u + 1], kinf, a.nnz,
-                                a.thr_beta, kMode);
-    if (lane == 0 && hit) outb[loc] = 1;
+                                           const uint16_t *items, uint8_t *outb, Key kinf) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // heavy rows wave, wave + 16, ..: lane j loads the bounds of the wave's row
+  // j, so that a row costs its entries' round trip and not two more before it
+  constexpr int kWaves = kSirThreads / 64;
+  for (int32_t k0 = wave; k0 < nh; k0 += kWaves * 64) {
+    const int32_t mine = k0 + lane * kWaves;
+    const int my_loc = mine < nh ? (int)items[kTile - 1 - mine] : 0;
+    const int2 my = item_bounds(a, sub, mine < nh, my_loc);
+    const int rows = (nh - k0 + kWaves - 1) / kWaves < 64 ? (nh - k0 + kWaves - 1) / kWaves : 64;
+    for (int j = 0; j < rows; ++j) {
+      const int loc = __builtin_amdgcn_readlane(my_loc, j);
+      const bool hit = scan_heavy(a.col, bm, __builtin_amdgcn_readlane(my.x, j),
+                                  __builtin_amdgcn_readlane(my.y, j), kinf, a.nnz, a.thr_beta,
+                                  kMode);
+      if (lane == 0 && hit) outb[loc] = 1;
+    }
   }
-  for (int32_t k0 = tid; k0 < nl; k0 += kSirThreads * kScanGroup) {
-    int loc[kScanGroup];
-    int32_t e[kScanGroup], hi[kScanGroup];
-    light_group_rows(a, sub, k0, nl, items, loc, e, hi);
-    const uint32_t hitm = scan_light_group(a.col, bm, e, hi, kinf, a.nnz, a.thr_beta, kMode);
-#pragma unroll
-    for (int g = 0; g < kScanGroup; ++g)
-      if ((hitm >> g) & 1u) outb[loc[g]] = 1;
+  // light rows, a lane each; the next row's bounds load under this one's scan
+  int loc = tid < nl ? (int)items[tid] : 0;
+  int2 at = item_bounds(a, sub, tid < nl, loc);
+  for (int32_t k = tid; k < nl; k += kSirThreads) {
+    const int32_t kn = k + kSirThreads;
+    const int next_loc = kn < nl ? (int)items[kn] : 0;
+    const int2 next = item_bounds(a, sub, kn < nl, next_loc);
+    if (scan_light(a.col, bm, at.x, at.y, kinf, a.nnz, a.thr_beta, kMode)) outb[loc] = 1;
+    loc = next_loc;
+    at = next;
   }
 }
 
@@ -333,10 +305,11 @@ __global__ void __launch_bounds__(kSirThreads) k_sir_step(SirStep a) {
   extern __shared__ uint4 lds_bm4[];  // kLds: the bitmap words
   __shared__ __align__(16) uint8_t outb[kTile];
   __shared__ __align__(16) uint16_t items[kTile];
-  __shared__ int32_t n_light, n_heavy, m_light, m_heavy, next_heavy, next_mark;
+  __shared__ int32_t n_light, n_heavy, m_light, m_heavy;
   __shared__ int32_t cnt[3];
   const int tid = threadIdx.x, lane = tid & 63;
   if (tid < 3) cnt[tid] = 0;
+  if (a.begun && blockIdx.x == 0 && tid == 0) tell_host(&a.watch[0], a.begun);
   // the first chunk's bounds and the previous step's live flag (one
   // uniform word: no block-wide reduction or barrier) load together
   int64_t c0 = a.chunk_ptr[blockIdx.x], c1 = a.chunk_ptr[blockIdx.x + 1];
@@ -346,6 +319,7 @@ __global__ void __launch_bounds__(kSirThreads) k_sir_step(SirStep a) {
     // previous step's counts forward).  The next bitmap B[(t+1)&1] is the
     // infected set after step t-2: empty when step t-2 left no infected agent,
     // so only the first identity step clears its spans.
+    if (a.watch && blockIdx.x == 0 && tid == 0) tell_host(&a.watch[1], 1);
     if (!(a.prev2_slots && a.prev2_slots[kLiveFlag] == 0)) {
       for (int32_t c = blockIdx.x; c < a.n_chunks; c += gridDim.x) {
         const int64_t w0 = (int64_t)a.chunk_ptr[c] >> 5;
@@ -368,7 +342,7 @@ __global__ void __launch_bounds__(kSirThreads) k_sir_step(SirStep a) {
     }
     for (int64_t sub = c0; sub < c1; sub += kTile) {
       if (tid == 0) {
-        n_light = n_heavy = m_light = m_heavy = next_heavy = next_mark = 0;
+        n_light = n_heavy = m_light = m_heavy = 0;
       }
       // phase 1: this thread's 8 consecutive agents v0 .. v0+7 (one 8-byte
       // state load, one 16-byte mark load; chunk starts are 64-aligned)
@@ -431,9 +405,9 @@ __global__ void __launch_bounds__(kSirThreads) k_sir_step(SirStep a) {
           }
           if (kLds && staged)
             scan_items<kMode>(a, reinterpret_cast<const uint32_t *>(lds_bm4), sub, nl, nh,
-                              items, outb, kinf, &next_heavy);
+                              items, outb, kinf);
           else
-            scan_items<kMode>(a, a.bm_in, sub, nl, nh, items, outb, kinf, &next_heavy);
+            scan_items<kMode>(a, a.bm_in, sub, nl, nh, items, outb, kinf);
           lds_barrier();
         }
       }
@@ -483,19 +457,14 @@ __global__ void __launch_bounds__(kSirThreads) k_sir_step(SirStep a) {
       {
         const int32_t nl = m_light, nh = m_heavy;
         if (nl + nh > 0) {
-          for (;;) {
-            int32_t k = 0;
-            if (lane == 0) k = atomicAdd(&next_mark, 1);
-            k = __shfl(k, 0);
-            if (k >= nh) break;
+          const int wave = tid >> 6;
+          for (int32_t k = wave; k < nh; k += kSirThreads / 64) {
             const int64_t u = sub + items[kTile - 1 - k];
             mark_heavy(a.col, a.mark, a.row_ptr[u], a.row_ptr[u + 1], new_mark);
           }
-          for (int32_t k0 = tid; k0 < nl; k0 += kSirThreads * kScanGroup) {
-            int loc[kScanGroup];
-            int32_t e[kScanGroup], hi[kScanGroup];
-            light_group_rows(a, sub, k0, nl, items, loc, e, hi);
-            mark_light_group(a.col, a.mark, e, hi, new_mark);
+          for (int32_t k = tid; k < nl; k += kSirThreads) {
+            const int2 at = item_bounds(a, sub, true, items[k]);
+            mark_light(a.col, a.mark, at.x, at.y, a.nnz, new_mark);
           }
           lds_barrier();
         }
@@ -692,8 +661,10 @@ int launch_step(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
                 const uint32_t *bm_in, uint32_t *bm_out, uint32_t t,
                 const uint32_t *keys4, uint32_t tb, uint32_t tg, int mode,
                 const int32_t *prev_slots, const int32_t *prev2_slots, int32_t *slots,
-                hipStream_t s) {
+                int32_t *watch, int32_t begun, hipStream_t s) {
   SirStep a;
+  a.watch = watch;
+  a.begun = begun;
   a.n = g->n;
   a.nnz = g->nnz;
   a.row_ptr = g->row_ptr;
@@ -726,6 +697,88 @@ int launch_step(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
     auto *kg = part ? k_sir_step<false, kModePartitionable> : k_sir_step<false, kModeOriginal>;
     hipLaunchKernelGGL(kg, dim3(blocks), dim3(kSirThreads), 0, s, a);
   }
+  return kOk;
+}
+
+// A watched run learns from the step kernels themselves how far it is (a store
+// to host memory at a step's start, no launch or copy of its own).  The store
+// costs its step about 1 us at the end, so only every kWatchEvery-th step
+// tells; the host launches kWatchEvery steps once the step as many before them
+// has begun, and up to twice as many identity steps, 2 us each, follow the last
+// infection.  1M agents x 365 steps: 3.34 ms a pass when every step tells,
+// 3.11 when each eighth does, 3.25 without a watch.
+constexpr int32_t kWatchEvery = 8;
+
+// Waits until step `begun` (counted from 1) has begun, or one was the identity.
+// An error of the stream ends the wait, and so does a stream that has finished
+// without saying so.
+int wait_begun(const int32_t *watch, int32_t begun, hipStream_t s, const char *who,
+               bool *settled) {
+  for (uint32_t spin = 0;; ++spin) {
+    *settled = __atomic_load_n(&watch[1], __ATOMIC_RELAXED) != 0;
+    if (*settled || __atomic_load_n(&watch[0], __ATOMIC_RELAXED) >= begun) return kOk;
+    if ((spin & 0x3FFF) != 0x3FFF) continue;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    if (e != hipSuccess) return hip_fail(e, who);
+    if (__atomic_load_n(&watch[0], __ATOMIC_ACQUIRE) >= begun) return kOk;
+    set_error(std::string(who) + ": watch must be host memory the device can write");
+    return kErrInvalid;
+  }
+}
+
+// The steps of a run; with watch, launching stops once a step was the identity:
+// so is every later one, and the count reduction fills in their zeroed slots as
+// if they had been launched.
+int sir_run(const char *who, const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
+            uint32_t *bitmaps, uint32_t t0, const uint32_t *keys, int32_t steps, float beta,
+            float gamma, int mode, int32_t *slots, int32_t *counts, int32_t *watch,
+            int32_t *launched, hipStream_t s) {
+  if (int rc = check_graph(g, who)) return rc;
+  if (!(state && mark && bitmaps && keys && slots && counts)) {
+    set_error(std::string(who) + ": null buffer");
+    return kErrInvalid;
+  }
+  if (!(steps >= 0 && (mode == 0 || mode == 1))) {
+    set_error(std::string(who) + ": bad steps or mode");
+    return kErrInvalid;
+  }
+  if (int rc = check_buffers(state, mark, bitmaps, bitmaps + bitmap_words(g->n), who)) return rc;
+  if (steps == 0) return kOk;
+  const uint32_t tb = unit_threshold(beta), tg = unit_threshold(gamma);
+  const int64_t words = bitmap_words(g->n);
+  const int64_t ns = (int64_t)steps * kStride;
+  if (watch) {
+    __atomic_store_n(&watch[0], 0, __ATOMIC_RELAXED);
+    __atomic_store_n(&watch[1], 0, __ATOMIC_RELEASE);
+  }
+  hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for(ns, 256)), dim3(256), 0, s,
+                     slots, ns, 0);
+  uint32_t *bm[2] = {bitmaps, bitmaps + words};
+  int32_t t = 0;
+  for (; t < steps; ++t) {
+    const bool tells = watch && t % kWatchEvery == 0;
+    if (tells && t >= 2 * kWatchEvery) {
+      bool settled = false;
+      if (int rc = wait_begun(watch, t + 1 - kWatchEvery, s, who, &settled)) return rc;
+      if (settled) break;
+    }
+    if (int rc = launch_step(g, state, mark, bm[t & 1], bm[(t + 1) & 1],
+                             t0 + (uint32_t)t, keys + 4 * (int64_t)t, tb, tg, mode,
+                             t ? slots + (int64_t)(t - 1) * kStride : nullptr,
+                             t > 1 ? slots + (int64_t)(t - 2) * kStride : nullptr,
+                             slots + (int64_t)t * kStride, watch, tells ? t + 1 : 0, s))
+      return rc;
+  }
+  hipLaunchKernelGGL(k_sir_reduce_slots, dim3(blocks_for(3 * (int64_t)steps, 256)),
+                     dim3(256), 0, s, slots, (int64_t)steps, counts);
+  hipLaunchKernelGGL(k_sir_carry_counts, dim3(blocks_for(3 * (int64_t)steps, 256)),
+                     dim3(256), 0, s, (const int32_t *)slots, (int64_t)steps, counts);
+  if (t & 1)
+    ABM_CHECK_HIP(hipMemcpyAsync(bm[0], bm[1], (size_t)words * 4,
+                                 hipMemcpyDeviceToDevice, s));
+  if (launched) *launched = t;
+  ABM_LAUNCH_CHECK(who);
   return kOk;
 }
 
@@ -794,38 +847,18 @@ int abm_sir_run(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
                 uint32_t *bitmaps, uint32_t t0, const uint32_t *keys,
                 int32_t steps, float beta, float gamma, int mode, int32_t *slots,
                 int32_t *counts, void *stream) {
-  if (int rc = check_graph(g, "abm_sir_run")) return rc;
-  ABM_REQUIRE(state && mark && bitmaps && keys && slots && counts,
-              "abm_sir_run: null buffer");
-  ABM_REQUIRE(steps >= 0 && (mode == 0 || mode == 1),
-              "abm_sir_run: bad steps or mode");
-  if (int rc = check_buffers(state, mark, bitmaps, bitmaps + bitmap_words(g->n),
-                             "abm_sir_run"))
-    return rc;
-  if (steps == 0) return kOk;
-  hipStream_t s = (hipStream_t)stream;
-  const uint32_t tb = unit_threshold(beta), tg = unit_threshold(gamma);
-  const int64_t words = bitmap_words(g->n);
-  const int64_t ns = (int64_t)steps * kStride;
-  hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for(ns, 256)), dim3(256), 0, s,
-                     slots, ns, 0);
-  uint32_t *bm[2] = {bitmaps, bitmaps + words};
-  for (int32_t t = 0; t < steps; ++t)
-    if (int rc = launch_step(g, state, mark, bm[t & 1], bm[(t + 1) & 1],
-                             t0 + (uint32_t)t, keys + 4 * (int64_t)t, tb, tg, mode,
-                             t ? slots + (int64_t)(t - 1) * kStride : nullptr,
-                             t > 1 ? slots + (int64_t)(t - 2) * kStride : nullptr,
-                             slots + (int64_t)t * kStride, s))
-      return rc;
-  hipLaunchKernelGGL(k_sir_reduce_slots, dim3(blocks_for(3 * (int64_t)steps, 256)),
-                     dim3(256), 0, s, slots, (int64_t)steps, counts);
-  hipLaunchKernelGGL(k_sir_carry_counts, dim3(blocks_for(3 * (int64_t)steps, 256)),
-                     dim3(256), 0, s, (const int32_t *)slots, (int64_t)steps, counts);
-  if (steps & 1)
-    ABM_CHECK_HIP(hipMemcpyAsync(bm[0], bm[1], (size_t)words * 4,
-                                 hipMemcpyDeviceToDevice, s));
-  ABM_LAUNCH_CHECK("abm_sir_run");
-  return kOk;
+  return sir_run("abm_sir_run", g, state, mark, bitmaps, t0, keys, steps, beta, gamma, mode, slots,
+                 counts, nullptr, nullptr, (hipStream_t)stream);
+}
+
+int abm_sir_run_watched(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
+                        uint32_t *bitmaps, uint32_t t0, const uint32_t *keys, int32_t steps,
+                        float beta, float gamma, int mode, int32_t *slots, int32_t *counts,
+                        int32_t *watch, int32_t *launched, void *stream) {
+  ABM_REQUIRE(watch && launched, "abm_sir_run_watched: null buffer");
+  *launched = 0;
+  return sir_run("abm_sir_run_watched", g, state, mark, bitmaps, t0, keys, steps, beta, gamma,
+                 mode, slots, counts, watch, launched, (hipStream_t)stream);
 }
 
 int abm_sir_step(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
@@ -838,7 +871,7 @@ int abm_sir_step(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
               "abm_sir_step: bad argument");
   if (int rc = check_buffers(state, mark, bm_in, bm_out, "abm_sir_step")) return rc;
   if (int rc = launch_step(g, state, mark, bm_in, bm_out, t, keys4, unit_threshold(beta),
-                           unit_threshold(gamma), mode, prev_slots, nullptr, slots,
+                           unit_threshold(gamma), mode, prev_slots, nullptr, slots, nullptr, 0,
                            (hipStream_t)stream))
     return rc;
   ABM_LAUNCH_CHECK("abm_sir_step");

@@ -83,6 +83,8 @@ class SIRNetworkEngine:
         self.n_seed_infected = int(min(n_seed_infected, self.n))
         self.seed = int(seed)
         self.rng = np.zeros(2, np.uint32)
+        self._watch = None         # pinned host words of a watched run
+        self.steps_launched = 0    # by the last run()
         self.reset(seed)
 
     # -- init: jaxabm/model.py:118-144 with C = 1 collection
@@ -124,10 +126,21 @@ class SIRNetworkEngine:
             self.t += int(steps)
 
     def run(self, steps: int) -> np.ndarray:
-        """Run ``steps`` steps; returns host counts [steps, 3] (S, I, R)."""
+        """Run ``steps`` steps; returns host counts [steps, 3] (S, I, R).
+        Steps are launched while the host waits for the run, and no more of
+        them once the last infection is over (abm_sir_run_watched)."""
         keys = self.key_table(steps)
         counts = torch.empty((max(steps, 1), 3), dtype=torch.int32, device=self.device)
-        self.launch(keys, steps, counts)
+        if self._watch is None:
+            self._watch = torch.empty(2, dtype=torch.int32, pin_memory=True)
+        launched = C.c_int32()
+        check(lib().abm_sir_run_watched(
+            C.byref(self._g), ptr(self.state), ptr(self.mark), ptr(self.bitmaps),
+            self.t & 0xFFFFFFFF, ptr(keys), int(steps), self.beta, self.gamma, self.mode,
+            ptr(self.slot_buffer(steps)), ptr(counts), C.c_void_p(self._watch.data_ptr()),
+            C.byref(launched), stream_handle()), "sir_run")
+        self.t += int(steps)
+        self.steps_launched = int(launched.value)
         return counts[:steps].cpu().numpy()
 
     def states(self) -> torch.Tensor:

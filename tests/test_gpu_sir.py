@@ -141,3 +141,49 @@ def test_seed_refuses_bad_chunk_tables(sir):
                                 ptr(eng.bitmaps), 0, stream_handle())
         with pytest.raises(AbmError, match="chunk_ptr"):
             check(rc, "abm_sir_seed")
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("steps", [1, 31, 32, 33, 47, 48, 49, 130])
+@pytest.mark.parametrize("n0,gamma", [(0, 0.5), (30, 0.5), (30, 0.02)])
+def test_settling_run_equals_oracle_and_continues(sir, mode, steps, n0, gamma):
+    """A run that stops launching once nobody is infected: the oracle's counts,
+    state and key, also when another run continues it; one that stays infected
+    launches every step."""
+    n, beta = 1500, 0.01
+    row_ptr, col = O.ba_csr(n, 3, graph_seed=4)
+    eng = sir.SIRNetworkEngine(n, csr=(row_ptr, col), beta=beta, gamma=gamma,
+                               n_seed_infected=n0, seed=8, mode=mode)
+    st, rng = O.sir_init(n, n0, 8, mode)
+    for part in (steps, 40):
+        want = O.sir_run(row_ptr, col, st, rng, beta, gamma, part, mode)
+        got = eng.run(part)
+        np.testing.assert_array_equal(got, want)
+        np.testing.assert_array_equal(eng.state_host(), st)
+        np.testing.assert_array_equal(eng.rng, rng)
+        dead = np.flatnonzero(want[:, 1] == 0)
+        if len(dead):   # launched up to two groups of 8 past the first that found none
+            assert min(part, dead[0] + 1) <= eng.steps_launched <= min(part, dead[0] + 2 + 16)
+        else:
+            assert eng.steps_launched == part
+
+
+def test_rows_at_the_end_of_the_entry_array(sir):
+    """Rows of every length up to the wide loads' eight entries as the last
+    rows of the array, where a wide load would pass its end."""
+    for tail in range(1, 10):
+        n = 200 + tail
+        rng = np.random.default_rng(tail)
+        # node n - 1 has `tail` neighbours; the others form a ring
+        src = np.r_[np.arange(n - 1), np.full(tail, n - 1)]
+        dst = np.r_[(np.arange(n - 1) + 1) % (n - 1), rng.choice(n - 1, tail, replace=False)]
+        from jaxabm_amd.network import csr_undirected
+
+        row_ptr, col = csr_undirected(n, src.astype(np.int32), dst.astype(np.int32))
+        assert row_ptr[n] - row_ptr[n - 1] == tail
+        eng = sir.SIRNetworkEngine(n, csr=(row_ptr, col), beta=0.6, gamma=0.1,
+                                   n_seed_infected=60, seed=tail)
+        st, key = O.sir_init(n, 60, tail, O.MODE_PARTITIONABLE)
+        want = O.sir_run(row_ptr, col, st, key, 0.6, 0.1, 20, O.MODE_PARTITIONABLE)
+        np.testing.assert_array_equal(eng.run(20), want)
+        np.testing.assert_array_equal(eng.state_host(), st)
