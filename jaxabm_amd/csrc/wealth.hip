@@ -743,13 +743,14 @@ __global__ void k_wealth_zero_acc(uint32_t *acc) {
   for (int i = threadIdx.x; i < ABM_WEALTH_GRID_ACC_WORDS; i += blockDim.x) acc[i] = 0;
 }
 
-__global__ void k_wealth_init(const uint32_t *__restrict__ init_key, int64_t n,
+__global__ void k_wealth_init(const uint32_t *__restrict__ init_key, Key key, int64_t n,
                               float *__restrict__ x, float *__restrict__ y,
                               int32_t *__restrict__ w, int mode) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  if (init_key) key = Key{init_key[0], init_key[1]};
   Key kx, ky;
-  split2(split_at(Key{init_key[0], init_key[1]}, n, i, mode), kx, ky, mode);
+  split2(split_at(key, n, i, mode), kx, ky, mode);
   x[i] = unit_float(bits_scalar(kx, mode));
   y[i] = unit_float(bits_scalar(ky, mode));
   w[i] = 1;
@@ -810,8 +811,20 @@ int abm_wealth_init(const uint32_t *init_key, int64_t n, float *x, float *y, int
                   (mode == 0 || mode == 1),
               "abm_wealth_init: bad arguments");
   hipLaunchKernelGGL(k_wealth_init, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                     (hipStream_t)stream, init_key, n, x, y, w, mode);
+                     (hipStream_t)stream, init_key, Key{0u, 0u}, n, x, y, w, mode);
   ABM_LAUNCH_CHECK("abm_wealth_init");
+  return kOk;
+}
+
+int abm_wealth_init_host_key(const uint32_t init_key[2], int64_t n, float *x, float *y, int32_t *w,
+                             int mode, void *stream) {
+  ABM_REQUIRE(init_key && x && y && w && n > 1 && n < (1ll << 31) &&
+                  (mode == 0 || mode == 1),
+              "abm_wealth_init_host_key: bad arguments");
+  hipLaunchKernelGGL(k_wealth_init, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream, (const uint32_t *)nullptr, Key{init_key[0], init_key[1]},
+                     n, x, y, w, mode);
+  ABM_LAUNCH_CHECK("abm_wealth_init_host_key");
   return kOk;
 }
 

@@ -29,6 +29,7 @@ import torch
 from .. import random as jr
 from .._lib import (DEFFUANT_COLUMNS, DEFFUANT_TAPE_LAST, DeffuantProblem, check, lib, ptr,
                     require_gpu, stream_handle)
+from ._staging import Staging
 
 STATS_LEN = 34
 HIST_BINS = 32
@@ -90,8 +91,11 @@ class DeffuantModel:
         self.stats = torch.empty((B, STATS_LEN), dtype=f64, device=dev)
         self.loss = torch.empty((B,), dtype=f64, device=dev)
         self.grads = torch.empty((2, B), dtype=f64, device=dev)
-        self.target = torch.zeros((STATS_LEN,), dtype=f64, device=dev)
-        self.weights = torch.ones((STATS_LEN,), dtype=f64, device=dev)
+        # target and weights, which a forward sets in one copy
+        self._aims = torch.ones((2, STATS_LEN), dtype=f64, device=dev)
+        self.target, self.weights = self._aims[0], self._aims[1]
+        self.target.zero_()
+        self._stage = Staging(dev)
         self.eps = torch.zeros((B,), dtype=torch.float32, device=dev)
         self.mu = torch.zeros((B,), dtype=torch.float32, device=dev)
         self.version = 0
@@ -126,9 +130,11 @@ class DeffuantModel:
             raise ValueError(f"eps and mu need {self.batch} values")
         self.eps.copy_(eps)
         self.mu.copy_(mu)
-        self.target.copy_(torch.as_tensor(np.asarray(target, np.float64).reshape(STATS_LEN)))
-        w = np.ones(STATS_LEN) if weights is None else np.asarray(weights, np.float64)
-        self.weights.copy_(torch.as_tensor(w.reshape(STATS_LEN)))
+        aims = np.ones((2, STATS_LEN))
+        aims[0] = np.asarray(target, np.float64).reshape(STATS_LEN)
+        if weights is not None:
+            aims[1] = np.asarray(weights, np.float64).reshape(STATS_LEN)
+        self._aims.copy_(self._stage.upload(aims).view(torch.float64).view(2, STATS_LEN))
         check(lib().abm_deffuant_forward(C.byref(self._problem(DEFFUANT_TAPE_LAST)),
                                          stream_handle()), "deffuant_forward")
         self.version += 1

@@ -21,6 +21,7 @@ import torch
 
 from .. import random as jr
 from .._lib import SchellingGrid, check, lib, ptr, require_gpu, stream_handle
+from ._staging import Staging
 
 
 class SchellingEngine:
@@ -49,21 +50,24 @@ class SchellingEngine:
                                 self.block_counts.data_ptr())
         self.n_agents = 0
         self._peek = None
+        self._stage = Staging(self.device)
         self.rng = np.zeros(2, np.uint32)
         self.reset(seed)
 
     def reset(self, seed: int) -> None:
-        key = torch.from_numpy(jr.host_prng_key(seed).view(np.int32).copy()).to(self.device)
+        key = self._stage.upload(jr.host_prng_key(seed))
         na = C.c_int32()
         check(lib().abm_schelling_init(C.byref(self._g), ptr(key), self.mode, C.byref(na),
                                        stream_handle()), "schelling_init")
         self.n_agents = int(na.value)
         self.rng = jr.host_split(jr.host_prng_key(seed), 2, self.mode)[0].copy()
 
-    def key_table(self, steps: int) -> torch.Tensor:
+    def _host_keys(self, steps: int) -> np.ndarray:
         tab = jr.step_key_table(self.rng, steps, 1, True, False, self.mode)
-        ck = np.ascontiguousarray(tab[:, 0:2])
-        return torch.from_numpy(ck.view(np.int32)).to(self.device)
+        return np.ascontiguousarray(tab[:, 0:2])
+
+    def key_table(self, steps: int) -> torch.Tensor:
+        return torch.from_numpy(self._host_keys(steps).view(np.int32)).to(self.device)
 
     def launch(self, keys, steps, counters, happy, moves, stream=None, prev=None):
         """abm_schelling_run; with ``prev`` (the counters of the step before,
@@ -83,12 +87,13 @@ class SchellingEngine:
         """Run ``steps`` steps; returns host (fraction happy, moves) arrays.
         ``chunk``: steps per launch, with the settled-grid exit of
         run_settling (0: all steps in one launch)."""
-        keys = self.key_table(steps)
+        keys = self._stage.upload(self._host_keys(steps)).view(torch.int32).view(-1, 2)
         counters = torch.empty((max(steps, 1), 2), dtype=torch.int32, device=self.device)
-        happy = torch.empty(max(steps, 1), dtype=torch.float32, device=self.device)
-        moves = torch.empty(max(steps, 1), dtype=torch.int32, device=self.device)
+        out = torch.empty((2, max(steps, 1)), dtype=torch.int32, device=self.device)
+        happy, moves = out[0].view(torch.float32), out[1]
         self.run_settling(keys, steps, counters, happy, moves, chunk)
-        return happy[:steps].cpu().numpy(), moves[:steps].cpu().numpy()
+        got = out.cpu().numpy()   # both records in one copy
+        return got[0, :steps].view(np.float32), got[1, :steps]
 
     def run_settling(self, keys, steps, counters, happy, moves, chunk=SETTLE_CHUNK, stream=None,
                      launch=None) -> int:

@@ -23,6 +23,7 @@ import torch
 from .. import random as jr
 from .._lib import SirGraph, check, lib, ptr, require_gpu, stream_handle
 from ..network import DeviceCSR, ba_csr_device, node_chunks
+from ._staging import Staging
 
 S, I, R = 0, 1, 2
 
@@ -83,6 +84,7 @@ class SIRNetworkEngine:
         self.n_seed_infected = int(min(n_seed_infected, self.n))
         self.seed = int(seed)
         self.rng = np.zeros(2, np.uint32)
+        self._stage = Staging(self.device)
         self._watch = None         # pinned host words of a watched run
         self.steps_launched = 0    # by the last run()
         self.reset(seed)
@@ -94,17 +96,20 @@ class SIRNetworkEngine:
         keys = jr.host_split(jr.host_prng_key(self.seed), 2, self.mode)
         self.rng = keys[0].copy()
         self.t = 0
-        init_key = torch.from_numpy(keys[1].view(np.int32).copy()).to(self.device)
+        init_key = self._stage.upload(keys[1]).view(torch.int32)
         perm = jr.permutation(init_key, self.n, mode=self.mode)
         check(lib().abm_sir_seed(C.byref(self._g), ptr(perm), self.n_seed_infected,
                                  ptr(self.state), ptr(self.mark), ptr(self.bitmaps), self.t,
                                  stream_handle()),
               "sir_seed")
 
+    def _host_keys(self, steps: int) -> np.ndarray:
+        tab = jr.step_key_table(self.rng, steps, 1, True, True, self.mode)
+        return np.ascontiguousarray(tab[:, 2:6])
+
     def key_table(self, steps: int) -> torch.Tensor:
         """Per-step (k_inf, k_rec) keys for the next ``steps`` steps; advances rng."""
-        tab = jr.step_key_table(self.rng, steps, 1, True, True, self.mode)
-        return torch.from_numpy(np.ascontiguousarray(tab[:, 2:6]).view(np.int32)).to(self.device)
+        return torch.from_numpy(self._host_keys(steps).view(np.int32)).to(self.device)
 
     def slot_buffer(self, steps: int) -> torch.Tensor:
         return torch.empty((max(steps, 1), self.slots_per_step, 3), dtype=torch.int32,
@@ -129,7 +134,7 @@ class SIRNetworkEngine:
         """Run ``steps`` steps; returns host counts [steps, 3] (S, I, R).
         Steps are launched while the host waits for the run, and no more of
         them once the last infection is over (abm_sir_run_watched)."""
-        keys = self.key_table(steps)
+        keys = self._stage.upload(self._host_keys(steps))
         counts = torch.empty((max(steps, 1), 3), dtype=torch.int32, device=self.device)
         if self._watch is None:
             self._watch = torch.empty(2, dtype=torch.int32, pin_memory=True)

@@ -21,6 +21,7 @@ import torch
 from .. import random as jr
 from .._lib import (WEALTH_GRID_ACC_WORDS, WEALTH_INST, check, lib, ptr, require_gpu,
                     stream_handle)
+from ._staging import Staging
 
 
 # up to here one workgroup can run a whole simulation out of LDS, whatever the
@@ -51,15 +52,16 @@ class WealthEngine:
         self.inc = torch.zeros(self.n, dtype=torch.int32, device=self.device)
         self.hist = torch.zeros(self.n + 1, dtype=torch.int32, device=self.device)
         self.rng = np.zeros(2, np.uint32)
+        self._stage = Staging(self.device)
         self.reset(seed)
 
     def reset(self, seed: int) -> None:
         """jaxabm/model.py:118-144 with one collection: rng, init_key = split(PRNGKey(seed))."""
         keys = jr.host_split(jr.host_prng_key(seed), 2, self.mode)
         self.rng = keys[0].copy()
-        ik = torch.from_numpy(keys[1].view(np.int32).copy()).to(self.device)
-        check(lib().abm_wealth_init(ptr(ik), self.n, ptr(self.x), ptr(self.y), ptr(self.w),
-                                    self.mode, stream_handle()), "wealth_init")
+        check(lib().abm_wealth_init_host_key(np.ascontiguousarray(keys[1]), self.n, ptr(self.x),
+                                             ptr(self.y), ptr(self.w), self.mode,
+                                             stream_handle()), "wealth_init")
 
     def key_table(self, steps: int) -> torch.Tensor:
         tab = jr.step_key_table(self.rng, steps, 1, True, False, self.mode)
@@ -87,25 +89,32 @@ class WealthEngine:
         runs above GRID_MIN_AGENTS whose draws would take more than
         DRAW_BUFFER_MAX_BYTES) spread every step over the whole GPU
         (abm_wealth_run_grid).  Same results either way."""
-        keys = self.key_table(steps)
-        mean = torch.empty(max(steps, 1), dtype=torch.float32, device=self.device)
-        gini = torch.empty(max(steps, 1), dtype=torch.float32, device=self.device)
+        tab = jr.step_key_table(self.rng, steps, 1, True, False, self.mode)
+        out = torch.empty((2, max(steps, 1)), dtype=torch.float32, device=self.device)
+        mean, gini = out[0], out[1]
+        # the key table and the descriptor in one copy
+        table, desc = tab.nbytes, WEALTH_INST.itemsize
+        dev, host = self._stage.open(table + desc)
+        host[:table] = tab.view(np.uint8).reshape(-1)
         if self.n > GRID_MIN_AGENTS and (self.n > EXCHANGE_MAX_AGENTS or
                                          12 * self.n * steps > DRAW_BUFFER_MAX_BYTES):
             # draws computed inline by the step kernels; scratch for the
             # second copies of what one launch per step reads and adds to
             scratch = self.draw_buffer(1)
-            host = self.descriptor(keys, steps, mean, gini, scratch)
+            inst = self.descriptor(dev, steps, mean, gini, scratch)
+            self._stage.send()
             acc = torch.empty(WEALTH_GRID_ACC_WORDS, dtype=torch.int32, device=self.device)
-            check(lib().abm_wealth_run_grid(host.ctypes.data, ptr(acc), self.mode,
+            check(lib().abm_wealth_run_grid(inst.ctypes.data, ptr(acc), self.mode,
                                             stream_handle()), "wealth_run_grid")
         else:
             draws = self.draw_buffer(steps)   # held until the run has read it
-            host = self.descriptor(keys, steps, mean, gini, draws)
-            desc = torch.from_numpy(host.view(np.uint8)).to(self.device)
-            check(lib().abm_wealth_run_batch(ptr(desc), 1, self.n, self.mode, stream_handle()),
-                  "wealth_run")
-        return mean[:steps].cpu().numpy(), gini[:steps].cpu().numpy()
+            inst = self.descriptor(dev, steps, mean, gini, draws)
+            host[table:] = inst.view(np.uint8)
+            self._stage.send()
+            check(lib().abm_wealth_run_batch(dev.data_ptr() + table, 1, self.n, self.mode,
+                                             stream_handle()), "wealth_run")
+        got = out.cpu().numpy()
+        return got[0, :steps], got[1, :steps]
 
 
 def run_batch(engines: list[WealthEngine], steps: list[int], stream=None):

@@ -287,3 +287,17 @@ def test_column_run_equals_step_kernels(dm, monkeypatch, n, B, steps, k):
         np.testing.assert_array_equal(np.isfinite(a), fin)
         scale = np.abs(b[fin]).max() if fin.any() else 0.0
         np.testing.assert_allclose(a[fin], b[fin], rtol=max(tol, 1e-12) * 100, atol=scale * tol * 100)
+
+
+def test_forward_is_refused_under_capture(dm):
+    """Its target and weights come from the host; the model works afterwards."""
+    import torch
+
+    m = dm.DeffuantModel(64, 2, 3, seed=1)
+    args = (np.float32([0.2, 0.3]), np.float32([0.3, 0.2]), np.zeros(34))
+    want = m.forward(*args).cpu().numpy()
+    g = torch.cuda.CUDAGraph()
+    with pytest.raises(RuntimeError):
+        with torch.cuda.graph(g):
+            m.forward(*args)
+    np.testing.assert_array_equal(m.forward(*args).cpu().numpy(), want)
