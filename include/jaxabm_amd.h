@@ -318,6 +318,9 @@ typedef struct abm_schelling_grid {
 /* Length in int32 of the block_counts scratch for a grid of n_cells cells:
  * 16 x ceil(n_cells / 1024). */
 int64_t abm_schelling_block_count(int64_t n_cells);
+/* 1 when a run on this grid (n_agents set) is one launch of one workgroup,
+ * which ends by itself once the grid settles: small grids that fit its LDS. */
+int abm_schelling_one_launch(const abm_schelling_grid *g);
 /* Cells from uniform(key, (H*W,)) and the row-major agent numbering; sets
  * g->n_agents (synchronises the stream once). */
 int abm_schelling_init(abm_schelling_grid *g, const uint32_t *key, int mode, int32_t *n_agents_out,

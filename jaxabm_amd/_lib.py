@@ -203,6 +203,7 @@ SIGNATURES = {
     "abm_grid_moore_sum_f32": (_int, [_i64, _i64, _i32, _p, _p, _p]),
     "abm_grid_moore_counts_i8": (_int, [_i64, _i64, _i32, _p, _p, _p, _p]),
     "abm_schelling_block_count": (_i64, [_i64]),
+    "abm_schelling_one_launch": (_int, [C.POINTER(SchellingGrid)]),
     "abm_schelling_init": (_int, [C.POINTER(SchellingGrid), _p, _int, C.POINTER(_i32), _p]),
     "abm_schelling_run": (_int, [C.POINTER(SchellingGrid), _p, _i32, _int, _p, _p, _p, _p]),
     "abm_schelling_run_from": (_int, [C.POINTER(SchellingGrid), _p, _i32, _int, _p, _p, _p, _p,

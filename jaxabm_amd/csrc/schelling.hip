@@ -33,7 +33,9 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <mutex>
 
+#define ABM_STRAIGHT_DRAWS
 #include "common.hpp"
 #include "jaxabm_amd.h"
 
@@ -387,6 +389,230 @@ __global__ void __launch_bounds__(kMovesThreads) k_schelling_moves(int64_t n_age
   }
 }
 
+// ---- small grids: a whole run in one launch by one workgroup
+//
+// The two types as bit planes of whole words per row, agent ids, the empty
+// list and its claims in LDS.  A step: the unhappy cells, 32 at a time by
+// bitwise counts, and the empty ones; one scan of both counts; both lists; the
+// draws of the unhappy agents, on full waves, and their claims; the winners'
+// moves.  Four barriers.  The run ends at the first identity step, whose
+// record every later step repeats.
+//
+// Bound by the draws (450 instructions an unhappy agent, on one CU) and by the
+// latency of the barriers.  Runs of 80 steps, which settle at 13 to 20: 24 x 24
+// cells 141 us, 61 x 90 176, 100 x 100 179, 150 x 150 210, with the two
+// launches a step of the kernels above 493, 523, 517 and 527; 12 steps of
+// 150 x 150, the least favourable, 184 against 293.  So every grid that the LDS
+// holds runs here (about 24,000 cells; the one CU's draws would meet the
+// launches at some 60,000).  Happiness by agent from byte cells: 61 x 90 236 us.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / 64;
+constexpr size_t kSmallLds = 155 * 1024;
+
+struct SchellingSmall {
+  int32_t H, W, row_words, n_agents, n_empty, steps;
+  int8_t *cells;
+  int32_t *id, *pos;
+  const uint32_t *keys;  // [steps][2]
+  const int32_t *prev;   // counters of the step before, or null
+  int32_t *counters;     // [steps][2]
+  float *happy_frac;
+  int32_t *moves;
+};
+
+// LDS: the planes and the unhappy bits u32[3][words], claim u32[n_empty],
+// id u16[cells], list u16[n_empty], work and draw u16[n_agents]
+size_t schelling_small_lds(int32_t H, int32_t W, int64_t n_agents) {
+  const int64_t nc = (int64_t)H * W, words = (int64_t)H * ((W + 31) / 32);
+  return (size_t)(12 * words + 6 * (nc - n_agents) + 2 * nc + 4 * n_agents);
+}
+
+bool schelling_small(int32_t H, int32_t W, int64_t n_agents) {
+  return schelling_small_lds(H, W, n_agents) <= kSmallLds;  // so H * W < 2^16
+}
+
+// at_least[i]: bits where at least 2^i of the eight words have theirs set;
+// exact[i]: where exactly i have, i < 3
+__device__ __forceinline__ void bit_counts(const uint32_t (&x)[8], uint32_t (&at_least)[3],
+                                           uint32_t (&exact)[3]) {
+  const uint32_t s1 = x[0] ^ x[1] ^ x[2], c1 = (x[0] & x[1]) | (x[2] & (x[0] ^ x[1]));
+  const uint32_t s2 = x[3] ^ x[4] ^ x[5], c2 = (x[3] & x[4]) | (x[5] & (x[3] ^ x[4]));
+  const uint32_t s3 = x[6] ^ x[7], c3 = x[6] & x[7];
+  const uint32_t b0 = s1 ^ s2 ^ s3, c4 = (s1 & s2) | (s3 & (s1 ^ s2));
+  const uint32_t t = c1 ^ c2 ^ c3, f1 = (c1 & c2) | (c3 & (c1 ^ c2));
+  const uint32_t b1 = t ^ c4, f2 = t & c4;
+  at_least[2] = f1 | f2;  // 4 or more
+  at_least[1] = at_least[2] | b1;
+  at_least[0] = at_least[1] | b0;
+  exact[0] = ~at_least[0];
+  exact[1] = b0 & ~at_least[1];
+  exact[2] = b1 & ~b0 & ~at_least[2];
+}
+
+// the eight neighbours' bits of word w of row r on the torus
+__device__ __forceinline__ void bit_neighbours(const uint32_t *plane, int32_t r, int32_t w,
+                                               int32_t H, int32_t W, int32_t row_words,
+                                               uint32_t (&x)[8]) {
+  const int32_t rows[3] = {r ? r - 1 : H - 1, r, r + 1 < H ? r + 1 : 0};
+  const int32_t last = row_words - 1, end = (W - 1) & 31;  // the last column's word and bit
+  uint32_t *out = x;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const uint32_t *row = plane + rows[q] * row_words;
+    const uint32_t mid = row[w];
+    const uint32_t from_left = w ? row[w - 1] >> 31 : (row[last] >> end) & 1u;
+    const uint32_t from_right = w < last ? row[w + 1] << 31 : (row[0] & 1u) << end;
+    *out++ = (mid << 1) | from_left;
+    *out++ = (mid >> 1) | from_right;
+    if (q != 1) *out++ = mid;
+  }
+}
+
+template <int kMode>
+__global__ void __launch_bounds__(kSmallThreads) k_schelling_small(SchellingSmall a) {
+  extern __shared__ uint32_t small_lds[];
+  __shared__ uint32_t wsum[kSmallWaves];
+  __shared__ int32_t moved_sum[2];  // by step parity
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int32_t W = a.W, nc = a.H * W, na = a.n_agents, ne = a.n_empty;
+  const int32_t rw = a.row_words, words = a.H * rw;
+  uint32_t *one = small_lds, *two = one + words, *sad = two + words, *claim = sad + words;
+  uint16_t *id = reinterpret_cast<uint16_t *>(claim + ne);
+  uint16_t *list = id + nc, *work = list + ne, *draw = work + na;
+  const uint32_t tail = (W & 31) ? (1u << (W & 31)) - 1 : ~0u;  // columns of a row's last word
+  // c / W for c < 2^16: (c + 0.5) / W is 0.5 / W or more from a whole number,
+  // its rounding errors are below 2^-6 / W
+  const float inv_w = 1.0f / (float)W;
+  auto row_of = [&](int32_t c) { return (int32_t)(((float)c + 0.5f) * inv_w); };
+  for (int32_t w = tid; w < words; w += kSmallThreads) one[w] = two[w] = 0;
+  for (int32_t j = tid; j < ne; j += kSmallThreads) claim[j] = INT_MAX;
+  if (tid < 2) moved_sum[tid] = 0;
+  __syncthreads();
+  for (int32_t c = tid; c < nc; c += kSmallThreads) {
+    const int8_t v = a.cells[c];
+    id[c] = (uint16_t)a.id[c];
+    const int32_t r = row_of(c), col = c - r * W;
+    if (v) atomicOr(&(v == 1 ? one : two)[r * rw + (col >> 5)], 1u << (col & 31));
+  }
+  // words of a thread: neighbouring ones, so that the scan numbers the cells row by row
+  const int32_t per = (words + kSmallThreads - 1) / kSmallThreads;
+  const int32_t w0 = min(tid * per, words), w1 = min(w0 + per, words);
+  int32_t prev_happy = a.prev ? a.prev[0] : -1;
+  Key key{a.keys[0], a.keys[1]};
+  int32_t t = 0;
+  __syncthreads();
+  for (; t < a.steps && prev_happy != na; ++t) {  // block-uniform
+    const int32_t tn = t + 1 < a.steps ? t + 1 : t;
+    const Key ck = key;
+    key = Key{a.keys[2 * tn], a.keys[2 * tn + 1]};  // the next step's, on its way meanwhile
+    // 8 same < 3 (same + other) is 5 same < 3 other: no like neighbour and 1
+    // or more others, 1 and 2 or more, 2 and 4 or more (3 would need 6)
+    uint32_t count = 0;  // empty cells << 16 | unhappy agents
+    for (int32_t w = w0; w < w1; ++w) {
+      const int32_t r = w / rw, col = w - r * rw;
+      uint32_t x1[8], x2[8], least1[3], least2[3], is1[3], is2[3];
+      bit_neighbours(one, r, col, a.H, W, rw, x1);
+      bit_neighbours(two, r, col, a.H, W, rw, x2);
+      bit_counts(x1, least1, is1);
+      bit_counts(x2, least2, is2);
+      const uint32_t o = one[w], p = two[w];
+      const uint32_t u =
+          (o & ((is1[0] & least2[0]) | (is1[1] & least2[1]) | (is1[2] & least2[2]))) |
+          (p & ((is2[0] & least1[0]) | (is2[1] & least1[1]) | (is2[2] & least1[2])));
+      sad[w] = u;
+      const uint32_t e = ~(o | p) & (col == rw - 1 ? tail : ~0u);
+      count += (uint32_t)__popc(e) << 16 | (uint32_t)__popc(u);
+    }
+    uint32_t at = count;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(at, off);
+      if (lane >= off) at += y;
+    }
+    if (lane == 63) wsum[wave] = at;
+    __syncthreads();
+    at -= count;
+    uint32_t total = 0;
+#pragma unroll
+    for (int q = 0; q < kSmallWaves; ++q) {
+      if (q == wave) at += total;
+      total += wsum[q];
+    }
+    const int32_t unhappy = (int32_t)(total & 0xffffu);
+    const int32_t nwork = ne > 0 ? min(unhappy, na) : 0;
+    for (int32_t w = w0; w < w1; ++w) {
+      const int32_t r = w / rw, col = w - r * rw, c0 = r * W + 32 * col;
+      for (uint32_t u = sad[w]; u; u &= u - 1) {
+        const uint32_t i = at++ & 0xffffu;
+        if (i < (uint32_t)na) work[i] = (uint16_t)(c0 + __ffs(u) - 1);
+      }
+      for (uint32_t e = ~(one[w] | two[w]) & (col == rw - 1 ? tail : ~0u); e; e &= e - 1) {
+        const uint32_t j = at >> 16;
+        if (j < (uint32_t)ne) list[j] = (uint16_t)(c0 + __ffs(e) - 1);
+        at += 1u << 16;
+      }
+    }
+    __syncthreads();
+    // draws and claims (lowest agent wins)
+    for (int32_t i = tid; i < nwork; i += kSmallThreads) {
+      const uint32_t k = id[work[i]];
+      Key k1, k2;
+      split2(split_at(ck, na, k, kMode), k1, k2, kMode);
+      const uint32_t j = randint_offset(bits_scalar(k1, kMode), bits_scalar(k2, kMode),
+                                        (uint32_t)ne);
+      draw[i] = (uint16_t)j;
+      atomicMin(&claim[j], k);
+    }
+    if (tid == 0) moved_sum[(t + 1) & 1] = 0;  // last read before this step's first barrier
+    __syncthreads();
+    // moves: old cells and targets are distinct; a winner frees its claim (a
+    // loser that reads it then still loses)
+    int32_t moved = 0;
+    for (int32_t i = tid; i < nwork; i += kSmallThreads) {
+      const int32_t old = work[i], j = draw[i];
+      const uint32_t k = id[old];
+      if (claim[j] == k) {
+        const int32_t to = list[j], r0 = row_of(old), r1 = row_of(to);
+        const int32_t col0 = old - r0 * W, col1 = to - r1 * W;
+        const int32_t from = r0 * rw + (col0 >> 5), into = r1 * rw + (col1 >> 5);
+        const uint32_t bit = 1u << (col0 & 31);
+        uint32_t *plane = (one[from] & bit) ? one : two;
+        atomicAnd(&plane[from], ~bit);
+        atomicOr(&plane[into], 1u << (col1 & 31));
+        id[to] = (uint16_t)k;
+        claim[j] = INT_MAX;
+        ++moved;
+      }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) moved += __shfl_xor(moved, off);
+    if (lane == 0 && moved) atomicAdd(&moved_sum[t & 1], moved);
+    __syncthreads();
+    prev_happy = na - unhappy;
+    if (tid == 0) {
+      const int32_t m = moved_sum[t & 1];
+      a.counters[2 * t] = prev_happy;
+      a.counters[2 * t + 1] = m;
+      a.happy_frac[t] = (float)prev_happy / (float)(na > 0 ? na : 1);
+      a.moves[t] = m;
+    }
+  }
+  for (int32_t u = t + tid; u < a.steps; u += kSmallThreads) {  // identity steps
+    a.counters[2 * u] = na;
+    a.counters[2 * u + 1] = 0;
+    a.happy_frac[u] = (float)na / (float)(na > 0 ? na : 1);
+    a.moves[u] = 0;
+  }
+  if (t == 0) return;
+  for (int32_t c = tid; c < nc; c += kSmallThreads) {
+    const int32_t r = row_of(c), col = c - r * W, w = r * rw + (col >> 5), b = col & 31;
+    const int8_t v = (int8_t)((one[w] >> b & 1u) + 2 * (two[w] >> b & 1u));
+    a.cells[c] = v;
+    a.id[c] = v ? id[c] : -1;
+    if (v) a.pos[id[c]] = c;
+  }
+}
+
 // record[t] = (happy fraction, moves) from the integer counters
 __global__ void k_schelling_record(const int32_t *__restrict__ counters, int32_t steps,
                                    int64_t n_agents, float *__restrict__ happy_frac,
@@ -428,6 +654,27 @@ __global__ void k_fill_i32_s(int32_t *__restrict__ p, int64_t n, int32_t v) {
   if (i < n) p[i] = v;
 }
 
+// k_schelling_small may need more than 64 KB of dynamic LDS: the limit is
+// raised once per device, under a lock.
+constexpr int kMaxDevices = 64;
+std::mutex g_small_attr_mu;
+bool g_small_attr_set[kMaxDevices];
+
+int small_lds_attr() {
+  int dev = -1;
+  ABM_CHECK_HIP(hipGetDevice(&dev));
+  ABM_REQUIRE(dev >= 0 && dev < kMaxDevices, "schelling: device index out of range");
+  std::lock_guard<std::mutex> lock(g_small_attr_mu);
+  if (!g_small_attr_set[dev]) {
+    for (const void *k : {(const void *)k_schelling_small<kModeOriginal>,
+                          (const void *)k_schelling_small<kModePartitionable>})
+      ABM_CHECK_HIP(
+          hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
+    g_small_attr_set[dev] = true;
+  }
+  return kOk;
+}
+
 inline unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 int check_grid(const abm_schelling_grid *g, const char *who) {
@@ -449,6 +696,11 @@ extern "C" {
 
 int64_t abm_schelling_block_count(int64_t n_cells) {
   return kCountCopies * ((n_cells + kCellsPerBlock - 1) / kCellsPerBlock);
+}
+
+int abm_schelling_one_launch(const abm_schelling_grid *g) {
+  if (check_grid(g, "abm_schelling_one_launch")) return 0;
+  return schelling_small(g->height, g->width, g->n_agents) ? 1 : 0;
 }
 
 int abm_schelling_init(abm_schelling_grid *g, const uint32_t *key, int mode,
@@ -511,6 +763,30 @@ static int schelling_steps(const abm_schelling_grid *g, const uint32_t *keys, in
   uint32_t *ebits = reinterpret_cast<uint32_t *>(g->empty);  // nwords <= H*W words
   ABM_REQUIRE(((uintptr_t)ebits & 15u) == 0,
               "abm_schelling_run: the empty scratch must be 16-byte aligned");
+  if (schelling_small(g->height, g->width, g->n_agents)) {
+    if (int rc = small_lds_attr()) return rc;
+    SchellingSmall a;
+    a.H = g->height;
+    a.W = g->width;
+    a.row_words = (a.W + 31) / 32;
+    a.n_agents = (int32_t)g->n_agents;
+    a.n_empty = (int32_t)n_empty;
+    a.steps = steps;
+    a.cells = g->cells;
+    a.id = g->id;
+    a.pos = g->pos;
+    a.keys = keys;
+    a.prev = prev0;
+    a.counters = counters;
+    a.happy_frac = happy_frac;
+    a.moves = moves;
+    hipLaunchKernelGGL(mode == kModePartitionable ? k_schelling_small<kModePartitionable>
+                                                  : k_schelling_small<kModeOriginal>,
+                       dim3(1), dim3(kSmallThreads),
+                       schelling_small_lds(g->height, g->width, g->n_agents), s, a);
+    ABM_LAUNCH_CHECK(what);
+    return kOk;
+  }
   hipLaunchKernelGGL(k_fill_i32_s, dim3(nblk(2 * (int64_t)steps, 256)), dim3(256), 0, s,
                      counters, 2 * (int64_t)steps, 0);
   if (!prev0) {

@@ -86,11 +86,14 @@ class SchellingEngine:
     def run(self, steps: int, chunk: int = SETTLE_CHUNK):
         """Run ``steps`` steps; returns host (fraction happy, moves) arrays.
         ``chunk``: steps per launch, with the settled-grid exit of
-        run_settling (0: all steps in one launch)."""
+        run_settling (0: all steps in one launch; so is a run on a small grid,
+        whose one kernel has that exit itself)."""
         keys = self._stage.upload(self._host_keys(steps)).view(torch.int32).view(-1, 2)
         counters = torch.empty((max(steps, 1), 2), dtype=torch.int32, device=self.device)
         out = torch.empty((2, max(steps, 1)), dtype=torch.int32, device=self.device)
         happy, moves = out[0].view(torch.float32), out[1]
+        if lib().abm_schelling_one_launch(C.byref(self._g)):
+            chunk = 0
         self.run_settling(keys, steps, counters, happy, moves, chunk)
         got = out.cpu().numpy()   # both records in one copy
         return got[0, :steps].view(np.float32), got[1, :steps]

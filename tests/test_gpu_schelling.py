@@ -140,3 +140,36 @@ def test_schelling_near_the_grid_size_limit(schelling):
     np.testing.assert_array_equal(hf, ohf)
     np.testing.assert_array_equal(eng.grid().reshape(-1), cells)
     np.testing.assert_array_equal(eng.positions(), pos)
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("H,W,one", [(1, 1, 1), (1, 70, 1), (65, 1, 1), (2, 2, 1), (3, 341, 1),
+                                     (8500, 1, 1), (154, 155, 1), (157, 157, 0)])
+def test_schelling_one_launch_runs(schelling, mode, H, W, one):
+    """Grids that run in one launch, up to the largest that fits the LDS and
+    the first that does not: records, cells, positions and cell ids equal the
+    oracle's over a run of 7 steps continued for 40 more (past settling)."""
+    import ctypes as C
+
+    import torch
+
+    from jaxabm_amd._lib import lib
+
+    eng = schelling.SchellingEngine(H, W, seed=4, mode=mode)
+    assert lib().abm_schelling_one_launch(C.byref(eng._g)) == one
+    cells, pos, typ, rng = O.schelling_init(H, W, 4, mode)
+    ohf, omv = O.schelling_run(H, W, cells, pos, typ, rng, 47, mode)
+    S = 47
+    keys = eng.key_table(S)
+    counters = torch.empty((S, 2), dtype=torch.int32, device="cuda")
+    happy = torch.empty(S, dtype=torch.float32, device="cuda")
+    moves = torch.empty(S, dtype=torch.int32, device="cuda")
+    eng.launch(keys, 7, counters, happy, moves)
+    eng.launch(keys[7:], 40, counters[7:], happy[7:], moves[7:], prev=counters[6])
+    np.testing.assert_array_equal(moves.cpu().numpy(), omv)
+    np.testing.assert_array_equal(happy.cpu().numpy(), ohf)
+    np.testing.assert_array_equal(eng.grid().reshape(-1), cells)
+    np.testing.assert_array_equal(eng.positions(), pos)
+    want = np.full(H * W, -1, np.int32)
+    want[pos] = np.arange(len(pos))
+    np.testing.assert_array_equal(eng.id.cpu().numpy().reshape(-1), want)
