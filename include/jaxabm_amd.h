@@ -340,6 +340,16 @@ int abm_schelling_run(const abm_schelling_grid *g, const uint32_t *keys, int32_t
 int abm_schelling_run_from(const abm_schelling_grid *g, const uint32_t *keys, int32_t steps,
                            int mode, const int32_t *prev_counters, int32_t *counters,
                            float *happy_frac, int32_t *moves, void *stream);
+/* abm_schelling_run (prev_counters NULL) or abm_schelling_run_from for a caller
+ * that waits for the records anyway: the same results, but the host keeps only
+ * a few steps launched ahead and launches no more once one found every agent
+ * happy before it.  watch: two words of pinned host memory, not in use by
+ * another run; *launched receives the number of steps launched.  Not for stream
+ * capture: the call returns when the last of them is launched. */
+int abm_schelling_run_watched(const abm_schelling_grid *g, const uint32_t *keys, int32_t steps,
+                              int mode, const int32_t *prev_counters, int32_t *counters,
+                              float *happy_frac, int32_t *moves, int32_t *watch,
+                              int32_t *launched, void *stream);
 /* Records `steps` settled steps without launching them.  A step whose
  * previous step found every agent happy is the identity (nothing moves, so
  * every agent is happy again), and so is every step after it.  prev_counters:

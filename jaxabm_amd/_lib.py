@@ -206,6 +206,8 @@ SIGNATURES = {
     "abm_schelling_one_launch": (_int, [C.POINTER(SchellingGrid)]),
     "abm_schelling_init": (_int, [C.POINTER(SchellingGrid), _p, _int, C.POINTER(_i32), _p]),
     "abm_schelling_run": (_int, [C.POINTER(SchellingGrid), _p, _i32, _int, _p, _p, _p, _p]),
+    "abm_schelling_run_watched": (_int, [C.POINTER(SchellingGrid), _p, _i32, _int, _p, _p, _p,
+                                         _p, _p, C.POINTER(_i32), _p]),
     "abm_schelling_run_from": (_int, [C.POINTER(SchellingGrid), _p, _i32, _int, _p, _p, _p, _p,
                                        _p]),
     "abm_schelling_settled": (_int, [C.POINTER(SchellingGrid), _p, _i32, _p, _p, _p, _p]),

@@ -20,15 +20,15 @@
 // never materialised: every agents block scans the block counts (1 KB at
 // 512 x 512) into an LDS prefix, and empty[j] is then a search of that prefix
 // and a popcount scan of one block's 32 bitmap words.  Two kernels per step
-// (captured with the rest of the run):
+// (captured with the rest of the run; small grids run in one launch, below):
 //   k_schelling_agents  32x32 cell tiles + 1-cell torus halo in LDS;
 //                       happiness, draw, empty[j], atomicMin claim
 //   k_schelling_moves   winners move; bitmap, block counts and claims updated
 // Layout (HBM): cells int8[H*W], id int32[H*W] (agent on a cell or -1),
 // claim int32[H*W] (INT32_MAX when unclaimed), pos int32[n_agents],
 // type int8[n_agents], target int32[n_agents], empty-cell bitmap
-// uint32[ceil(H*W/32)] (in the grid's `empty` scratch), empty cells per
-// 1024-cell block int32[8][ceil(H*W/1024)] (8 copies summed by readers; in
+// uint32[32 * ceil(H*W/1024)] (in the grid's `empty` scratch), empty cells per
+// 1024-cell block int32[16][ceil(H*W/1024)] (16 copies summed by readers; in
 // the `block_counts` scratch).
 #include <hip/hip_runtime.h>
 
@@ -38,6 +38,7 @@
 #define ABM_STRAIGHT_DRAWS
 #include "common.hpp"
 #include "jaxabm_amd.h"
+#include "watch.hpp"
 
 namespace abm {
 
@@ -111,17 +112,17 @@ __global__ void __launch_bounds__(kCellsPerBlock)
   }
 }
 
-// Empty-cell bitmap of the current grid: one ballot per 64 cells.
+// Empty-cell bitmap of the current grid: one ballot per 64 cells; cells past
+// the last one are not empty.
 __global__ void __launch_bounds__(kCellsPerBlock)
-    k_empty_bits(const int8_t *__restrict__ cells, int64_t nc, int64_t nwords,
-                 uint32_t *__restrict__ ebits) {
+    k_empty_bits(const int8_t *__restrict__ cells, int64_t nc, uint32_t *__restrict__ ebits) {
   const int64_t c = (int64_t)blockIdx.x * kCellsPerBlock + threadIdx.x;
   const bool e = c < nc && cells[c] == 0;
   const uint64_t m = __ballot(e);
   if ((threadIdx.x & 63) == 0) {
     const int64_t w = c >> 5;  // c is the wave's first cell (a multiple of 64)
-    if (w < nwords) ebits[w] = (uint32_t)m;
-    if (w + 1 < nwords) ebits[w + 1] = (uint32_t)(m >> 32);
+    ebits[w] = (uint32_t)m;
+    ebits[w + 1] = (uint32_t)(m >> 32);
   }
 }
 
@@ -189,10 +190,10 @@ __device__ void empty_prefix(const int32_t *__restrict__ ecount, int nb, int32_t
 }
 
 // Cell of the j-th empty cell in row-major order (j < P[nb]): the block b with
-// P[b] <= j < P[b + 1], then the (j - P[b])-th set bit of its 32 bitmap words.
+// P[b] <= j < P[b + 1], then the (j - P[b])-th set bit of its 32 bitmap words,
+// one cache line, read 16 bytes at a time.
 __device__ __forceinline__ int32_t jth_empty(uint32_t j, const int32_t *P, int nb,
-                                             const uint32_t *__restrict__ ebits,
-                                             int64_t nwords) {
+                                             const uint32_t *__restrict__ ebits) {
   int lo = 0, hi = nb;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
@@ -205,22 +206,36 @@ __device__ __forceinline__ int32_t jth_empty(uint32_t j, const int32_t *P, int n
   const int64_t w0 = (int64_t)lo * kWordsPerBlock;
   uint32_t wv[kWordsPerBlock];
 #pragma unroll
-  for (int q = 0; q < kWordsPerBlock; ++q) wv[q] = w0 + q < nwords ? ebits[w0 + q] : 0u;
-  int32_t cell = -1;
+  for (int q = 0; q < kWordsPerBlock / 4; ++q) {
+    const uint4 v = reinterpret_cast<const uint4 *>(ebits + w0)[q];
+    wv[4 * q] = v.x;
+    wv[4 * q + 1] = v.y;
+    wv[4 * q + 2] = v.z;
+    wv[4 * q + 3] = v.w;
+  }
+  // the word: the last one with at most r bits before it
+  uint32_t n = 0, before = 0, word = 0, w = 0;
 #pragma unroll
   for (int q = 0; q < kWordsPerBlock; ++q) {
-    const uint32_t pc = (uint32_t)__popc(wv[q]);
-    if (cell < 0) {
-      if (r < pc) {
-        uint32_t v = wv[q];
-        for (uint32_t k = 0; k < r; ++k) v &= v - 1;
-        cell = (int32_t)((w0 + q) * 32 + __builtin_ctz(v));
-      } else {
-        r -= pc;
-      }
+    const bool here = n <= r;
+    before = here ? n : before;
+    word = here ? wv[q] : word;
+    w = here ? q : w;
+    n += (uint32_t)__popc(wv[q]);
+  }
+  if (r >= n) return -1;
+  // the bit, by halves
+  r -= before;
+  uint32_t bit = 0;
+#pragma unroll
+  for (int half = 16; half > 0; half >>= 1) {
+    const uint32_t low = (uint32_t)__popc((word >> bit) & ((1u << half) - 1));
+    if (r >= low) {
+      r -= low;
+      bit += half;
     }
   }
-  return cell;
+  return (int32_t)((w0 + w) * 32 + bit);
 }
 
 struct SchellingStep {
@@ -230,16 +245,16 @@ struct SchellingStep {
   const int32_t *id;
   const uint32_t *ebits;
   const int32_t *ecount;
-  int64_t nwords;
   int32_t nb;
   int32_t *claim, *target;
   const uint32_t *ck;
-  int mode;
   int32_t *happy_count;
   // the previous step's happy count (null at a run's first step): when every
   // agent was happy then, nobody moved, the grid is unchanged and this step
   // is the identity
   const int32_t *prev_happy;
+  int32_t *watch;  // host words of a watched run, or null
+  int32_t begun;   // value for watch[0], or 0: this step does not tell
 };
 
 // True when the step is the identity: the previous step found every agent
@@ -248,7 +263,15 @@ __device__ __forceinline__ bool schelling_identity(const int32_t *prev_happy, in
   return prev_happy && (int64_t)*prev_happy == n_agents;
 }
 
-__global__ void __launch_bounds__(kTileDim * kTileDim) k_schelling_agents(SchellingStep a) {
+// Bound by its chain, not by bytes or instructions: one round of loads, the
+// prefix's barriers, the draw, the bitmap line, the claim's atomic, each from
+// memory that another XCD wrote a launch before.  14.5 -> 10.8 us in the first
+// steps at 512 x 512 with the identity word loaded beside the tile, no modulo,
+// and the line read 16 bytes at a time.  (Bit planes of the whole grid read and
+// scanned by every workgroup in place of counts, tiles and the search in memory
+// took 12.4, and 779 us against 600 for 40 steps of 614 x 640.)
+template <int kMode>
+__global__ void __launch_bounds__(kTileDim * kTileDim, 8) k_schelling_agents(SchellingStep a) {
   extern __shared__ int32_t empty_prefix_lds[];  // [nb + 1]
   __shared__ int8_t tile[kTileDim + 2][kTileDim + 2];
   __shared__ int32_t wc[16];
@@ -257,33 +280,42 @@ __global__ void __launch_bounds__(kTileDim * kTileDim) k_schelling_agents(Schell
   __shared__ int32_t nwork;
   constexpr int kHalo = (kTileDim + 2) * (kTileDim + 2);  // 34 x 34 cells, <= 2 per thread
   const int tid = threadIdx.x;
-  if (schelling_identity(a.prev_happy, a.n_agents)) {  // grid-uniform
-    // every agent happy again; no target is drawn (the last step left each
-    // agent's target at -1) and the moves kernel exits too
-    if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *a.happy_count = (int32_t)a.n_agents;
-    return;
-  }
+  const bool first_thread = blockIdx.x == 0 && blockIdx.y == 0 && tid == 0;
+  if (a.begun && first_thread) tell_host(&a.watch[0], a.begun);
   const int tx = tid % kTileDim, ty = tid / kTileDim;
   const int r0 = blockIdx.y * kTileDim, c0 = blockIdx.x * kTileDim;
   const int r = r0 + ty, c = c0 + tx;
   const bool inside = r < a.H && c < a.W;
   const int64_t cell = (int64_t)r * a.W + c;
   // one memory round trip: the tile and its torus halo, this thread's block
-  // count for the prefix, the agent on this thread's cell
+  // count for the prefix, the agent on this thread's cell, the step before's
+  // count
   int8_t tv[2] = {0, 0};
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int q = tid + i * (int)blockDim.x;
     if (q < kHalo) {
       const int lr = q / (kTileDim + 2), lc = q % (kTileDim + 2);
+      // r0 < H and c0 < W; the tile may pass the edge by up to 32 cells
       int gr = r0 + lr - 1, gc = c0 + lc - 1;
-      gr = (gr % a.H + a.H) % a.H;
-      gc = (gc % a.W + a.W) % a.W;
+      if (gr < 0) gr += a.H;
+      while (gr >= a.H) gr -= a.H;
+      if (gc < 0) gc += a.W;
+      while (gc >= a.W) gc -= a.W;
       tv[i] = a.cells[(int64_t)gr * a.W + gc];
     }
   }
   const int32_t first = tid < a.nb ? block_empty(a.ecount, a.nb, tid) : 0;
   const int32_t k = inside ? a.id[cell] : -1;
+  if (schelling_identity(a.prev_happy, a.n_agents)) {  // grid-uniform
+    // every agent happy again; no target is drawn (the last step left each
+    // agent's target at -1) and the moves kernel exits too
+    if (first_thread) {
+      *a.happy_count = (int32_t)a.n_agents;
+      if (a.watch) tell_host(&a.watch[1], 1);
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int q = tid + i * (int)blockDim.x;
@@ -324,10 +356,10 @@ __global__ void __launch_bounds__(kTileDim * kTileDim) k_schelling_agents(Schell
   if (tid < nwork) {
     const int32_t kd = work[tid];
     Key k1, k2;
-    split2(split_at(Key{a.ck[0], a.ck[1]}, a.n_agents, kd, a.mode), k1, k2, a.mode);
-    const uint32_t j = randint_offset(bits_scalar(k1, a.mode), bits_scalar(k2, a.mode),
+    split2(split_at(Key{a.ck[0], a.ck[1]}, a.n_agents, kd, kMode), k1, k2, kMode);
+    const uint32_t j = randint_offset(bits_scalar(k1, kMode), bits_scalar(k2, kMode),
                                       (uint32_t)a.n_empty);
-    const int32_t tg = jth_empty(j, empty_prefix_lds, a.nb, a.ebits, a.nwords);
+    const int32_t tg = jth_empty(j, empty_prefix_lds, a.nb, a.ebits);
     if (tg >= 0) atomicMin(&a.claim[tg], kd);
     a.target[kd] = tg;
   }
@@ -341,37 +373,48 @@ __global__ void __launch_bounds__(kTileDim * kTileDim) k_schelling_agents(Schell
   }
 }
 
-// one thread per agent; large workgroups keep the grid small, which is most
-// of the cost of a step that only checks the identity condition
+// One thread per agent; large workgroups keep the grid small, which is most of
+// the cost of a step that only checks the identity condition.  Bound by its
+// chain of loads (the identity word and the target, then the claim, the old
+// cell and the type, together) and by the drain of its scattered atomics: 7.5 ->
+// 5 us in the middle steps at 512 x 512 from two round trips more.
 constexpr int kMovesThreads = 1024;
 
-__global__ void __launch_bounds__(kMovesThreads) k_schelling_moves(int64_t n_agents, int8_t *__restrict__ cells,
-                                  int32_t *__restrict__ id, int32_t *__restrict__ claim,
-                                  int32_t *__restrict__ pos, const int8_t *__restrict__ type,
-                                  const int32_t *__restrict__ target, uint32_t *__restrict__ ebits,
-                                  int32_t *__restrict__ ecount, int32_t nb,
-                                  int32_t *__restrict__ moves,
-                                  const int32_t *__restrict__ prev_happy) {
-  if (schelling_identity(prev_happy, n_agents)) return;  // grid-uniform: no move
+struct SchellingMoves {
+  int64_t n_agents;
+  int8_t *cells;
+  int32_t *id, *claim, *pos;
+  const int8_t *type;
+  const int32_t *target;
+  uint32_t *ebits;
+  int32_t *ecount;
+  int32_t nb;
+  int32_t *moves;
+  const int32_t *prev_happy;
+};
+
+__global__ void __launch_bounds__(kMovesThreads) k_schelling_moves(SchellingMoves a) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int32_t tg = k < a.n_agents ? a.target[k] : -1;
+  if (schelling_identity(a.prev_happy, a.n_agents)) return;  // grid-uniform: no move
   bool moved = false;
-  if (k < n_agents) {
-    const int32_t tg = target[k];
-    if (tg >= 0 && claim[tg] == (int32_t)k) {
-      const int32_t old = pos[k];
-      cells[old] = 0;
-      id[old] = -1;
-      cells[tg] = type[k];
-      id[tg] = (int32_t)k;
-      pos[k] = tg;
-      claim[tg] = INT_MAX;
+  if (tg >= 0) {
+    const int32_t winner = a.claim[tg], old = a.pos[k];
+    const int8_t type = a.type[k];
+    if (winner == (int32_t)k) {
+      a.cells[old] = 0;
+      a.id[old] = -1;
+      a.cells[tg] = type;
+      a.id[tg] = (int32_t)k;
+      a.pos[k] = tg;
+      a.claim[tg] = INT_MAX;
       // the old cell becomes empty, the target occupied (distinct cells: a
       // target was empty before the step, an old cell occupied)
-      atomicOr(&ebits[old >> 5], 1u << (old & 31));
-      atomicAnd(&ebits[tg >> 5], ~(1u << (tg & 31)));
+      atomicOr(&a.ebits[old >> 5], 1u << (old & 31));
+      atomicAnd(&a.ebits[tg >> 5], ~(1u << (tg & 31)));
       const int32_t bo = old / kCellsPerBlock, bt = tg / kCellsPerBlock;
       if (bo != bt) {
-        int32_t *copy = ecount + (int64_t)(blockIdx.x % kCountCopies) * nb;
+        int32_t *copy = a.ecount + (int64_t)(blockIdx.x % kCountCopies) * a.nb;
         atomicAdd(&copy[bo], 1);
         atomicSub(&copy[bt], 1);
       }
@@ -385,7 +428,7 @@ __global__ void __launch_bounds__(kMovesThreads) k_schelling_moves(int64_t n_age
   if (threadIdx.x == 0) {
     int32_t s = 0;
     for (int w = 0; w < kMovesThreads / 64; ++w) s += wc[w];
-    if (s) atomicAdd(moves, s);
+    if (s) atomicAdd(a.moves, s);
   }
 }
 
@@ -449,7 +492,20 @@ __device__ __forceinline__ void bit_counts(const uint32_t (&x)[8], uint32_t (&at
   exact[2] = b1 & ~b0 & ~at_least[2];
 }
 
-// the eight neighbours' bits of word w of row r on the torus
+// the unhappy bits of a word.  8 same < 3 (same + other) is 5 same < 3 other:
+// no like neighbour and 1 or more others, 1 and 2 or more, 2 and 4 or more (3
+// would need 6)
+__device__ __forceinline__ uint32_t bit_unhappy(uint32_t one, uint32_t two,
+                                                const uint32_t (&x1)[8],
+                                                const uint32_t (&x2)[8]) {
+  uint32_t least1[3], least2[3], is1[3], is2[3];
+  bit_counts(x1, least1, is1);
+  bit_counts(x2, least2, is2);
+  return (one & ((is1[0] & least2[0]) | (is1[1] & least2[1]) | (is1[2] & least2[2]))) |
+         (two & ((is2[0] & least1[0]) | (is2[1] & least1[1]) | (is2[2] & least1[2])));
+}
+
+// The eight neighbours' bits of word w of row r on the torus.
 __device__ __forceinline__ void bit_neighbours(const uint32_t *plane, int32_t r, int32_t w,
                                                int32_t H, int32_t W, int32_t row_words,
                                                uint32_t (&x)[8]) {
@@ -505,20 +561,14 @@ __global__ void __launch_bounds__(kSmallThreads) k_schelling_small(SchellingSmal
     const int32_t tn = t + 1 < a.steps ? t + 1 : t;
     const Key ck = key;
     key = Key{a.keys[2 * tn], a.keys[2 * tn + 1]};  // the next step's, on its way meanwhile
-    // 8 same < 3 (same + other) is 5 same < 3 other: no like neighbour and 1
-    // or more others, 1 and 2 or more, 2 and 4 or more (3 would need 6)
     uint32_t count = 0;  // empty cells << 16 | unhappy agents
     for (int32_t w = w0; w < w1; ++w) {
       const int32_t r = w / rw, col = w - r * rw;
-      uint32_t x1[8], x2[8], least1[3], least2[3], is1[3], is2[3];
+      uint32_t x1[8], x2[8];
       bit_neighbours(one, r, col, a.H, W, rw, x1);
       bit_neighbours(two, r, col, a.H, W, rw, x2);
-      bit_counts(x1, least1, is1);
-      bit_counts(x2, least2, is2);
       const uint32_t o = one[w], p = two[w];
-      const uint32_t u =
-          (o & ((is1[0] & least2[0]) | (is1[1] & least2[1]) | (is1[2] & least2[2]))) |
-          (p & ((is2[0] & least1[0]) | (is2[1] & least1[1]) | (is2[2] & least1[2])));
+      const uint32_t u = bit_unhappy(o, p, x1, x2);
       sad[w] = u;
       const uint32_t e = ~(o | p) & (col == rw - 1 ? tail : ~0u);
       count += (uint32_t)__popc(e) << 16 | (uint32_t)__popc(u);
@@ -613,13 +663,15 @@ __global__ void __launch_bounds__(kSmallThreads) k_schelling_small(SchellingSmal
   }
 }
 
-// record[t] = (happy fraction, moves) from the integer counters
-__global__ void k_schelling_record(const int32_t *__restrict__ counters, int32_t steps,
-                                   int64_t n_agents, float *__restrict__ happy_frac,
-                                   int32_t *__restrict__ moves) {
+// record[t] = (happy fraction, moves) from the integer counters; the steps from
+// `launched` on are the identity and get their counters here
+__global__ void k_schelling_record(int32_t *__restrict__ counters, int32_t steps,
+                                   int32_t launched, int64_t n_agents,
+                                   float *__restrict__ happy_frac, int32_t *__restrict__ moves) {
   const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= steps) return;
-  happy_frac[t] = (float)counters[2 * t] / (float)n_agents;
+  if (t >= launched) counters[2 * t] = (int32_t)n_agents;
+  happy_frac[t] = (float)counters[2 * t] / (float)(n_agents > 0 ? n_agents : 1);
   moves[t] = counters[2 * t + 1];
 }
 
@@ -657,20 +709,20 @@ __global__ void k_fill_i32_s(int32_t *__restrict__ p, int64_t n, int32_t v) {
 // k_schelling_small may need more than 64 KB of dynamic LDS: the limit is
 // raised once per device, under a lock.
 constexpr int kMaxDevices = 64;
-std::mutex g_small_attr_mu;
-bool g_small_attr_set[kMaxDevices];
+std::mutex g_schelling_attr_mu;
+bool g_schelling_attr_set[kMaxDevices];
 
-int small_lds_attr() {
+int schelling_lds_attr() {
   int dev = -1;
   ABM_CHECK_HIP(hipGetDevice(&dev));
   ABM_REQUIRE(dev >= 0 && dev < kMaxDevices, "schelling: device index out of range");
-  std::lock_guard<std::mutex> lock(g_small_attr_mu);
-  if (!g_small_attr_set[dev]) {
+  std::lock_guard<std::mutex> lock(g_schelling_attr_mu);
+  if (!g_schelling_attr_set[dev]) {
     for (const void *k : {(const void *)k_schelling_small<kModeOriginal>,
                           (const void *)k_schelling_small<kModePartitionable>})
       ABM_CHECK_HIP(
           hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
-    g_small_attr_set[dev] = true;
+    g_schelling_attr_set[dev] = true;
   }
   return kOk;
 }
@@ -742,16 +794,25 @@ int abm_schelling_init(abm_schelling_grid *g, const uint32_t *key, int mode,
 
 }  // extern "C"
 
+// A watched run learns from the agents kernels how far it is; each
+// kWatchEvery-th step tells, and up to twice as many identity steps follow the
+// last move: 28 of 200 steps launched at 512 x 512, where 23 move or look, against
+// 48 in launches of 16 steps.  A run 648 us before, 484 with this and the kernels'
+// single round of loads.
+constexpr int32_t kWatchEvery = 4;
+
 // the step loop of a run; prev0: the counters of the step before the first
-// (nullptr: a fresh run, whose bitmap and block counts are built from the
-// cells first)
+// (nullptr: a fresh run, whose bitmap and block counts are built from the cells
+// first); watch: launching stops once a step was the identity
 static int schelling_steps(const abm_schelling_grid *g, const uint32_t *keys, int32_t steps,
                            int mode, const int32_t *prev0, int32_t *counters, float *happy_frac,
-                           int32_t *moves, void *stream, const char *what) {
+                           int32_t *moves, int32_t *watch, int32_t *launched, void *stream,
+                           const char *what) {
   if (int rc = check_grid(g, what)) return rc;
   ABM_REQUIRE(keys && counters && happy_frac && moves && steps >= 0 &&
                   (mode == 0 || mode == 1),
               "abm_schelling_run: bad arguments");
+  if (launched) *launched = steps;
   if (steps == 0) return kOk;
   hipStream_t s = (hipStream_t)stream;
   const int64_t nc = (int64_t)g->height * g->width;
@@ -759,12 +820,13 @@ static int schelling_steps(const abm_schelling_grid *g, const uint32_t *keys, in
   const unsigned nb = nblk(nc, kCellsPerBlock);
   ABM_REQUIRE(nb <= kMaxEmptyBlocks,
               "abm_schelling_run: grids of more than 15,360,000 cells are not supported");
-  const int64_t nwords = (nc + 31) / 32;
-  uint32_t *ebits = reinterpret_cast<uint32_t *>(g->empty);  // nwords <= H*W words
+  // whole blocks of bitmap words fit: 32 * nb <= H*W for any grid not run below
+  uint32_t *ebits = reinterpret_cast<uint32_t *>(g->empty);
   ABM_REQUIRE(((uintptr_t)ebits & 15u) == 0,
               "abm_schelling_run: the empty scratch must be 16-byte aligned");
+  const bool part = mode == kModePartitionable;
   if (schelling_small(g->height, g->width, g->n_agents)) {
-    if (int rc = small_lds_attr()) return rc;
+    if (int rc = schelling_lds_attr()) return rc;
     SchellingSmall a;
     a.H = g->height;
     a.W = g->width;
@@ -780,18 +842,18 @@ static int schelling_steps(const abm_schelling_grid *g, const uint32_t *keys, in
     a.counters = counters;
     a.happy_frac = happy_frac;
     a.moves = moves;
-    hipLaunchKernelGGL(mode == kModePartitionable ? k_schelling_small<kModePartitionable>
-                                                  : k_schelling_small<kModeOriginal>,
+    hipLaunchKernelGGL(part ? k_schelling_small<kModePartitionable>
+                            : k_schelling_small<kModeOriginal>,
                        dim3(1), dim3(kSmallThreads),
                        schelling_small_lds(g->height, g->width, g->n_agents), s, a);
     ABM_LAUNCH_CHECK(what);
     return kOk;
   }
+  if (watch) clear_watch(watch);
   hipLaunchKernelGGL(k_fill_i32_s, dim3(nblk(2 * (int64_t)steps, 256)), dim3(256), 0, s,
                      counters, 2 * (int64_t)steps, 0);
   if (!prev0) {
-    hipLaunchKernelGGL(k_empty_bits, dim3(nb), dim3(kCellsPerBlock), 0, s, g->cells, nc, nwords,
-                       ebits);
+    hipLaunchKernelGGL(k_empty_bits, dim3(nb), dim3(kCellsPerBlock), 0, s, g->cells, nc, ebits);
     // copy 0 = the grid's empty counts, the other copies start at zero
     hipLaunchKernelGGL(k_cells_count, dim3(nb), dim3(kCellsPerBlock), 0, s, g->cells, nc, 1,
                        g->block_counts);
@@ -802,7 +864,15 @@ static int schelling_steps(const abm_schelling_grid *g, const uint32_t *keys, in
   const dim3 tiles((unsigned)((g->width + kTileDim - 1) / kTileDim),
                    (unsigned)((g->height + kTileDim - 1) / kTileDim));
   const size_t prefix_lds = (size_t)(nb + 1) * sizeof(int32_t);
-  for (int32_t t = 0; t < steps; ++t) {
+  int32_t t = 0;
+  for (; t < steps; ++t) {
+    const bool tells = watch && t % kWatchEvery == 0;
+    if (tells && t >= 2 * kWatchEvery) {
+      bool settled = false;
+      if (int rc = wait_begun(watch, t + 1 - kWatchEvery, s, what, &settled)) return rc;
+      if (settled) break;
+    }
+    const int32_t *prev = t ? counters + 2 * (int64_t)(t - 1) : prev0;
     SchellingStep a;
     a.H = g->height;
     a.W = g->width;
@@ -812,24 +882,38 @@ static int schelling_steps(const abm_schelling_grid *g, const uint32_t *keys, in
     a.id = g->id;
     a.ebits = ebits;
     a.ecount = g->block_counts;
-    a.nwords = nwords;
     a.nb = (int32_t)nb;
     a.claim = g->claim;
     a.target = g->target;
     a.ck = keys + 2 * (int64_t)t;
-    a.mode = mode;
     a.happy_count = counters + 2 * (int64_t)t;
-    a.prev_happy = t ? counters + 2 * (int64_t)(t - 1) : prev0;
-    hipLaunchKernelGGL(k_schelling_agents, tiles, dim3(kTileDim * kTileDim), prefix_lds, s, a);
-    if (g->n_agents > 0)
+    a.prev_happy = prev;
+    a.watch = watch;
+    a.begun = tells ? t + 1 : 0;
+    hipLaunchKernelGGL(part ? k_schelling_agents<kModePartitionable>
+                            : k_schelling_agents<kModeOriginal>,
+                       tiles, dim3(kTileDim * kTileDim), prefix_lds, s, a);
+    if (g->n_agents > 0) {
+      SchellingMoves m;
+      m.n_agents = g->n_agents;
+      m.cells = g->cells;
+      m.id = g->id;
+      m.claim = g->claim;
+      m.pos = g->pos;
+      m.type = g->type;
+      m.target = g->target;
+      m.ebits = ebits;
+      m.ecount = g->block_counts;
+      m.nb = (int32_t)nb;
+      m.moves = counters + 2 * (int64_t)t + 1;
+      m.prev_happy = prev;
       hipLaunchKernelGGL(k_schelling_moves, dim3(nblk(g->n_agents, kMovesThreads)),
-                         dim3(kMovesThreads), 0, s,
-                         g->n_agents, g->cells, g->id, g->claim, g->pos, g->type, g->target,
-                         ebits, g->block_counts, (int32_t)nb, counters + 2 * (int64_t)t + 1,
-                         a.prev_happy);
+                         dim3(kMovesThreads), 0, s, m);
+    }
   }
   hipLaunchKernelGGL(k_schelling_record, dim3(nblk(steps, 256)), dim3(256), 0, s, counters,
-                     steps, g->n_agents > 0 ? g->n_agents : 1, happy_frac, moves);
+                     steps, t, g->n_agents, happy_frac, moves);
+  if (launched) *launched = t;
   ABM_LAUNCH_CHECK(what);
   return kOk;
 }
@@ -839,8 +923,8 @@ extern "C" {
 int abm_schelling_run(const abm_schelling_grid *g, const uint32_t *keys, int32_t steps,
                       int mode, int32_t *counters, float *happy_frac, int32_t *moves,
                       void *stream) {
-  return schelling_steps(g, keys, steps, mode, nullptr, counters, happy_frac, moves, stream,
-                         "abm_schelling_run");
+  return schelling_steps(g, keys, steps, mode, nullptr, counters, happy_frac, moves, nullptr,
+                         nullptr, stream, "abm_schelling_run");
 }
 
 int abm_schelling_run_from(const abm_schelling_grid *g, const uint32_t *keys, int32_t steps,
@@ -848,7 +932,16 @@ int abm_schelling_run_from(const abm_schelling_grid *g, const uint32_t *keys, in
                            float *happy_frac, int32_t *moves, void *stream) {
   ABM_REQUIRE(prev_counters, "abm_schelling_run_from: prev_counters is null");
   return schelling_steps(g, keys, steps, mode, prev_counters, counters, happy_frac, moves,
-                         stream, "abm_schelling_run_from");
+                         nullptr, nullptr, stream, "abm_schelling_run_from");
+}
+
+int abm_schelling_run_watched(const abm_schelling_grid *g, const uint32_t *keys, int32_t steps,
+                              int mode, const int32_t *prev_counters, int32_t *counters,
+                              float *happy_frac, int32_t *moves, int32_t *watch,
+                              int32_t *launched, void *stream) {
+  ABM_REQUIRE(watch && launched, "abm_schelling_run_watched: null buffer");
+  return schelling_steps(g, keys, steps, mode, prev_counters, counters, happy_frac, moves, watch,
+                         launched, stream, "abm_schelling_run_watched");
 }
 
 int abm_schelling_settled(const abm_schelling_grid *g, const int32_t *prev_counters, int32_t steps,

@@ -54,6 +54,7 @@
 
 #include "common.hpp"
 #include "jaxabm_amd.h"
+#include "watch.hpp"
 
 namespace abm {
 
@@ -101,10 +102,6 @@ struct SirStep {
   int32_t *watch;  // host memory, or null: [0] steps begun, [1] 1 once one was the identity
   int32_t begun;   // value for watch[0], or 0: this step does not tell
 };
-
-__device__ __forceinline__ void tell_host(int32_t *p, int32_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 
 // Workgroup barrier that orders LDS only.  Every intra-block exchange in the
 // step kernel goes through LDS (state, marks and bitmaps are never read back
@@ -709,24 +706,6 @@ int launch_step(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
 // 3.11 when each eighth does, 3.25 without a watch.
 constexpr int32_t kWatchEvery = 8;
 
-// Waits until step `begun` (counted from 1) has begun, or one was the identity.
-// An error of the stream ends the wait, and so does a stream that has finished
-// without saying so.
-int wait_begun(const int32_t *watch, int32_t begun, hipStream_t s, const char *who,
-               bool *settled) {
-  for (uint32_t spin = 0;; ++spin) {
-    *settled = __atomic_load_n(&watch[1], __ATOMIC_RELAXED) != 0;
-    if (*settled || __atomic_load_n(&watch[0], __ATOMIC_RELAXED) >= begun) return kOk;
-    if ((spin & 0x3FFF) != 0x3FFF) continue;
-    const hipError_t e = hipStreamQuery(s);
-    if (e == hipErrorNotReady) continue;
-    if (e != hipSuccess) return hip_fail(e, who);
-    if (__atomic_load_n(&watch[0], __ATOMIC_ACQUIRE) >= begun) return kOk;
-    set_error(std::string(who) + ": watch must be host memory the device can write");
-    return kErrInvalid;
-  }
-}
-
 // The steps of a run; with watch, launching stops once a step was the identity:
 // so is every later one, and the count reduction fills in their zeroed slots as
 // if they had been launched.
@@ -748,10 +727,7 @@ int sir_run(const char *who, const abm_sir_graph *g, uint8_t *state, uint16_t *m
   const uint32_t tb = unit_threshold(beta), tg = unit_threshold(gamma);
   const int64_t words = bitmap_words(g->n);
   const int64_t ns = (int64_t)steps * kStride;
-  if (watch) {
-    __atomic_store_n(&watch[0], 0, __ATOMIC_RELAXED);
-    __atomic_store_n(&watch[1], 0, __ATOMIC_RELEASE);
-  }
+  if (watch) clear_watch(watch);
   hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for(ns, 256)), dim3(256), 0, s,
                      slots, ns, 0);
   uint32_t *bm[2] = {bitmaps, bitmaps + words};

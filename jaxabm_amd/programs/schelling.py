@@ -50,6 +50,8 @@ class SchellingEngine:
                                 self.block_counts.data_ptr())
         self.n_agents = 0
         self._peek = None
+        self._watch = None   # pinned host words of a watched run
+        self.steps_launched = 0   # by the last run()
         self._stage = Staging(self.device)
         self.rng = np.zeros(2, np.uint32)
         self.reset(seed)
@@ -85,16 +87,25 @@ class SchellingEngine:
 
     def run(self, steps: int, chunk: int = SETTLE_CHUNK):
         """Run ``steps`` steps; returns host (fraction happy, moves) arrays.
-        ``chunk``: steps per launch, with the settled-grid exit of
-        run_settling (0: all steps in one launch; so is a run on a small grid,
-        whose one kernel has that exit itself)."""
+        ``chunk`` > 0: steps are launched while the host waits for the run, and
+        no more of them once the grid has settled (abm_schelling_run_watched);
+        0: all steps are launched."""
         keys = self._stage.upload(self._host_keys(steps)).view(torch.int32).view(-1, 2)
         counters = torch.empty((max(steps, 1), 2), dtype=torch.int32, device=self.device)
         out = torch.empty((2, max(steps, 1)), dtype=torch.int32, device=self.device)
         happy, moves = out[0].view(torch.float32), out[1]
-        if lib().abm_schelling_one_launch(C.byref(self._g)):
-            chunk = 0
-        self.run_settling(keys, steps, counters, happy, moves, chunk)
+        self.steps_launched = steps
+        if steps > 0 and chunk > 0:
+            if self._watch is None:
+                self._watch = torch.empty(2, dtype=torch.int32, pin_memory=True)
+            launched = C.c_int32()
+            check(lib().abm_schelling_run_watched(
+                C.byref(self._g), ptr(keys), int(steps), self.mode, None, ptr(counters),
+                ptr(happy), ptr(moves), C.c_void_p(self._watch.data_ptr()), C.byref(launched),
+                stream_handle()), "schelling_run")
+            self.steps_launched = int(launched.value)
+        elif steps > 0:
+            self.launch(keys, steps, counters, happy, moves)
         got = out.cpu().numpy()   # both records in one copy
         return got[0, :steps].view(np.float32), got[1, :steps]
 

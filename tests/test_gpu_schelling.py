@@ -173,3 +173,41 @@ def test_schelling_one_launch_runs(schelling, mode, H, W, one):
     want = np.full(H * W, -1, np.int32)
     want[pos] = np.arange(len(pos))
     np.testing.assert_array_equal(eng.id.cpu().numpy().reshape(-1), want)
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("H,W,steps", [(157, 157, 40), (800, 33, 40), (192, 160, 3),
+                                       (12289, 3, 8), (1, 25000, 8), (2, 13001, 8),
+                                       (614, 640, 8)])
+def test_schelling_watched_runs(schelling, mode, H, W, steps):
+    """Grids of two launches a step, among them ones of fewer rows or columns
+    than a tile and with a ragged last block of the bitmap: a watched run, and
+    the same steps on a second engine as 2 launched and the rest continued,
+    both equal to the oracle; a settled run stops launching."""
+    import torch
+
+    eng = schelling.SchellingEngine(H, W, seed=4, mode=mode)
+    cells, pos, typ, rng = O.schelling_init(H, W, 4, mode)
+    ohf, omv = O.schelling_run(H, W, cells, pos, typ, rng, steps, mode)
+    hf, mv = eng.run(steps)
+    S = steps
+    two = schelling.SchellingEngine(H, W, seed=4, mode=mode)
+    keys = two.key_table(S)
+    counters = torch.empty((S, 2), dtype=torch.int32, device="cuda")
+    happy = torch.empty(S, dtype=torch.float32, device="cuda")
+    moves = torch.empty(S, dtype=torch.int32, device="cuda")
+    two.launch(keys, 2, counters, happy, moves)
+    two.launch(keys[2:], S - 2, counters[2:], happy[2:], moves[2:], prev=counters[1])
+    want = np.full(H * W, -1, np.int32)
+    want[pos] = np.arange(len(pos))
+    for e, h, m in ((eng, hf, mv), (two, happy.cpu().numpy(), moves.cpu().numpy())):
+        np.testing.assert_array_equal(m, omv)
+        np.testing.assert_array_equal(h, ohf)
+        np.testing.assert_array_equal(e.grid().reshape(-1), cells)
+        np.testing.assert_array_equal(e.positions(), pos)
+        np.testing.assert_array_equal(e.id.cpu().numpy().reshape(-1), want)
+    if ohf[-1] == 1.0:
+        settled = int(np.argmax(ohf == 1.0)) + 1   # steps that are not the identity
+        assert settled <= eng.steps_launched <= min(S, settled + 9)
+    else:
+        assert eng.steps_launched == S
