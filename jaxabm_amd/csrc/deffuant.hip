@@ -84,11 +84,60 @@ __device__ __forceinline__ float gate(float eps, float d) {
   return 1.0f / den;
 }
 
+// x / kGateScale rounded once, in three operations: with y = 50 the rounded
+// reciprocal, q + (x - q c) y corrects q = x y to the rounded quotient
+// (Markstein, IBM J. Res. Dev. 34(1), 1990).  Equal to the IEEE division for
+// every float32 of [2^-60, 1.6] (all tested); below, the gate is 1 / 2 either
+// way.  As exact on 2^-87 <= x, where the remainder is a float32.
+__device__ __forceinline__ float div_gate_scale(float x) {
+  const float q = x * 50.0f;
+  return fmaf(fmaf(-q, kGateScale, x), 50.0f, q);
+}
+
+// 1 / d rounded once for 1 <= d < 2^120: the hardware estimate (1 ulp) and two
+// corrections (the second exact, Markstein as above).
+__device__ __forceinline__ float inv_rounded(float d) {
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
+
+// The gates of P differences, the same bits as gate(): its quotients
+// by div_gate_scale and inv_rounded, and abm_expf without its range branches,
+// for |eps - |d|| <= 1.2 (|z| <= 60); any other argument of the wavefront, NaN
+// included, sends it through gate().  34 operations a gate instead of about 58.
+// eps(u): the bound of difference u.
+template <int P, class Eps>
+__device__ __forceinline__ void gates(Eps eps, const float (&d)[P], float (&g)[P]) {
+  bool odd = false;
+#pragma unroll
+  for (int u = 0; u < P; ++u) {
+    const float num = eps(u) - fabsf(d[u]);
+    odd |= !(fabsf(num) <= 1.2f);
+    const float x = -div_gate_scale(num);
+    const float m = __builtin_rintf(x * 0x1.715476p0f);
+    const float r = (x - m * 0x1.62e4p-1f) - m * 0x1.7f7d1cp-20f;
+    float q = 0x1.a01a02p-13f;
+    q = 0x1.6c16c2p-10f + q * r;
+    q = 0x1.111112p-7f + q * r;
+    q = 0x1.555556p-5f + q * r;
+    q = 0x1.555556p-3f + q * r;
+    q = 0.5f + q * r;
+    const float p = 1.0f + (r + (r * r) * q);
+    g[u] = inv_rounded(1.0f + __builtin_ldexpf(p, (int)m));  // exact: no subnormal here
+  }
+  if (__ballot(odd)) {
+#pragma unroll
+    for (int u = 0; u < P; ++u) g[u] = gate(eps(u), d[u]);
+  }
+}
+
 // Pairs each wavefront holds in flight per loop iteration of the step kernel:
 // eight 1 KB row loads outstanding per wave (measured: 4 beats 2 and 8).
 constexpr int kDefStepPairs = 4;
 
-// One step for the whole batch.  src == dst updates in place (pairs are
+// One step for the whole batch.  Bound by the 128 MB a step moves at 65,536 x
+// 256 (23 us a step with gates(), 25.7 with gate()).  src == dst updates in place (pairs are
 // disjoint); otherwise every row of dst is written (the odd agent is copied).
 template <int VEC>
 __global__ void __launch_bounds__(kDefThreads)
@@ -129,14 +178,18 @@ __global__ void __launch_bounds__(kDefThreads)
       load_cols<VEC>(src + c[i] * B + col, xc[i]);
     }
 #pragma unroll
-    for (int i = 0; i < kDefStepPairs; ++i)
+    for (int i = 0; i < kDefStepPairs; ++i) {
+      float d[VEC], g[VEC];
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) d[v] = xc[i][v] - xa[i][v];
+      gates<VEC>([&](int v) { return e[v]; }, d, g);
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
-        const float d = xc[i][v] - xa[i][v];
-        const float delta = (m[v] * gate(e[v], d)) * d;
+        const float delta = (m[v] * g[v]) * d[v];
         xa[i][v] = xa[i][v] + delta;
         xc[i][v] = xc[i][v] - delta;
       }
+    }
 #pragma unroll
     for (int i = 0; i < kDefStepPairs; ++i)
       if (live[i]) {
@@ -151,6 +204,11 @@ __global__ void __launch_bounds__(kDefThreads)
     store_cols<VEC>(dst + r * B + col, x);
   }
 }
+
+// Pairs a wavefront holds in flight in the sweep: eight 1 KB row loads, as above.
+// 65,536 x 256: 36.3 us a sweep against 37.3 with one pair and IEEE quotients, bound
+// by the 192 MB that it moves.
+constexpr int kDefSweepPairs = 2;
 
 // Reverse sweep of one step: x_pre is the state before the step, lam holds
 // dL/dx after it and is updated in place to dL/dx before it.
@@ -178,29 +236,51 @@ __global__ void __launch_bounds__(kDefThreads)
     }
     const int64_t npairs = n >> 1;
     const int64_t stride = (int64_t)gridDim.y * kDefWaves;
-    for (int64_t p = (int64_t)blockIdx.y * kDefWaves + wave; p < npairs; p += stride) {
-      const int64_t a = perm[2 * p], c = perm[2 * p + 1];
-      float xa[VEC], xc[VEC], la[VEC], lc[VEC];
-      load_cols<VEC>(x_pre + a * B + col, xa);
-      load_cols<VEC>(x_pre + c * B + col, xc);
-      load_cols<VEC>(lam + a * B + col, la);
-      load_cols<VEC>(lam + c * B + col, lc);
+    for (int64_t p0 = (int64_t)blockIdx.y * kDefWaves + wave; p0 < npairs;
+         p0 += kDefSweepPairs * stride) {
+      // pairs p0, p0 + stride; one past the end re-reads pair p0 and counts
+      // and stores nothing
+      int64_t a[kDefSweepPairs], c[kDefSweepPairs];
+      bool live[kDefSweepPairs];
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) {
-        const float d = xc[v] - xa[v];
-        const float g = gate(e[v], d);
-        const float gp = g * (1.0f - g) / kGateScale;
-        const float fd = m[v] * (g - fabsf(d) * gp);
-        const float fe = m[v] * d * gp;
-        const float fm = g * d;
-        const float w = la[v] - lc[v];
-        la[v] = la[v] - w * fd;
-        lc[v] = lc[v] + w * fd;
-        ge[v] += (double)(w * fe);
-        gm[v] += (double)(w * fm);
+      for (int i = 0; i < kDefSweepPairs; ++i) {
+        const int64_t p = p0 + i * stride;
+        live[i] = p < npairs;
+        const int64_t pp = live[i] ? p : p0;
+        a[i] = perm[2 * pp];
+        c[i] = perm[2 * pp + 1];
       }
-      store_cols<VEC>(lam + a * B + col, la);
-      store_cols<VEC>(lam + c * B + col, lc);
+      float xa[kDefSweepPairs][VEC], xc[kDefSweepPairs][VEC];
+      float la[kDefSweepPairs][VEC], lc[kDefSweepPairs][VEC];
+#pragma unroll
+      for (int i = 0; i < kDefSweepPairs; ++i) {
+        load_cols<VEC>(x_pre + a[i] * B + col, xa[i]);
+        load_cols<VEC>(x_pre + c[i] * B + col, xc[i]);
+        load_cols<VEC>(lam + a[i] * B + col, la[i]);
+        load_cols<VEC>(lam + c[i] * B + col, lc[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < kDefSweepPairs; ++i) {
+        float d[VEC], g[VEC];
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) d[v] = xc[i][v] - xa[i][v];
+        gates<VEC>([&](int v) { return e[v]; }, d, g);
+        if (!live[i]) continue;
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) {
+          const float gp = div_gate_scale(g[v] * (1.0f - g[v]));
+          const float fd = m[v] * (g[v] - fabsf(d[v]) * gp);
+          const float fe = m[v] * d[v] * gp;
+          const float fm = g[v] * d[v];
+          const float w = la[i][v] - lc[i][v];
+          la[i][v] = la[i][v] - w * fd;
+          lc[i][v] = lc[i][v] + w * fd;
+          ge[v] += (double)(w * fe);
+          gm[v] += (double)(w * fm);
+        }
+        store_cols<VEC>(lam + a[i] * B + col, la[i]);
+        store_cols<VEC>(lam + c[i] * B + col, lc[i]);
+      }
     }
   }
 #pragma unroll
@@ -422,53 +502,6 @@ __device__ __forceinline__ void column_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// x / kGateScale rounded once, in three operations: with y = 50 the rounded
-// reciprocal, q + (x - q c) y corrects q = x y to the rounded quotient
-// (Markstein, IBM J. Res. Dev. 34(1), 1990).  Equal to the IEEE division for
-// every float32 of [2^-60, 1.6] (all tested); below, the gate is 1 / 2 either
-// way.
-__device__ __forceinline__ float div_gate_scale(float x) {
-  const float q = x * 50.0f;
-  return fmaf(fmaf(-q, kGateScale, x), 50.0f, q);
-}
-
-// 1 / d rounded once for 1 <= d < 2^120: the hardware estimate (1 ulp) and two
-// corrections (the second exact, Markstein as above).
-__device__ __forceinline__ float inv_rounded(float d) {
-  float r = __builtin_amdgcn_rcpf(d);
-  r = fmaf(fmaf(-d, r, 1.0f), r, r);
-  return fmaf(fmaf(-d, r, 1.0f), r, r);
-}
-
-// The gates of P differences, the same bits as gate(): its quotients
-// by div_gate_scale and inv_rounded, and abm_expf without its range branches,
-// for |eps - |d|| <= 1.6 (|z| <= 80); any other argument of the wavefront, NaN
-// included, sends it through gate().  34 operations a gate instead of about 58.
-template <int P>
-__device__ __forceinline__ void gates(float eps, const float (&d)[P], float (&g)[P]) {
-  bool odd = false;
-#pragma unroll
-  for (int u = 0; u < P; ++u) {
-    const float num = eps - fabsf(d[u]);
-    odd |= !(fabsf(num) <= 1.6f);
-    const float x = -div_gate_scale(num);
-    const float m = __builtin_rintf(x * 0x1.715476p0f);
-    const float r = (x - m * 0x1.62e4p-1f) - m * 0x1.7f7d1cp-20f;
-    float q = 0x1.a01a02p-13f;
-    q = 0x1.6c16c2p-10f + q * r;
-    q = 0x1.111112p-7f + q * r;
-    q = 0x1.555556p-5f + q * r;
-    q = 0x1.555556p-3f + q * r;
-    q = 0.5f + q * r;
-    const float p = 1.0f + (r + (r * r) * q);
-    g[u] = inv_rounded(1.0f + __builtin_ldexpf(p, (int)m));  // exact: no subnormal here
-  }
-  if (__ballot(odd)) {
-#pragma unroll
-    for (int u = 0; u < P; ++u) g[u] = gate(eps, d[u]);
-  }
-}
-
 // Accesses below go through raw buffers of one row: a pair past the end loads
 // pair (0, 0) and stores nothing, without a branch around the access (which
 // would make every later wait a full one).
@@ -532,7 +565,7 @@ __device__ __forceinline__ void column_steps(const ColumnRun &a, float *x, int32
         xc[u] = x[pr.p[u].y];
         d[u] = xc[u] - xa[u];
       }
-      gates<P>(eps, d, g);
+      gates<P>([eps](int) { return eps; }, d, g);
 #pragma unroll
       for (int u = 0; u < P; ++u) {
         const float delta = (mu * g[u]) * d[u];
@@ -608,7 +641,7 @@ __device__ __forceinline__ void column_sweep(const ColumnRun &a, float *l, int32
         la[u] = l[pr.p[u].x];
         lc[u] = l[pr.p[u].y];
       }
-      gates<P>(eps, d, g);
+      gates<P>([eps](int) { return eps; }, d, g);
 #pragma unroll
       for (int u = 0; u < P; ++u) {
         const float gp = div_gate_scale(g[u] * (1.0f - g[u]));
