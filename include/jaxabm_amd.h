@@ -489,6 +489,9 @@ int abm_graph_destroy(abm_graph *g);
  * nodes is refused (kErrInvalid) and left unchanged.  counts[4]: memsets
  * replaced, kernel nodes, memcpy nodes, empty nodes. */
 int abm_graph_sanitize(void *graph, int32_t *counts);
+/* A graph that runs a captured hipGraph_t (which it copies) `times` times in a
+ * row, for abm_graph_launch and abm_graph_destroy. */
+int abm_graph_repeat(void *graph, int32_t times, abm_graph **out);
 /* One launch of up to ABM_MAX_COPY_ITEMS device copies: item i copies
  * `bytes` from src to dst + row[0] * row_stride (row_stride 0: dst as is;
  * rows at or past row_limit are skipped).  The items (a host array) travel
@@ -566,6 +569,13 @@ typedef struct abm_reduce_item {
   int32_t reserved;
 } abm_reduce_item;
 int abm_reduce_batch(const abm_reduce_item *items, int32_t count, void *stream);
+/* abm_reduce_batch and abm_commit_step in one launch.  Items from n_early on
+ * (of n_items) copy results: their src is the out of a reduction.  No item's
+ * destination may overlap a reduction's input.  One node of a replayed step of JaxModel.run(graph=True). */
+int abm_reduce_commit_step(const abm_reduce_item *red, int32_t n_red, const abm_copy_item *items,
+                           int32_t n_early, int32_t n_items, int64_t *row, int32_t *ts,
+                           uint32_t *done, const uint32_t *key_table, int64_t key_rows,
+                           int32_t key_words, uint32_t *key_dst, void *stream);
 /* *out = Gini of int32 values: sorted x, S = sum (i+1) x_(i), T = sum x in
  * int32 (wrapping), G = f32(2S) / f32(nT) - f32((n+1)/n), 0 when T <= 1e-6. */
 int abm_gini_i32(const int32_t *x, int64_t n, float *out, void *ws, size_t ws_bytes,

@@ -215,6 +215,7 @@ SIGNATURES = {
     "abm_fill_i32": (_int, [_p, _i64, _i32, _p]),
     "abm_graph_begin": (_int, [_p]),
     "abm_graph_end": (_int, [_p, C.POINTER(_p)]),
+    "abm_graph_repeat": (_int, [_p, _i32, C.POINTER(_p)]),
     "abm_graph_launch": (_int, [_p, _p]),
     "abm_graph_destroy": (_int, [_p]),
     "abm_graph_sanitize": (_int, [_p, _p]),
@@ -230,6 +231,8 @@ SIGNATURES = {
     "abm_sum_i32": (_int, [_p, _i64, _p, _p, _sz, _p]),
     "abm_sum_u8": (_int, [_p, _i64, _p, _p, _sz, _p]),
     "abm_reduce_batch": (_int, [_p, _i32, _p]),
+    "abm_reduce_commit_step": (_int, [_p, _i32, _p, _i32, _i32, _p, _p, _p, _p, _i64, _i32, _p,
+                                      _p]),
     "abm_soft_hist_f32": (_int, [_p, _i64, _i32, C.c_double, _p, _p, _sz, _p]),
     "abm_gini_i32_noalloc": (_int, [_p, _i64, _p, _p]),
     "abm_rtc_compile": (_int, [C.c_char_p, C.c_char_p, C.POINTER(_p), C.POINTER(C.c_size_t)]),

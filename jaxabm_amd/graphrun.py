@@ -25,11 +25,10 @@ graph=True)`` turns that loop into graph replays:
 4. each replayed step reads its keys from row t of the table and the time
    step from a device counter.  It writes agent and env state back into the
    same buffers, and its metrics into row t of a device history.  So a graph
-   of several step bodies in a row replays several steps: a run of at least
-   BATCH_MIN_STEPS steps also captures STEPS_PER_LAUNCH bodies as one graph
-   and replays it while that many steps are left (then the one-step graph),
-   which saves most of a graph launch per step; shorter runs do not pay
-   for the extra capture.
+   that holds the captured one several times in a row replays several steps:
+   a run of at least BATCH_MIN_STEPS steps makes one of STEPS_PER_LAUNCH and
+   replays it while that many steps are left (then the one-step graph),
+   which saves most of a graph launch per step.
 
 Results are those of the eager loop bit for bit (same kernels, same order).
 Env values that are Python scalars become 0-d device tensors (int32,
@@ -38,7 +37,7 @@ after it; ``model_state['time_step']`` is a 0-d int32 device tensor during a
 replayed run.  Python values that a step computes from Python-side state are
 constants of the graph; a step whose Python values differ between steps is
 not replayed.  Capture evaluates the step's Python code once more than the
-steps it runs (STEPS_PER_LAUNCH + 1 times more in a batched run).
+steps it runs.
 """
 from __future__ import annotations
 
@@ -50,14 +49,15 @@ import torch
 
 from . import random as jr
 from . import reductions
-from ._lib import MAX_COPY_ITEMS, CopyItem, check, lib, stream_handle
+from ._lib import MAX_COPY_ITEMS, REDUCE_BATCH_MAX, CopyItem, check, lib, stream_handle
 
 _SCALARS = (bool, int, float)
-# step bodies per replayed graph in runs of at least BATCH_MIN_STEPS steps
-# (measured on a 10,000-agent model: about 24.6 us per replayed step one a
-# launch, 18.9 us eight a launch; capturing the eight costs about 2 ms)
+# steps per graph launch in runs of at least BATCH_MIN_STEPS steps.  Measured on
+# a 10,000-agent model: 21.5 us a replayed step one a launch, 18.3 eight a launch,
+# 17.7 thirty-two; making the graph of eight costs about 60 us, of thirty-two 200,
+# so that a run of 50 steps gains nothing from eight and one of 100 steps 7%
 STEPS_PER_LAUNCH = 8
-BATCH_MIN_STEPS = 400
+BATCH_MIN_STEPS = 64
 
 
 class NotReplayable(Exception):
@@ -106,6 +106,7 @@ class _Runner:
         self.env_python: Dict[str, Any] = {}
         self.hist: Dict[str, torch.Tensor] = {}
         self.metric_python: Dict[str, Any] = {}
+        self.waiting: List[Any] = []   # reductions of the last body, launched by its commit
         self.info: Dict[str, Any] = {"mode": "eager", "steps": n}
 
     # -------------------------------------------------------------- the body
@@ -123,8 +124,9 @@ class _Runner:
             c.update(current, keys[i], self.m.config)
         updated = {name: c.states for name, c in self.colls}
         env_new = dict(self.env)
-        # the callbacks' whole-array sums and means go out as one launch
-        with reductions.deferring():
+        # the callbacks' whole-array sums and means wait for commit(), which
+        # launches them with its copies
+        with reductions.deferring(hold=True):
             if self.has_env:
                 env_new = self.m._update_state_fn(dict(self.env), updated, self.m._params,
                                                   keys[len(self.colls)])
@@ -132,8 +134,11 @@ class _Runner:
                     raise NotReplayable("update_state_fn did not return a dict")
             metrics = (self.m._metrics_fn(env_new, updated, self.m._params)
                        if self.m._metrics_fn else {})
-        return (updated, reductions.materialize(env_new),
-                dict(reductions.materialize(metrics)))
+        if not all(v is None or isinstance(v, (torch.Tensor, str, *_SCALARS))
+                   for d in (env_new, metrics) for v in d.values()):
+            reductions.flush()   # a result may be inside a container
+        self.waiting = reductions.take()
+        return updated, reductions.plain(env_new), dict(reductions.plain(metrics))
 
     def _check(self, updated, env_new, metrics, first: bool):
         for name, _c in self.colls:
@@ -182,6 +187,19 @@ class _Runner:
             elif isinstance(slot, torch.Tensor):
                 env_fill.append((slot, v))
         dst_storages = {d.untyped_storage().data_ptr() for d, _ in pairs}
+        # The waiting reductions go out with the copies in one launch, and the
+        # copies of their results after them.  On their own before anything
+        # else, when there are too many, or one reads a buffer written here.
+        waiting, self.waiting = self.waiting, []
+
+        def launch_waiting():
+            reductions.launch(waiting)
+            waiting.clear()
+
+        if (len(waiting) > REDUCE_BATCH_MAX or
+                any(v.untyped_storage().data_ptr() in dst_storages for _op, v, *_ in waiting)):
+            launch_waiting()
+        results = {out.data_ptr() for _op, _v, out, *_ in waiting}
         srcs = []
         for d, t in pairs:
             if t is d or (t.data_ptr() == d.data_ptr() and t.stride() == d.stride()):
@@ -206,8 +224,10 @@ class _Runner:
 
         for (d, _), t in zip(pairs, srcs):
             if t is not None and not batched(t, d):
+                launch_waiting()
                 d.copy_(t)
         for slot, v in env_fill:
+            launch_waiting()
             slot.fill_(v)
         for name, c in self.colls:
             c._states = self.static[name]
@@ -216,14 +236,23 @@ class _Runner:
             if isinstance(v, torch.Tensor):
                 row = v.reshape(h.shape[1:])
                 if not batched(row, h, h[0].numel() * h.element_size(), h.shape[0]):
+                    launch_waiting()
                     h.index_copy_(0, self.row, v.reshape(1, *h.shape[1:]))
             else:
                 h.index_fill_(0, self.row, v)
+        tail = (self.row.data_ptr(), self.ts.data_ptr(), self.done.data_ptr(),
+                self.table.data_ptr(), self.n, 2 * self.width, self.keys.data_ptr(),
+                stream_handle())
+        if waiting:
+            early = [it for it in items if it.src not in results]
+            late = [it for it in items if it.src in results]
+            arr = (CopyItem * max(len(items), 1))(*early, *late)
+            check(lib().abm_reduce_commit_step(reductions.items(waiting), len(waiting), arr,
+                                               len(early), len(items), *tail),
+                  "reduce_commit_step")
+            return
         arr = (CopyItem * max(len(items), 1))(*items)
-        check(lib().abm_commit_step(arr, len(items), self.row.data_ptr(), self.ts.data_ptr(),
-                                    self.done.data_ptr(), self.table.data_ptr(), self.n,
-                                    2 * self.width, self.keys.data_ptr(), stream_handle()),
-              "commit_step")
+        check(lib().abm_commit_step(arr, len(items), *tail), "commit_step")
 
     def first_step(self):
         """Step 1, eagerly, on the model's own env values and Python time
@@ -271,22 +300,17 @@ class _Runner:
         self._check(updated, env_new, metrics, first=False)
         self.commit(updated, env_new, metrics)
 
-    def capture(self, steps: int = 1):
-        """A graph of ``steps`` step bodies in a row, each committed before
-        the next reads the fixed buffers."""
-        from ._lib import check, lib
-
+    def capture(self):
+        """A graph of one step body, committed into the fixed buffers."""
         g = torch.cuda.CUDAGraph(keep_graph=True)
         problem = None
         with torch.cuda.graph(g):
-            for _ in range(steps):
-                updated, env_new, metrics = self.body()
-                try:
-                    self._check(updated, env_new, metrics, first=False)
-                except NotReplayable as e:
-                    problem = e   # end the capture normally, then discard it
-                    break
+            updated, env_new, metrics = self.body()
+            try:
+                self._check(updated, env_new, metrics, first=False)
                 self.commit(updated, env_new, metrics)
+            except NotReplayable as e:
+                problem = e   # end the capture normally, then discard it
         if problem is not None:
             for name, c in self.colls:
                 c._states = self.static[name]
@@ -294,9 +318,8 @@ class _Runner:
         counts = (C.c_int32 * 4)()
         check(lib().abm_graph_sanitize(C.c_void_p(g.raw_cuda_graph()), counts), "graph_sanitize")
         g.instantiate()
-        if steps == 1:
-            self.info.update({"memsets_replaced": counts[0], "kernel_nodes": counts[1],
-                              "memcpy_nodes": counts[2]})
+        self.info.update({"memsets_replaced": counts[0], "kernel_nodes": counts[1],
+                          "memcpy_nodes": counts[2]})
         return g
 
     def finish(self, done: int):
@@ -345,7 +368,7 @@ def _needs_grad(model) -> bool:
 
 def run_graph(model, n: int, between=None) -> Dict[str, Any]:
     """Run up to ``n`` steps of ``model``: steps 1 and 2 eagerly, steps
-    3..n as replays of captured steps (STEPS_PER_LAUNCH a launch in runs of
+    3..n as replays of the captured step (STEPS_PER_LAUNCH a launch in runs of
     at least BATCH_MIN_STEPS steps while that many are left, else one).  Returns the run's info
     (``steps_done``: 0 when step 1 fails, 1 when step 2 cannot be replayed,
     2 when the capture is refused, n otherwise; ``mode``, ``reason``, node
@@ -376,24 +399,31 @@ def run_graph(model, n: int, between=None) -> Dict[str, Any]:
         r.finish(2)
         return {"mode": "eager", "steps": n, "steps_done": 2, "reason": "two steps"}
     k = STEPS_PER_LAUNCH if n >= BATCH_MIN_STEPS and STEPS_PER_LAUNCH > 1 else 1
+    gk = C.c_void_p()
     try:
         g = r.capture()
-        gk = r.capture(k) if k > 1 else None
+        if k > 1:
+            check(lib().abm_graph_repeat(C.c_void_p(g.raw_cuda_graph()), k, C.byref(gk)),
+                  "graph_repeat")
     except Exception as e:  # noqa: BLE001
         r.finish(2)
         return {"mode": "eager", "steps": n, "steps_done": 2,
                 "reason": f"capture: {type(e).__name__}: {e}"}
-    left = n - 2
-    while left > 0:
-        if gk is not None and left >= k:
-            gk.replay()
-            left -= k
-        else:
-            g.replay()
-            left -= 1
-        if between is not None and left > 0:
-            between()
-    r.finish(n)
-    del g, gk
+    try:
+        left = n - 2
+        while left > 0:
+            if k > 1 and left >= k:
+                check(lib().abm_graph_launch(gk, stream_handle()), "graph_launch")
+                left -= k
+            else:
+                g.replay()
+                left -= 1
+            if between is not None and left > 0:
+                between()
+        r.finish(n)
+    finally:
+        torch.cuda.current_stream().synchronize()
+        check(lib().abm_graph_destroy(gk), "graph_destroy")
+    del g
     r.info.update({"mode": "graph", "steps_done": n, "steps_per_launch": k})
     return r.info

@@ -126,11 +126,11 @@ def _pending() -> list:
     return p
 
 
-def flush() -> None:
-    """Launch the waiting reductions (abm_reduce_batch, up to 16 a launch)."""
+def take() -> list:
+    """The waiting reductions, no longer waiting here: the caller launches
+    them (``launch``, or ``items`` for a launch of its own) before anything
+    reads a result or changes an input."""
     pend = _pending()
-    if not pend:
-        return
     _tls.pending = []
     for _op, v, _out, _s, version in pend:
         if v._version != version:
@@ -138,35 +138,56 @@ def flush() -> None:
             raise RuntimeError("an array was modified in place after a whole-array sum or mean "
                                "of it inside a model callback; compute the reduction after the "
                                "update, or update a copy")
-    stream = pend[0][3]
+    return pend
+
+
+def items(part: list):
+    return (ReduceItem * len(part))(*[ReduceItem(v.data_ptr(), v.numel(), out.data_ptr(), op, 0)
+                                      for op, v, out, _s, _ver in part])
+
+
+def launch(pend: list) -> None:
+    """abm_reduce_batch, up to 16 a launch."""
     for i in range(0, len(pend), REDUCE_BATCH_MAX):
         part = pend[i:i + REDUCE_BATCH_MAX]
-        items = (ReduceItem * len(part))(*[ReduceItem(v.data_ptr(), v.numel(), out.data_ptr(),
-                                                      op, 0) for op, v, out, _s, _ver in part])
-        check(_fn("abm_reduce_batch")(items, len(part), stream), "reduce_batch")
+        check(_fn("abm_reduce_batch")(items(part), len(part), part[0][3]), "reduce_batch")
+
+
+def flush() -> None:
+    """Launch the waiting reductions."""
+    launch(take())
 
 
 @contextlib.contextmanager
-def deferring():
+def deferring(hold: bool = False):
     """Batch the whole-array sums and means issued inside into one launch
-    (at the end of the outermost scope, or earlier when a result is read)."""
+    (at the end of the outermost scope, or earlier when a result is read).
+    ``hold``: a scope that ends without an error leaves them for ``take``."""
     depth = getattr(_tls, "depth", 0)
     _tls.depth = depth + 1
+    done = False
     try:
         yield
+        done = True
     finally:
         _tls.depth = depth
-        if depth == 0:
+        if depth == 0 and not (hold and done):
             flush()
+
+
+def plain(d):
+    """``d`` (a dict of callback results) with deferred results replaced by
+    their tensors."""
+    if isinstance(d, dict) and any(isinstance(v, _Deferred) for v in d.values()):
+        return {k: (v._abm_plain if isinstance(v, _Deferred) else v) for k, v in d.items()}
+    return d
 
 
 def materialize(d):
     """``d`` (a dict of callback results) with deferred results replaced by
     plain tensors, the waiting reductions launched first."""
     flush()
-    if isinstance(d, dict) and any(isinstance(v, _Deferred) for v in d.values()):
-        return {k: (v._abm_plain if isinstance(v, _Deferred) else v) for k, v in d.items()}
-    return d
+    return plain(d)
 
 
 def _whole_call(name: str, v: torch.Tensor, out_dtype) -> torch.Tensor:
