@@ -187,3 +187,31 @@ def test_rows_at_the_end_of_the_entry_array(sir):
         want = O.sir_run(row_ptr, col, st, key, 0.6, 0.1, 20, O.MODE_PARTITIONABLE)
         np.testing.assert_array_equal(eng.run(20), want)
         np.testing.assert_array_equal(eng.state_host(), st)
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("chunk_cost", [1, 3000, 1 << 40])
+def test_heavy_row_units_and_light_groups(sir, mode, chunk_cost):
+    """150 hubs (more than one batch of 64) of degrees around multiples of 64
+    beside light rows whose number at risk passes the group limits: tiles of 64
+    agents up to one tile of all, equal to the oracle at every step."""
+    n, steps, n0 = 6000, 60, 3
+    rs = np.random.default_rng(11)
+    adj = [set() for _ in range(n)]
+    degrees = [33, 63, 64, 65, 127, 128, 129, 192, 600]
+    for h in range(150):
+        for u in rs.choice(np.arange(150, n), degrees[h % len(degrees)], replace=False):
+            adj[h].add(int(u))
+            adj[int(u)].add(h)
+    for v in range(150, n - 1):   # a path: nobody is out of reach
+        adj[v].add(v + 1)
+        adj[v + 1].add(v)
+    row_ptr = np.concatenate([[0], np.cumsum([len(a) for a in adj])]).astype(np.int32)
+    col = np.concatenate([np.sort(np.fromiter(a, np.int32)) for a in adj]).astype(np.int32)
+    eng = sir.SIRNetworkEngine(n, csr=(row_ptr, col), beta=0.03, gamma=0.05, n_seed_infected=n0,
+                               seed=6, mode=mode, chunk_cost=chunk_cost)
+    st, rng = O.sir_init(n, n0, 6, mode)
+    want = O.sir_run(row_ptr, col, st, rng, 0.03, 0.05, steps, mode)
+    np.testing.assert_array_equal(eng.run(steps), want)
+    np.testing.assert_array_equal(eng.state_host(), st)
+    assert want[:, 1].max() > n // 4
