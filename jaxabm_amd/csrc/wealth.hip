@@ -32,6 +32,7 @@
 // (20 bytes per agent), a larger one on its global buffers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #define ABM_STRAIGHT_DRAWS
@@ -775,6 +776,14 @@ const ExchangeVariant kExchange[] = {
     exchange_variant<16, false>(), exchange_variant<20, false>(), exchange_variant<24, true>(),
     exchange_variant<32, true>(),  exchange_variant<40, true>()};
 
+// Workgroups of the draws kernel for each of `count` instances.  A draw is a
+// chain of about 900 dependent operations, so a SIMD wants its 8 wavefronts:
+// 2,048 workgroups fill the chip (5,003 x 150: 29 us, 33 with 512); many
+// instances fill it with 512 each.
+unsigned draw_blocks(int32_t count) {
+  return (unsigned)std::max(512, std::min(2048, 4096 / std::max(count, 1)));
+}
+
 // These kernels may need more than 64 KB of dynamic LDS: the limits are
 // raised once per device, under a lock.
 constexpr int kMaxDevices = 64;
@@ -896,7 +905,7 @@ int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t ma
   if (dyn < (size_t)(cap + 1) * 4) dyn = (size_t)(cap + 1) * 4;
   hipLaunchKernelGGL(mode == kModePartitionable ? k_wealth_draws<kModePartitionable>
                                                 : k_wealth_draws<kModeOriginal>,
-                     dim3(512u, (unsigned)count), dim3(kDrawThreads), 0, s, insts);
+                     dim3(draw_blocks(count), (unsigned)count), dim3(kDrawThreads), 0, s, insts);
   hipLaunchKernelGGL(v->kernel, dim3((unsigned)(count * (1 + per))), dim3(kWealthThreads),
                      v->lds, s, insts, count, cap);
   hipLaunchKernelGGL(k_wealth_records, dim3(256u, (unsigned)count), dim3(kWealthThreads), dyn, s,
