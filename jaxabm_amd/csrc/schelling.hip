@@ -204,26 +204,36 @@ __device__ __forceinline__ int32_t jth_empty(uint32_t j, const int32_t *P, int n
   }
   uint32_t r = j - (uint32_t)P[lo];
   const int64_t w0 = (int64_t)lo * kWordsPerBlock;
-  uint32_t wv[kWordsPerBlock];
+  uint4 v[kWordsPerBlock / 4];
+#pragma unroll
+  for (int q = 0; q < kWordsPerBlock / 4; ++q) v[q] = reinterpret_cast<const uint4 *>(ebits + w0)[q];
+  // the four words, then the word: the last with at most r bits before it
+  uint32_t n = 0, before = 0, w = 0;
+  uint4 four = v[0];
 #pragma unroll
   for (int q = 0; q < kWordsPerBlock / 4; ++q) {
-    const uint4 v = reinterpret_cast<const uint4 *>(ebits + w0)[q];
-    wv[4 * q] = v.x;
-    wv[4 * q + 1] = v.y;
-    wv[4 * q + 2] = v.z;
-    wv[4 * q + 3] = v.w;
-  }
-  // the word: the last one with at most r bits before it
-  uint32_t n = 0, before = 0, word = 0, w = 0;
-#pragma unroll
-  for (int q = 0; q < kWordsPerBlock; ++q) {
     const bool here = n <= r;
     before = here ? n : before;
-    word = here ? wv[q] : word;
-    w = here ? q : w;
-    n += (uint32_t)__popc(wv[q]);
+    four.x = here ? v[q].x : four.x;
+    four.y = here ? v[q].y : four.y;
+    four.z = here ? v[q].z : four.z;
+    four.w = here ? v[q].w : four.w;
+    w = here ? 4 * q : w;
+    n += (uint32_t)(__popc(v[q].x) + __popc(v[q].y) + __popc(v[q].z) + __popc(v[q].w));
   }
   if (r >= n) return -1;
+  const uint32_t words[4] = {four.x, four.y, four.z, four.w};
+  uint32_t word = four.x;
+  n = before;
+  const uint32_t w4 = w;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const bool here = n <= r;
+    before = here ? n : before;
+    word = here ? words[q] : word;
+    w = here ? w4 + q : w;
+    n += (uint32_t)__popc(words[q]);
+  }
   // the bit, by halves
   r -= before;
   uint32_t bit = 0;
@@ -263,13 +273,16 @@ __device__ __forceinline__ bool schelling_identity(const int32_t *prev_happy, in
   return prev_happy && (int64_t)*prev_happy == n_agents;
 }
 
-// Bound by its chain, not by bytes or instructions: one round of loads, the
-// prefix's barriers, the draw, the bitmap line, the claim's atomic, each from
-// memory that another XCD wrote a launch before.  14.5 -> 10.8 us in the first
-// steps at 512 x 512 with the identity word loaded beside the tile, no modulo,
-// and the line read 16 bytes at a time.  (Bit planes of the whole grid read and
-// scanned by every workgroup in place of counts, tiles and the search in memory
-// took 12.4, and 779 us against 600 for 40 steps of 614 x 640.)
+// Bound by its chain, not by bytes or instructions: the step before's count, one
+// round of loads, the prefix's barriers, the draw, the bitmap line, the claim's
+// atomic, each from memory that another XCD wrote a launch before.  Two
+// workgroups a CU (8 wavefronts a SIMD, 64 registers) pay from about 300,000
+// cells on, but not with registers spilled: 40 steps of 1,030 x 1,030 took 1,331
+// us before the loads left their branches, 1,122 now, 1,278 at 72 registers and
+// 1,689 spilling; 200 steps of 512 x 512, all launched, 1,335 and 1,190.  (Bit
+// planes of the whole grid read and scanned by every workgroup in place of
+// counts, tiles and the search in memory took 779 us against 600 for 40 steps of
+// 614 x 640.)
 template <int kMode>
 __global__ void __launch_bounds__(kTileDim * kTileDim, 8) k_schelling_agents(SchellingStep a) {
   extern __shared__ int32_t empty_prefix_lds[];  // [nb + 1]
@@ -280,41 +293,51 @@ __global__ void __launch_bounds__(kTileDim * kTileDim, 8) k_schelling_agents(Sch
   __shared__ int32_t nwork;
   constexpr int kHalo = (kTileDim + 2) * (kTileDim + 2);  // 34 x 34 cells, <= 2 per thread
   const int tid = threadIdx.x;
-  const bool first_thread = blockIdx.x == 0 && blockIdx.y == 0 && tid == 0;
-  if (a.begun && first_thread) tell_host(&a.watch[0], a.begun);
   const int tx = tid % kTileDim, ty = tid / kTileDim;
   const int r0 = blockIdx.y * kTileDim, c0 = blockIdx.x * kTileDim;
   const int r = r0 + ty, c = c0 + tx;
   const bool inside = r < a.H && c < a.W;
   const int64_t cell = (int64_t)r * a.W + c;
-  // one memory round trip: the tile and its torus halo, this thread's block
-  // count for the prefix, the agent on this thread's cell, the step before's
-  // count
-  int8_t tv[2] = {0, 0};
+  // One memory round trip after the step before's count: the tile and its torus
+  // halo, this thread's block counts for the prefix, the agent on its cell.  No
+  // load is in a branch (one there waits for all before it): a thread without
+  // a place of its own loads another's.
+  const int32_t prev = *(a.prev_happy ? a.prev_happy : a.happy_count);
+  int8_t tv[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int q = tid + i * (int)blockDim.x;
-    if (q < kHalo) {
-      const int lr = q / (kTileDim + 2), lc = q % (kTileDim + 2);
-      // r0 < H and c0 < W; the tile may pass the edge by up to 32 cells
-      int gr = r0 + lr - 1, gc = c0 + lc - 1;
-      if (gr < 0) gr += a.H;
-      while (gr >= a.H) gr -= a.H;
-      if (gc < 0) gc += a.W;
-      while (gc >= a.W) gc -= a.W;
-      tv[i] = a.cells[(int64_t)gr * a.W + gc];
-    }
+    const int q = min(tid + i * kTileDim * kTileDim, kHalo - 1);
+    const int lr = q / (kTileDim + 2), lc = q % (kTileDim + 2);
+    // r0 < H and c0 < W: at most 32 cells past the edge
+    int gr = r0 + lr - 1 + a.H, gc = c0 + lc - 1 + a.W;
+    if (a.H <= kTileDim) gr %= a.H;
+    if (a.W <= kTileDim) gc %= a.W;
+    gr -= gr >= a.H ? a.H : 0;
+    gr -= gr >= a.H ? a.H : 0;
+    gc -= gc >= a.W ? a.W : 0;
+    gc -= gc >= a.W ? a.W : 0;
+    tv[i] = a.cells[(int64_t)gr * a.W + gc];
   }
-  const int32_t first = tid < a.nb ? block_empty(a.ecount, a.nb, tid) : 0;
-  const int32_t k = inside ? a.id[cell] : -1;
-  if (schelling_identity(a.prev_happy, a.n_agents)) {  // grid-uniform
+  const int block = min(tid, a.nb - 1);
+  int32_t copies[kCountCopies];
+#pragma unroll
+  for (int q = 0; q < kCountCopies; ++q) copies[q] = a.ecount[(int64_t)q * a.nb + block];
+  const int32_t id = a.id[inside ? cell : 0];
+  if (a.prev_happy && prev == (int32_t)a.n_agents) {  // grid-uniform: the identity
     // every agent happy again; no target is drawn (the last step left each
     // agent's target at -1) and the moves kernel exits too
-    if (first_thread) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) {
       *a.happy_count = (int32_t)a.n_agents;
-      if (a.watch) tell_host(&a.watch[1], 1);
+      if (a.watch) tell_host(&a.watch[1], 1);  // which ends the host's wait too
     }
     return;
+  }
+  if (a.begun && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) tell_host(&a.watch[0], a.begun);
+  const int32_t k = inside ? id : -1;
+  int32_t first = 0;
+  if (tid < a.nb) {
+#pragma unroll
+    for (int q = 0; q < kCountCopies; ++q) first += copies[q];
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
