@@ -184,7 +184,10 @@ def pmc_probe(workload: str = "sir") -> int:
     row_ptr, col = ba_csr(N_AGENTS, BA_M, GRAPH_SEED)
     eng = SIRNetworkEngine(N_AGENTS, csr=(row_ptr, col), beta=BETA, gamma=GAMMA,
                            n_seed_infected=N_SEED, seed=SEED)
-    counts = eng.run(SIM_STEPS)
+    # every step launched, as in the measured replays (run() stops at the last infection)
+    counts = torch.empty((SIM_STEPS, 3), dtype=torch.int32, device="cuda")
+    eng.launch(eng.key_table(SIM_STEPS), SIM_STEPS, counts)
+    torch.cuda.synchronize()
     print(json.dumps({"probe": "copy 256 MiB x3 (read 256 MiB + write 256 MiB each) + one "
                       "365-step SIR simulation", "copy_bytes": nbytes,
                       "final_counts": counts[-1].tolist()}))

@@ -313,7 +313,7 @@ typedef struct abm_schelling_grid {
   int32_t *empty;        /* device [H*W], 16-byte aligned: scratch (empty-cell bitmap) */
   int32_t *block_counts; /* device [abm_schelling_block_count(H*W)]: scratch (cells
                             per 1024-cell block: agents at init; empty cells
-                            during a run, in 8 copies summed by the readers) */
+                            during a run, in 16 copies summed by the readers) */
 } abm_schelling_grid;
 /* Length in int32 of the block_counts scratch for a grid of n_cells cells:
  * 16 x ceil(n_cells / 1024). */
