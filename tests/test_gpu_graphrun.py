@@ -427,3 +427,97 @@ def test_env_callback_that_updates_its_env_in_place(J):
         out.append(([float(v) for v in res["p"]], [int(v) for v in res["q"]]))
     assert out[0] == out[1]
     assert out[0][1] == list(range(1, 31))
+
+
+def test_repeated_graph_of_a_large_model(J):
+    """262,144 agents, 75 steps: graphs of eight captured steps that hold
+    copies and fills beside the kernels (multi-workgroup reductions with their
+    memsets replaced), with eager work and a synchronisation between the
+    replays, equal the eager loop; the run continues."""
+    import torch
+
+    from jaxabm_amd.graphrun import run_graph
+
+    a, b = make_trader(J), make_trader(J)
+    ra = a.run(75)
+    b.initialize()
+    b._history = []
+    scratch = torch.rand(1 << 20, device="cuda")
+
+    def between():
+        scratch.mul_(1.0001).sum()
+        torch.cuda.synchronize()
+
+    info = run_graph(b, 75, between=between)
+    assert info["mode"] == "graph" and info["steps_per_launch"] == 8
+    assert info["memsets_replaced"] > 0
+    out = {"step": [h["time_step"] for h in b._history]}
+    for k in b._history[0]["metrics"]:
+        out[k] = [h["metrics"][k] for h in b._history]
+    assert_same_run(a, b, dict(ra), out)
+    assert_same_run(a, b, a.run(66), b.run(66, graph=True))
+
+
+@pytest.mark.parametrize("extra", [0, 3, 17])
+def test_reductions_that_cannot_wait_for_the_commit(J, extra):
+    """Whole-array reductions go out with the commit's copies, unless one reads
+    an env buffer that the commit replaces, or there are more than a launch
+    takes: such models equal the eager loop."""
+    import torch
+
+    from jaxabm_amd import numpy as jnp
+
+    def env_fn(env, agents, params, key):
+        x = agents["t"]["x"]
+        out = dict(env)
+        out["old"] = jnp.sum(env["field"])   # reads the slot that the next line's copy replaces
+        out["field"] = x * 0.5 + 1.0
+        for i in range(extra):
+            out[f"s{i}"] = jnp.mean(x)
+        return out
+
+    def metrics(env, agents, params):
+        return {"old": env["old"], "mean": jnp.mean(agents["t"]["x"])}
+
+    def make():
+        m = make_trader(J, n=1500, metrics=metrics, env_fn=env_fn)
+        m.add_env_state("field", torch.ones(1500, device="cuda"))
+        m.add_env_state("old", torch.zeros((), device="cuda"))
+        for i in range(extra):
+            m.add_env_state(f"s{i}", torch.zeros((), device="cuda"))
+        return m
+
+    a, b = make(), make()
+    assert_same_run(a, b, a.run(70), b.run(70, graph=True))
+    assert b.last_run_info["mode"] == "graph", b.last_run_info
+    assert b.last_run_info["steps_per_launch"] == 8
+
+
+def test_reduction_inside_a_container(J):
+    """A deferred result inside a container is computed when the callbacks
+    end, whatever way the run then takes."""
+    from jaxabm_amd import numpy as jnp
+
+    def env_fn(env, agents, params, key):
+        return {**env, "pair": (jnp.mean(agents["t"]["x"]), 1)}
+
+    def metrics(env, agents, params):
+        return {"sum": jnp.sum(agents["t"]["x"])}
+
+    a = make_trader(J, n=1500, metrics=metrics, env_fn=env_fn)
+    b = make_trader(J, n=1500, metrics=metrics, env_fn=env_fn)
+    ra, rb = a.run(5), b.run(5, graph=True)
+    assert [float(v) for v in ra["sum"]] == [float(v) for v in rb["sum"]]
+    pa, pb = a._env_state["pair"], b._env_state["pair"]
+    assert float(pa[0]) == float(pb[0]) and pa[1] == pb[1] == 1
+
+
+def test_graph_repeat_rejects_bad_arguments(J):
+    import ctypes as C
+
+    from jaxabm_amd._lib import lib
+
+    out = C.c_void_p()
+    for times in (0, -1, 3):
+        assert lib().abm_graph_repeat(None, times, C.byref(out)) != 0
+    assert out.value is None

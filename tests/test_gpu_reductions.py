@@ -246,3 +246,62 @@ def test_reduction_routing_rules(R):
     g = torch.ones(5, device="cuda", requires_grad=True)
     jnp.mean(g * 2).backward()
     assert torch.allclose(g.grad, torch.full((5,), 0.4, device="cuda"))
+
+
+@pytest.mark.parametrize("n_red,n_early", [(1, 0), (1, 2), (5, 1), (16, 2)])
+@pytest.mark.parametrize("n", [1, 1023, 16_385, 65_536])
+def test_reduce_commit_step(R, n, n_red, n_early):
+    """One launch reduces, copies, and copies the results on: every result as
+    abm_reduce_batch gives it, in its slot and in the history row; early
+    copies of aligned and ragged sizes; counters and next keys as
+    abm_commit_step leaves them, over three steps of a two-row history."""
+    import torch
+
+    from jaxabm_amd._lib import CopyItem, ReduceItem, check, lib
+
+    rs = np.random.default_rng(n + n_red)
+    dtypes = [torch.float32, torch.float32, torch.int32, torch.int32, torch.uint8]
+    outs = [torch.float32, torch.float32, torch.int32, torch.float32, torch.int32]
+    xs = [torch.from_numpy(rs.integers(0, 200, n)).to(dtypes[i % 5]).cuda() for i in range(n_red)]
+    want = [torch.empty((), dtype=outs[i % 5], device="cuda") for i in range(n_red)]
+    got = [torch.zeros_like(w) for w in want]
+    slots = [torch.zeros_like(w) for w in want]
+    hist = [torch.zeros(2, dtype=w.dtype, device="cuda") for w in want]
+
+    def reduce_items(dst):
+        return (ReduceItem * n_red)(*[ReduceItem(x.data_ptr(), n, o.data_ptr(), i % 5, 0)
+                                      for i, (x, o) in enumerate(zip(xs, dst))])
+
+    check(lib().abm_reduce_batch(reduce_items(want), n_red, None), "reduce_batch")
+    red = reduce_items(got)
+    src = [torch.from_numpy(rs.integers(0, 255, 4 * n + 3).astype(np.uint8)).cuda()
+           for _ in range(n_early)]
+    dst = [torch.zeros_like(s) for s in src]
+    sizes = [4 * n + 3, 16 * (n // 4)][:n_early]
+    items = [CopyItem(s.data_ptr(), d.data_ptr(), b, 0, 0) for s, d, b in zip(src, dst, sizes)]
+    for g, sl, h in zip(got, slots, hist):
+        items += [CopyItem(g.data_ptr(), sl.data_ptr(), 4, 0, 0),
+                  CopyItem(g.data_ptr(), h.data_ptr(), 4, 4, 2)]
+    items = (CopyItem * len(items))(*items)
+    row = torch.zeros(1, dtype=torch.int64, device="cuda")
+    ts = torch.full((), 7, dtype=torch.int32, device="cuda")
+    done = torch.zeros(1, dtype=torch.int32, device="cuda")
+    table = torch.arange(6, dtype=torch.int32, device="cuda")
+    keys = table[:2].clone()
+    tail = (row.data_ptr(), ts.data_ptr(), done.data_ptr(), table.data_ptr(), 3, 2,
+            keys.data_ptr(), None)
+    torch.cuda.synchronize()
+    for step in range(3):
+        check(lib().abm_reduce_commit_step(red, n_red, items, n_early, len(items), *tail), "commit")
+        torch.cuda.synchronize()
+        assert (int(row), int(ts), int(done)) == (step + 1, 8 + step, 0)
+        r = min(step + 1, 2)
+        np.testing.assert_array_equal(keys.cpu().numpy(), [2 * r, 2 * r + 1])
+        for w, g, sl, h in zip(want, got, slots, hist):
+            assert g.item() == w.item() == sl.item()
+            np.testing.assert_array_equal(h.cpu().numpy()[:r], np.full(r, w.cpu().numpy()))
+    for s, d, b in zip(src, dst, sizes):
+        np.testing.assert_array_equal(d.cpu().numpy()[:b], s.cpu().numpy()[:b])
+        assert not d.cpu().numpy()[b:].any()
+    for count, early in ((0, n_early), (17, n_early), (n_red, -1), (n_red, len(items) + 1)):
+        assert lib().abm_reduce_commit_step(red, count, items, early, len(items), *tail) != 0
