@@ -8,6 +8,7 @@
 
 #include "common.hpp"
 #include "jaxabm_amd.h"
+#include "watch_wait.hpp"
 
 namespace abm {
 
@@ -20,22 +21,23 @@ inline void clear_watch(int32_t *watch) {
   __atomic_store_n(&watch[1], 0, __ATOMIC_RELEASE);
 }
 
-// Waits until step `begun` (counted from 1) has begun, or one was the identity.
-// An error of the stream ends the wait, and so does a stream that has finished
-// without saying so.
+// wait_watch on a stream; *settled: one step was the identity.
 inline int wait_begun(const int32_t *watch, int32_t begun, hipStream_t s, const char *who,
                       bool *settled) {
-  for (uint32_t spin = 0;; ++spin) {
-    *settled = __atomic_load_n(&watch[1], __ATOMIC_RELAXED) != 0;
-    if (*settled || __atomic_load_n(&watch[0], __ATOMIC_RELAXED) >= begun) return kOk;
-    if ((spin & 0x3FFF) != 0x3FFF) continue;
-    const hipError_t e = hipStreamQuery(s);
-    if (e == hipErrorNotReady) continue;
-    if (e != hipSuccess) return hip_fail(e, who);
-    if (__atomic_load_n(&watch[0], __ATOMIC_ACQUIRE) >= begun) return kOk;
+  hipError_t e = hipSuccess;
+  const Waited w = wait_watch(watch, begun, [&] {
+    e = hipStreamQuery(s);
+    return e == hipSuccess         ? StreamState::kIdle
+           : e == hipErrorNotReady ? StreamState::kRunning
+                                   : StreamState::kFailed;
+  });
+  *settled = w == Waited::kSettled;
+  if (w == Waited::kFailed) return hip_fail(e, who);
+  if (w == Waited::kSilent) {
     set_error(std::string(who) + ": watch must be host memory the device can write");
     return kErrInvalid;
   }
+  return kOk;
 }
 
 }  // namespace abm
