@@ -139,10 +139,13 @@ class SIRNetworkEngine:
         if self._watch is None:
             self._watch = torch.empty(2, dtype=torch.int32, pin_memory=True)
         launched = C.c_int32()
+        # held until the counts are back: the call launches while it waits, and
+        # lets other threads allocate meanwhile
+        slots = self.slot_buffer(steps)
         check(lib().abm_sir_run_watched(
             C.byref(self._g), ptr(self.state), ptr(self.mark), ptr(self.bitmaps),
             self.t & 0xFFFFFFFF, ptr(keys), int(steps), self.beta, self.gamma, self.mode,
-            ptr(self.slot_buffer(steps)), ptr(counts), C.c_void_p(self._watch.data_ptr()),
+            ptr(slots), ptr(counts), C.c_void_p(self._watch.data_ptr()),
             C.byref(launched), stream_handle()), "sir_run")
         self.t += int(steps)
         self.steps_launched = int(launched.value)
