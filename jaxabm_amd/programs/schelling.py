@@ -90,12 +90,15 @@ class SchellingEngine:
         ``chunk`` > 0: steps are launched while the host waits for the run, and
         no more of them once the grid has settled (abm_schelling_run_watched);
         0: all steps are launched."""
-        keys = self._stage.upload(self._host_keys(steps)).view(torch.int32).view(-1, 2)
-        counters = torch.empty((max(steps, 1), 2), dtype=torch.int32, device=self.device)
-        out = torch.empty((2, max(steps, 1)), dtype=torch.int32, device=self.device)
-        happy, moves = out[0].view(torch.float32), out[1]
+        table = self._host_keys(steps)
         self.steps_launched = steps
-        if steps > 0 and chunk > 0:
+        if steps == 0:
+            return np.empty(0, np.float32), np.empty(0, np.int32)
+        keys = self._stage.upload(table).view(torch.int32).view(-1, 2)
+        counters = torch.empty((steps, 2), dtype=torch.int32, device=self.device)
+        out = torch.empty((2, steps), dtype=torch.int32, device=self.device)
+        happy, moves = out[0].view(torch.float32), out[1]
+        if chunk > 0:
             if self._watch is None:
                 self._watch = torch.empty(2, dtype=torch.int32, pin_memory=True)
             launched = C.c_int32()
@@ -104,10 +107,10 @@ class SchellingEngine:
                 ptr(happy), ptr(moves), C.c_void_p(self._watch.data_ptr()), C.byref(launched),
                 stream_handle()), "schelling_run")
             self.steps_launched = int(launched.value)
-        elif steps > 0:
+        else:
             self.launch(keys, steps, counters, happy, moves)
         got = out.cpu().numpy()   # both records in one copy
-        return got[0, :steps].view(np.float32), got[1, :steps]
+        return got[0].view(np.float32), got[1]
 
     def run_settling(self, keys, steps, counters, happy, moves, chunk=SETTLE_CHUNK, stream=None,
                      launch=None) -> int:
