@@ -376,7 +376,8 @@ __global__ void __launch_bounds__(kWealthThreads)
     return;
   }
   const abm_wealth_inst in = insts[blockIdx.x];
-  if (!wealth_split_run(in, cap)) return;
+  // without steps there is no row of draws to load ahead
+  if (!wealth_split_run(in, cap) || in.steps <= 0) return;
   for (int32_t k = tid; k < 2 * exchange_words(A, kPacked); k += kWealthThreads) lds_inc[k] = 0;
   __syncthreads();
   exchange_steps<A, kPacked>(in, lds_inc);

@@ -256,3 +256,26 @@ def test_engine_routes_give_the_same_bits(wealth, monkeypatch):
         np.testing.assert_array_equal(u, v)
     for t in ("w", "x", "y"):
         np.testing.assert_array_equal(getattr(a, t).cpu().numpy(), getattr(b, t).cpu().numpy())
+
+
+@pytest.mark.parametrize("n,max_n", [(37, 0), (1000, 1000), (3000, 3000), (40_000, 40_000)])
+def test_batch_instance_of_no_steps(wealth, n, max_n):
+    """An instance of 0 steps has no row of draws: its buffer, here the end of a
+    live one, is not read, and its state and the other instance are untouched."""
+    import torch
+
+    from jaxabm_amd._lib import check, lib, ptr, stream_handle
+
+    idle, a, b = (wealth.WealthEngine(m, seed=6) for m in (n, 50, 50))
+    want = b.run(4)
+    keys, rec, draws = a.key_table(4), torch.empty(2, 4, device="cuda"), a.draw_buffer(4)
+    d0 = idle.descriptor(keys, 0, rec[0], rec[1], draws)
+    d0["draws"] = draws.data_ptr() + 4 * draws.numel()
+    before = [getattr(idle, t).clone() for t in ("x", "y", "w")]
+    table = torch.from_numpy(np.concatenate(
+        [d0, a.descriptor(keys, 4, rec[0], rec[1], draws)]).view(np.uint8)).to("cuda")
+    check(lib().abm_wealth_run_batch(ptr(table), 2, max_n, a.mode, stream_handle()), "run")
+    for t, was in zip(("x", "y", "w"), before):
+        assert torch.equal(getattr(idle, t), was)
+    for got, w in zip(rec.cpu().numpy(), want):
+        np.testing.assert_array_equal(got, w)
