@@ -173,8 +173,8 @@ class _Runner:
         """Write a step's results into the fixed buffers (recorded in the
         graph when called under capture).  A result that shares memory with
         one of the buffers (a variable returned unchanged under another name,
-        an env entry moved to another key) is cloned first, so the order of
-        the copies cannot matter."""
+        an env entry moved to another key, a metric that is one) is cloned
+        first, so the order of the copies cannot matter."""
         pairs = []
         for name, c in self.colls:
             st = self.static[name]
@@ -208,6 +208,13 @@ class _Runner:
                 srcs.append(t.clone())
             else:
                 srcs.append(t)
+        # a metric that is (part of) a buffer written here, as an env slot's
+        # value of before the step, is read before that
+        written = {d.untyped_storage().data_ptr() for (d, _), t in zip(pairs, srcs)
+                   if t is not None}
+        written.update(slot.untyped_storage().data_ptr() for slot, _ in env_fill)
+        metrics = {k: v.clone() if isinstance(v, torch.Tensor) and
+                   v.untyped_storage().data_ptr() in written else v for k, v in metrics.items()}
         # contiguous same-dtype copies and history rows go to one launch
         items, keep = [], []
 

@@ -521,3 +521,31 @@ def test_graph_repeat_rejects_bad_arguments(J):
     for times in (0, -1, 3):
         assert lib().abm_graph_repeat(None, times, C.byref(out)) != 0
     assert out.value is None
+
+
+def test_metric_of_the_env_value_of_the_step_before(J):
+    """A per-agent array kept in the env for one more step, recorded as a
+    metric: its buffer is written by the same commit that copies the row."""
+    import torch
+
+    from jaxabm_amd import numpy as jnp
+
+    def env_fn(env, agents, params, key):
+        return {"prev": env["cur"], "cur": agents["t"]["x"]}
+
+    def metrics(env, agents, params):
+        return {"was": env["prev"], "last": env["prev"][-1], "mean": jnp.mean(env["cur"])}
+
+    runs = []
+    for graph in (False, True):
+        m = make_trader(J, n=50_000, metrics=metrics, env_fn=env_fn)
+        zeros = torch.zeros(50_000, device="cuda")
+        m.add_env_state("prev", zeros.clone())
+        m.add_env_state("cur", zeros.clone())
+        runs.append((m, m.run(9, graph=graph)))
+    (a, ra), (b, rb) = runs
+    assert b.last_run_info["mode"] == "graph"
+    for k in ("was", "last", "mean"):
+        for t, (u, v) in enumerate(zip(ra[k], rb[k])):
+            assert torch.equal(u, v), (k, t)
+    assert not ra["was"][0].any() and ra["was"][1].any()
