@@ -190,11 +190,7 @@ class _Runner:
         # The waiting reductions go out with the copies in one launch, and the
         # copies of their results after them.  On their own before anything
         # else, when there are too many, or one reads a buffer written here.
-        waiting, self.waiting = self.waiting, []
-
-        def launch_waiting():
-            reductions.launch(waiting)
-            waiting.clear()
+        waiting, launch_waiting = self.waiting, self.launch_waiting
 
         if (len(waiting) > REDUCE_BATCH_MAX or
                 any(v.untyped_storage().data_ptr() in dst_storages for _op, v, *_ in waiting)):
@@ -257,9 +253,17 @@ class _Runner:
             check(lib().abm_reduce_commit_step(reductions.items(waiting), len(waiting), arr,
                                                len(early), len(items), *tail),
                   "reduce_commit_step")
+            waiting.clear()
             return
         arr = (CopyItem * max(len(items), 1))(*items)
         check(lib().abm_commit_step(arr, len(items), *tail), "commit_step")
+
+    def launch_waiting(self):
+        """The waiting reductions on their own: before a commit that they cannot
+        wait for, or for a step that is not committed, whose callbacks may have
+        kept a result."""
+        reductions.launch(self.waiting)
+        self.waiting.clear()
 
     def first_step(self):
         """Step 1, eagerly, on the model's own env values and Python time
@@ -392,6 +396,7 @@ def run_graph(model, n: int, between=None) -> Dict[str, Any]:
     try:
         r.first_step()
     except Exception as e:  # noqa: BLE001 - any failure: the plain loop runs instead
+        r.launch_waiting()
         for name, c in r.colls:
             c._states = originals[name]
         return {"mode": "eager", "steps": n, "steps_done": 0,
@@ -399,6 +404,7 @@ def run_graph(model, n: int, between=None) -> Dict[str, Any]:
     try:
         r.second_step()
     except Exception as e:  # noqa: BLE001
+        r.launch_waiting()
         r.finish(1)
         return {"mode": "eager", "steps": n, "steps_done": 1,
                 "reason": f"step 2: {type(e).__name__}: {e}"}

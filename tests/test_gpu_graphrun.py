@@ -549,3 +549,29 @@ def test_metric_of_the_env_value_of_the_step_before(J):
         for t, (u, v) in enumerate(zip(ra[k], rb[k])):
             assert torch.equal(u, v), (k, t)
     assert not ra["was"][0].any() and ra["was"][1].any()
+
+
+@pytest.mark.parametrize("refused", [1, 2])
+def test_results_kept_from_a_step_that_is_not_replayed(J, refused):
+    """Reductions whose results the callbacks keep: step 1 (a metric that is no
+    number) or step 2 (a Python value that changes) runs again eagerly, and what
+    its first run kept is as good."""
+    import torch
+
+    from jaxabm_amd import numpy as jnp
+
+    fill = [torch.full((), float(k), device="cuda") for k in range(-64, 0)]
+    del fill   # blocks that a result not computed would show
+    kept, calls = [], []
+
+    def metrics(env, agents, params):
+        calls.append(1)
+        kept.append(jnp.mean(agents["t"]["x"]))
+        return {"m": kept[-1], "k": "text" if refused == 1 else len(calls)}
+
+    m = make_trader(J, n=5000, metrics=metrics, env_fn=None)
+    hist = m.run(4, graph=True)
+    assert m.last_run_info["mode"] == "eager" and m.last_run_info["steps_done"] == refused - 1
+    values = [float(v) for v in kept]
+    assert values[refused - 1] == values[refused]   # the same step, twice
+    assert [float(v) for v in hist["m"]] == values[:refused - 1] + values[refused:]
