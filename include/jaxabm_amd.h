@@ -260,9 +260,9 @@ int abm_wealth_init(const uint32_t *init_key, int64_t n, float *x, float *y, int
 /* The same from a key in host memory (passed to the kernel by value). */
 int abm_wealth_init_host_key(const uint32_t init_key[2], int64_t n, float *x, float *y, int32_t *w,
                              int mode, void *stream);
-/* Runs every instance of the device array insts[count] for its steps (count
- * <= 65,535).  max_n: the largest n in the table (0 if unknown).  With draws,
- * an instance's draws are computed first by a grid-wide kernel; if n <= max_n
+/* Runs every instance of the device array insts[count] for its steps.  max_n:
+ * the largest n in the table (0 if unknown).  With draws, an instance's draws
+ * are computed first by a grid-wide kernel; if n <= max_n
  * <= 40,000 (or n <= 1,024), one workgroup then runs the exchange out of LDS
  * (leaving each step's wealth in place of its targets in draws) while others
  * walk the positions, and the records of all steps are taken at the end.

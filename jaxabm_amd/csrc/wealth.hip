@@ -777,6 +777,9 @@ const ExchangeVariant kExchange[] = {
     exchange_variant<16, false>(), exchange_variant<20, false>(), exchange_variant<24, true>(),
     exchange_variant<32, true>(),  exchange_variant<40, true>()};
 
+// Instances of a launch that has a grid row for each.
+constexpr int32_t kGridRows = 65535;
+
 // Workgroups of the draws kernel for each of `count` instances.  A draw is a
 // chain of about 900 dependent operations, so a SIMD wants its 8 wavefronts:
 // 2,048 workgroups fill the chip (5,003 x 150: 29 us, 33 with 512); many
@@ -889,7 +892,6 @@ int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t ma
   ABM_REQUIRE(insts && count >= 0 && max_n >= 0 && (mode == 0 || mode == 1),
               "abm_wealth_run_batch: bad arguments");
   if (count == 0) return kOk;
-  ABM_REQUIRE(count <= 65535, "abm_wealth_run_batch: at most 65,535 instances a call");
   if (int rc = wealth_lds_attr()) return rc;
   hipStream_t s = (hipStream_t)stream;
   // the exchange kernel takes instances of up to `cap` agents: the table's
@@ -904,13 +906,17 @@ int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t ma
   const int64_t lds_agents = max_n > 0 && max_n <= kWealthLdsAgents ? max_n : 0;
   size_t dyn = (size_t)(lds_agents * kWealthLdsBytesPerAgent + 4);
   if (dyn < (size_t)(cap + 1) * 4) dyn = (size_t)(cap + 1) * 4;
-  hipLaunchKernelGGL(mode == kModePartitionable ? k_wealth_draws<kModePartitionable>
-                                                : k_wealth_draws<kModeOriginal>,
-                     dim3(draw_blocks(count), (unsigned)count), dim3(kDrawThreads), 0, s, insts);
-  hipLaunchKernelGGL(v->kernel, dim3((unsigned)(count * (1 + per))), dim3(kWealthThreads),
-                     v->lds, s, insts, count, cap);
-  hipLaunchKernelGGL(k_wealth_records, dim3(256u, (unsigned)count), dim3(kWealthThreads), dyn, s,
-                     insts, cap, lds_agents, mode);
+  for (int32_t done = 0; done < count; done += kGridRows) {
+    const abm_wealth_inst *part = insts + done;
+    const int32_t rows = std::min(count - done, kGridRows);
+    hipLaunchKernelGGL(mode == kModePartitionable ? k_wealth_draws<kModePartitionable>
+                                                  : k_wealth_draws<kModeOriginal>,
+                       dim3(draw_blocks(rows), (unsigned)rows), dim3(kDrawThreads), 0, s, part);
+    hipLaunchKernelGGL(v->kernel, dim3((unsigned)(rows * (1 + per))), dim3(kWealthThreads),
+                       v->lds, s, part, rows, cap);
+    hipLaunchKernelGGL(k_wealth_records, dim3(256u, (unsigned)rows), dim3(kWealthThreads), dyn, s,
+                       part, cap, lds_agents, mode);
+  }
   ABM_LAUNCH_CHECK("abm_wealth_run_batch");
   return kOk;
 }

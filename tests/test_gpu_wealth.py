@@ -279,3 +279,34 @@ def test_batch_instance_of_no_steps(wealth, n, max_n):
         assert torch.equal(getattr(idle, t), was)
     for got, w in zip(rec.cpu().numpy(), want):
         np.testing.assert_array_equal(got, w)
+
+
+def test_batch_of_more_instances_than_a_grid_has_rows(wealth):
+    """65,537 instances of one seed: each one's records and state are the
+    engine's."""
+    import torch
+
+    from jaxabm_amd._lib import WEALTH_INST, check, lib, ptr, stream_handle
+
+    B, n, steps = 65_537, 5, 3
+    eng = wealth.WealthEngine(n, seed=8)
+    x, y, w = (t.repeat(B) for t in (eng.x, eng.y, eng.w))
+    inc = torch.zeros(B * n, dtype=torch.int32, device="cuda")
+    hist = torch.zeros(B * (n + 1), dtype=torch.int32, device="cuda")
+    keys = eng.key_table(steps)
+    rec = torch.empty(2, B * steps, device="cuda")
+    draws = torch.empty(B * steps * 3 * n, dtype=torch.int32, device="cuda")
+    d, k = np.zeros(B, WEALTH_INST), np.arange(B, dtype=np.uint64)
+    d["n"], d["steps"], d["keys"] = n, steps, keys.data_ptr()
+    for name, t, each in (("x", x, n), ("y", y, n), ("w", w, n), ("inc", inc, n),
+                          ("hist", hist, n + 1), ("mean_out", rec[0], steps),
+                          ("gini_out", rec[1], steps), ("draws", draws, steps * 3 * n)):
+        d[name] = t.data_ptr() + 4 * each * k
+    table = torch.from_numpy(d.view(np.uint8)).to("cuda")
+    check(lib().abm_wealth_run_batch(ptr(table), B, n, eng.mode, stream_handle()), "run")
+    eng.rng = wealth.WealthEngine(n, seed=8).rng   # key_table moved it on
+    mean, gini = eng.run(steps)
+    for got, want in ((rec[0], mean), (rec[1], gini)):
+        assert torch.equal(got.view(B, steps), torch.from_numpy(want.copy()).cuda().expand(B, steps))
+    for got, want in ((x, eng.x), (y, eng.y), (w, eng.w)):
+        assert torch.equal(got.view(B, n), want.expand(B, n))
