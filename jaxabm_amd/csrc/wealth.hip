@@ -383,15 +383,71 @@ __global__ void __launch_bounds__(kWealthThreads)
   exchange_steps<A, kPacked>(in, lds_inc);
 }
 
+// ---- records of a run whose exchange is done
+//
+// Up to this many agents a wavefront takes a step's record alone, from a
+// histogram of its own: a workgroup a record spends 10 us on barriers with most
+// of its lanes idle, which a batch of small instances pays over and over (256
+// instances of 1,000 agents x 100 steps: 542 us, and 162 for whole runs by a
+// workgroup each).
+constexpr int64_t kWaveRecordAgents = 1024;
+constexpr int kWealthWaves = kWealthThreads / 64;
+constexpr size_t kWaveRecordLds = kWealthWaves * (kWaveRecordAgents + 1) * 4;
+
+// One wavefront records step t from the wealth row; hist: n + 1 bins in LDS,
+// zero on entry and left zero.
+__device__ __forceinline__ void wealth_wave_record(const abm_wealth_inst &in, int32_t t,
+                                                   uint32_t *hist) {
+  constexpr int kLoads = 8;  // in flight
+  const int lane = threadIdx.x & 63;
+  const int32_t n = (int32_t)in.n;
+  const GlobalPtr<const uint32_t> row =
+      as_global<const uint32_t>(in.draws) + (int64_t)t * 3 * n + 2 * n;
+  for (int32_t i0 = lane; i0 - lane < n; i0 += 64 * kLoads) {
+    uint32_t v[kLoads];
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) v[k] = row[min(i0 + 64 * k, n - 1)];
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k)
+      if (i0 + 64 * k < n) atomicAdd(&hist[v[k]], 1u);  // v <= n: wealth is conserved
+  }
+  // LDS operations of a wavefront complete in order; the compiler keeps it
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  uint32_t S = 0, T = 0, counted = 0;
+  for (int32_t b = 0; counted < (uint32_t)n && b <= n; b += 64) {
+    const int32_t w = b + lane;
+    const uint32_t c = w <= n ? hist[w] : 0u;
+    if (c) hist[w] = 0;
+    uint32_t inc = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(inc, off);
+      if (lane >= off) inc += y;
+    }
+    const uint32_t before = counted + inc - c;
+    S += (uint32_t)w * (uint32_t)((uint64_t)c * before + (uint64_t)c * (c + 1) / 2);
+    T += (uint32_t)w * c;
+    counted += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    S += __shfl_xor(S, off);
+    T += __shfl_xor(T, off);
+  }
+  if (lane == 0) wealth_write_record(in, t, T, S);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // LDS limit of the records: n + 1 bins, or the state of kWealthLdsAgents.
 constexpr int64_t kRecordsLds = (kExchangeAgents + 1) * 4;
 static_assert(kRecordsLds >= kWealthLdsAgents * kWealthLdsBytesPerAgent + 4 &&
-                  kRecordsLds + 128 <= 160 * 1024,
+                  kRecordsLds >= (int64_t)kWaveRecordLds && kRecordsLds + 128 <= 160 * 1024,
               "records LDS");
 
 // Workgroup (b, instance): the records of steps b, b + gridDim.x, .. of an
 // instance whose exchange has run, each from a histogram of the step's wealth
-// row in LDS (n + 1 bins).  Workgroup 0 of an instance that the exchange
+// row in LDS (n + 1 bins), a step a wavefront for few agents (the first
+// wavefront of every workgroup first, then the second).  Workgroup 0 of an instance that the exchange
 // kernel did not take runs it whole instead, in LDS where lds_bytes allow.
 __global__ void __launch_bounds__(kWealthThreads)
     k_wealth_records(const abm_wealth_inst *__restrict__ insts, int64_t cap, int64_t lds_agents,
@@ -405,6 +461,14 @@ __global__ void __launch_bounds__(kWealthThreads)
   if (wealth_split_run(in, cap)) {
     int32_t *hist = lds_agents_mem;
     if ((int32_t)blockIdx.x >= in.steps) return;
+    if (n <= kWaveRecordAgents) {
+      const int32_t wave = tid >> 6;
+      uint32_t *mine = reinterpret_cast<uint32_t *>(lds_agents_mem) + wave * (n + 1);
+      for (int32_t b = tid & 63; b <= n; b += 64) mine[b] = 0;
+      for (int32_t t = blockIdx.x + wave * gridDim.x; t < in.steps; t += kWealthWaves * gridDim.x)
+        wealth_wave_record(in, t, mine);
+      return;
+    }
     for (int64_t b = tid; b <= n; b += kWealthThreads) hist[b] = 0;
     __syncthreads();
     for (int32_t t = blockIdx.x; t < in.steps; t += gridDim.x) {
@@ -788,6 +852,13 @@ unsigned draw_blocks(int32_t count) {
   return (unsigned)std::max(512, std::min(2048, 4096 / std::max(count, 1)));
 }
 
+// Workgroups of the records for each of `count` instances: a lone one has its
+// steps on as many CUs, many share a few thousand workgroups (256 for each of
+// 4,096 cost 2.5 ms to launch, most of them without a step).
+unsigned record_blocks(int32_t count) {
+  return (unsigned)std::max(1, std::min(256, 4096 / count));
+}
+
 // These kernels may need more than 64 KB of dynamic LDS: the limits are
 // raised once per device, under a lock.
 constexpr int kMaxDevices = 64;
@@ -906,6 +977,7 @@ int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t ma
   const int64_t lds_agents = max_n > 0 && max_n <= kWealthLdsAgents ? max_n : 0;
   size_t dyn = (size_t)(lds_agents * kWealthLdsBytesPerAgent + 4);
   if (dyn < (size_t)(cap + 1) * 4) dyn = (size_t)(cap + 1) * 4;
+  if (dyn < kWaveRecordLds) dyn = kWaveRecordLds;
   for (int32_t done = 0; done < count; done += kGridRows) {
     const abm_wealth_inst *part = insts + done;
     const int32_t rows = std::min(count - done, kGridRows);
@@ -914,8 +986,8 @@ int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t ma
                        dim3(draw_blocks(rows), (unsigned)rows), dim3(kDrawThreads), 0, s, part);
     hipLaunchKernelGGL(v->kernel, dim3((unsigned)(rows * (1 + per))), dim3(kWealthThreads),
                        v->lds, s, part, rows, cap);
-    hipLaunchKernelGGL(k_wealth_records, dim3(256u, (unsigned)rows), dim3(kWealthThreads), dyn, s,
-                       part, cap, lds_agents, mode);
+    hipLaunchKernelGGL(k_wealth_records, dim3(record_blocks(rows), (unsigned)rows),
+                       dim3(kWealthThreads), dyn, s, part, cap, lds_agents, mode);
   }
   ABM_LAUNCH_CHECK("abm_wealth_run_batch");
   return kOk;

@@ -310,3 +310,19 @@ def test_batch_of_more_instances_than_a_grid_has_rows(wealth):
         assert torch.equal(got.view(B, steps), torch.from_numpy(want.copy()).cuda().expand(B, steps))
     for got, want in ((x, eng.x), (y, eng.y), (w, eng.w)):
         assert torch.equal(got.view(B, n), want.expand(B, n))
+
+
+def test_records_of_a_large_batch_match_oracle(wealth):
+    """Instances around the sizes that a wavefront records alone (64 and 512
+    values a round of loads, 1,024 agents at most), so many that a workgroup and
+    its wavefronts take several steps each."""
+    sizes, steps = [2, 63, 64, 65, 511, 512, 513, 1023, 1024, 1025], 130
+    engines = [wealth.WealthEngine(n, seed=n) for _ in range(60) for n in sizes]
+    records = wealth.run_batch(engines, [steps] * len(engines))
+    for k, n in enumerate(sizes):
+        x, y, w, rng = O.wealth_init(n, n, engines[0].mode)
+        om, og = O.wealth_run(x, y, w, rng, steps, engines[0].mode)
+        for e, (mean, gini) in list(zip(engines, records))[k::len(sizes)]:
+            np.testing.assert_array_equal(mean, om)
+            np.testing.assert_array_equal(gini, og)
+            np.testing.assert_array_equal(e.w.cpu().numpy(), w)
