@@ -28,3 +28,22 @@ def test_sort_pairs_stable_at_tile_edges(n, distinct):
     order = np.argsort(keys, kind="stable")
     np.testing.assert_array_equal(dv.cpu().numpy(), order)
     np.testing.assert_array_equal(dk.cpu().numpy().view(np.uint32), keys[order])
+
+
+# the tiles (of 2,048) where the scan of a segment's counts changes its form
+@pytest.mark.parametrize("tiles", [1, 2, 4, 5, 16, 17, 32, 33])
+@pytest.mark.parametrize("segments", [1, 15, 16])
+@pytest.mark.parametrize("ragged", [0, 1])
+def test_segments_equal_single_permutations(tiles, segments, ragged):
+    import torch
+
+    import oracle as O
+    from jaxabm_amd import random as jr
+
+    n = tiles * 2048 - ragged * 77
+    keys = np.random.default_rng(tiles).integers(0, 1 << 32, (segments, 2), dtype=np.uint64)
+    keys = keys.astype(np.uint32)
+    got = jr.permutation_each(torch.from_numpy(keys.view(np.int32)).cuda(), n, 1).cpu().numpy()
+    for k in {0, segments // 2, segments - 1}:
+        np.testing.assert_array_equal(got[k], O.permutation(keys[k], n, 1))
+    assert (np.sort(got, axis=1) == np.arange(n)).all()
