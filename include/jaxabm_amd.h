@@ -310,7 +310,7 @@ typedef struct abm_schelling_grid {
   int32_t *pos;          /* device [H*W]: cell of agent k (first n_agents) */
   int8_t *type;          /* device [H*W]: type of agent k */
   int32_t *target;       /* device [H*W]: scratch */
-  int32_t *empty;        /* device [H*W], 16-byte aligned: scratch (empty-cell bitmap) */
+  int32_t *empty;        /* device [H*W]: scratch (empty-cell bitmap) */
   int32_t *block_counts; /* device [abm_schelling_block_count(H*W)]: scratch (cells
                             per 1024-cell block: agents at init; empty cells
                             during a run, in 16 copies summed by the readers) */

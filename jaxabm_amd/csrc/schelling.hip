@@ -843,10 +843,10 @@ static int schelling_steps(const abm_schelling_grid *g, const uint32_t *keys, in
   const unsigned nb = nblk(nc, kCellsPerBlock);
   ABM_REQUIRE(nb <= kMaxEmptyBlocks,
               "abm_schelling_run: grids of more than 15,360,000 cells are not supported");
-  // whole blocks of bitmap words fit: 32 * nb <= H*W for any grid not run below
-  uint32_t *ebits = reinterpret_cast<uint32_t *>(g->empty);
-  ABM_REQUIRE(((uintptr_t)ebits & 15u) == 0,
-              "abm_schelling_run: the empty scratch must be 16-byte aligned");
+  // the bitmap's lines are read 16 bytes at a time, so it begins at the first
+  // such boundary of the scratch; whole blocks of words fit from there: 32 * nb + 3
+  // <= H*W for any grid not run below
+  uint32_t *ebits = reinterpret_cast<uint32_t *>(((uintptr_t)g->empty + 15u) & ~(uintptr_t)15u);
   const bool part = mode == kModePartitionable;
   if (schelling_small(g->height, g->width, g->n_agents)) {
     if (int rc = schelling_lds_attr()) return rc;

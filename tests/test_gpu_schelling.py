@@ -211,3 +211,27 @@ def test_schelling_watched_runs(schelling, mode, H, W, steps):
         assert settled <= eng.steps_launched <= min(S, settled + 9)
     else:
         assert eng.steps_launched == S
+
+
+@pytest.mark.parametrize("H,W", [(20, 31), (157, 157), (300, 70)])
+@pytest.mark.parametrize("words", [1, 2, 3])
+def test_empty_scratch_of_any_alignment(schelling, H, W, words):
+    """The bitmap's scratch off a 16-byte boundary: a run and its continuation
+    equal the oracle, and nothing past the scratch is written."""
+    import torch
+
+    eng = schelling.SchellingEngine(H, W, seed=3)
+    scratch = torch.full((words + H * W + 4,), 7, dtype=torch.int32, device="cuda")
+    eng._g.empty = scratch.data_ptr() + 4 * words
+    cells, pos, typ, rng = O.schelling_init(H, W, 3, eng.mode)
+    ohf, omv = O.schelling_run(H, W, cells, pos, typ, rng, 9, eng.mode)
+    keys = eng.key_table(9)
+    counters = torch.empty((9, 2), dtype=torch.int32, device="cuda")
+    happy = torch.empty(9, dtype=torch.float32, device="cuda")
+    moves = torch.empty(9, dtype=torch.int32, device="cuda")
+    eng.launch(keys, 4, counters, happy, moves)
+    eng.launch(keys[4:], 5, counters[4:], happy[4:], moves[4:], prev=counters[3])
+    np.testing.assert_array_equal(moves.cpu().numpy(), omv)
+    np.testing.assert_array_equal(happy.cpu().numpy(), ohf)
+    np.testing.assert_array_equal(eng.positions(), pos)
+    assert (scratch[:words] == 7).all() and (scratch[words + H * W:] == 7).all()
