@@ -811,12 +811,23 @@ void launch_loss(const abm_deffuant_problem *p, const float *x, hipStream_t s) {
                      p->loss, p->coef);
 }
 
+// Above so many agents (three rounds of pairs a step) a column costs more than
+// the step kernels do for a few instances: forward and backward of 60 steps, 1
+// instance of 34,000 agents, 1,303 us in columns and 865 in step kernels; 9 of
+// 30,000, 1,102 and 985; 17 of 30,000, 1,140 and 1,056, but 3,254 and 3,414 with
+// 200 steps.  With 24,576 agents, 1 instance 872 and 840, 17 instances 902 and
+// 982.  A multiple of four instances takes four a lane in the step kernels, and
+// as long as 64: 4 of 40,000, 1,366 and 2,567.
+constexpr int64_t kColFewAgents = 3 * 2 * 4 * kColThreads;
+constexpr int32_t kColFewInstances = 16;
+
 // Whether a flagged descriptor takes the column run; the same answer in the
-// forward and the backward of one descriptor.
+// forward and the backward of one descriptor.  Either way the same opinions,
+// statistics and terms of the gradients, those summed in another order.
 bool column_run(const abm_deffuant_problem *p) {
   if (!(p->flags & ABM_DEFFUANT_COLUMNS) || p->n > kColAgents || p->steps < 1) return false;
   if (p->ckpt_every == 1 ? p->steps < 2 : !p->traj) return false;
-  return true;
+  return !(p->n > kColFewAgents && p->batch <= kColFewInstances && p->batch % 4 != 0);
 }
 
 ColumnRun column_args(const abm_deffuant_problem *p) {

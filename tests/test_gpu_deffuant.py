@@ -301,3 +301,13 @@ def test_forward_is_refused_under_capture(dm):
         with torch.cuda.graph(g):
             m.forward(*args)
     np.testing.assert_array_equal(m.forward(*args).cpu().numpy(), want)
+
+
+# the largest population that few instances run in columns and the next, the
+# most instances that count as few, and multiples of four, which never do
+@pytest.mark.parametrize("n,B,steps,k", [(24576, 2, 5, 2), (24577, 2, 5, 2), (24577, 1, 4, 1),
+                                         (24577, 15, 3, 2), (24577, 17, 3, 2), (24577, 4, 3, 2),
+                                         (40832, 17, 4, 2), (40832, 4, 4, 1)])
+def test_column_run_equals_step_kernels_where_few_instances_leave_it(dm, monkeypatch, n, B, steps,
+                                                                     k):
+    test_column_run_equals_step_kernels(dm, monkeypatch, n, B, steps, k)
