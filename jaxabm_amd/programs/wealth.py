@@ -27,10 +27,13 @@ from ._staging import Staging
 # up to here one workgroup can run a whole simulation out of LDS, whatever the
 # number of steps
 GRID_MIN_AGENTS = 8000
-# up to here the exchange of a run with a draw buffer fits one workgroup's LDS.
-# 100 steps of 8,000 / 20,000 / 40,000 agents: 259 / 437 / 717 us, and 673 /
-# 680 / 732 us spread over the GPU, where a step costs a launch
-EXCHANGE_MAX_AGENTS = 40_000
+# up to here one workgroup runs the exchange of a run with a draw buffer faster
+# than steps spread over the GPU, which cost a launch each: the largest number
+# of agents that takes 32 a thread.  Spread / one workgroup, us, at 10, 100 and
+# 1,500 steps: 16,000 agents 149 / 105, 626 / 295, 8,314 / 3,661; 32,000 agents
+# 159 / 134, 635 / 516, 8,368 / 7,648; 36,000 agents (40 a thread) 147 / 148,
+# 626 / 628, 8,293 / 9,362
+EXCHANGE_MAX_AGENTS = 32_768
 # largest draw buffer a run above GRID_MIN_AGENTS takes for that
 DRAW_BUFFER_MAX_BYTES = 1 << 30
 

@@ -326,3 +326,18 @@ def test_records_of_a_large_batch_match_oracle(wealth):
             np.testing.assert_array_equal(mean, om)
             np.testing.assert_array_equal(gini, og)
             np.testing.assert_array_equal(e.w.cpu().numpy(), w)
+
+
+@pytest.mark.parametrize("n", [32_768, 32_769])
+def test_engine_on_both_sides_of_the_exchange_limit(wealth, n):
+    """The largest engine that runs its exchange in one workgroup (32 agents a
+    thread), and the first that spreads its steps over the GPU."""
+    eng = wealth.WealthEngine(n, seed=5)
+    assert (n > wealth.EXCHANGE_MAX_AGENTS) == (n == 32_769)
+    mean, gini = eng.run(7)
+    x, y, w, rng = O.wealth_init(n, 5, eng.mode)
+    om, og = O.wealth_run(x, y, w, rng, 7, eng.mode)
+    np.testing.assert_array_equal(mean, om)
+    np.testing.assert_array_equal(gini, og)
+    for a, b in ((eng.w, w), (eng.x, x), (eng.y, y)):
+        np.testing.assert_array_equal(a.cpu().numpy(), b)
