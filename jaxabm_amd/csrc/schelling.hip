@@ -872,6 +872,7 @@ static int schelling_steps(const abm_schelling_grid *g, const uint32_t *keys, in
     ABM_LAUNCH_CHECK(what);
     return kOk;
   }
+  if (steps <= 2 * kWatchEvery) watch = nullptr;  // too short to stop: no step tells
   if (watch) clear_watch(watch);
   hipLaunchKernelGGL(k_fill_i32_s, dim3(nblk(2 * (int64_t)steps, 256)), dim3(256), 0, s,
                      counters, 2 * (int64_t)steps, 0);

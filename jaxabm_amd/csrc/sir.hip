@@ -787,6 +787,9 @@ int sir_run(const char *who, const abm_sir_graph *g, uint8_t *state, uint16_t *m
   const uint32_t tb = unit_threshold(beta), tg = unit_threshold(gamma);
   const int64_t words = bitmap_words(g->n);
   const int64_t ns = (int64_t)steps * kStride;
+  // too short to stop: no step tells (4 steps after the last infection: 66 us
+  // with the stores, 62 without)
+  if (steps <= 2 * kWatchEvery) watch = nullptr;
   if (watch) clear_watch(watch);
   hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for(ns, 256)), dim3(256), 0, s,
                      slots, ns, 0);
