@@ -41,11 +41,11 @@
 #include <mutex>
 
 #include "common.hpp"
+#include "deffuant_gate.hpp"
 #include "jaxabm_amd.h"
 
 namespace abm {
 
-constexpr float kGateScale = 0.02f;
 constexpr int kDefThreads = 256;
 constexpr int kDefWaves = kDefThreads / 64;
 // most row chunks of the statistics: two wavefronts per SIMD at 256 columns,
@@ -77,54 +77,18 @@ __device__ __forceinline__ void store_cols(float *p, const float (&v)[VEC]) {
   }
 }
 
-__device__ __forceinline__ float gate(float eps, float d) {
-  const float z = (eps - fabsf(d)) / kGateScale;
-  const float e = abm_expf(-z);
-  const float den = 1.0f + e;
-  return 1.0f / den;
-}
-
-// x / kGateScale rounded once, in three operations: with y = 50 the rounded
-// reciprocal, q + (x - q c) y corrects q = x y to the rounded quotient
-// (Markstein, IBM J. Res. Dev. 34(1), 1990).  Equal to the IEEE division for
-// every float32 of [2^-60, 1.6] (all tested); below, the gate is 1 / 2 either
-// way.  As exact on 2^-87 <= x, where the remainder is a float32.
-__device__ __forceinline__ float div_gate_scale(float x) {
-  const float q = x * 50.0f;
-  return fmaf(fmaf(-q, kGateScale, x), 50.0f, q);
-}
-
-// 1 / d rounded once for 1 <= d < 2^120: the hardware estimate (1 ulp) and two
-// corrections (the second exact, Markstein as above).
-__device__ __forceinline__ float inv_rounded(float d) {
-  float r = __builtin_amdgcn_rcpf(d);
-  r = fmaf(fmaf(-d, r, 1.0f), r, r);
-  return fmaf(fmaf(-d, r, 1.0f), r, r);
-}
-
-// The gates of P differences, the same bits as gate(): its quotients
-// by div_gate_scale and inv_rounded, and abm_expf without its range branches,
-// for |eps - |d|| <= 1.2 (|z| <= 60); any other argument of the wavefront, NaN
-// included, sends it through gate().  34 operations a gate instead of about 58.
-// eps(u): the bound of difference u.
+// The gates of P differences, the same bits as gate(): the short form, 34
+// operations a gate instead of about 58, unless an argument of the wavefront is
+// outside its range or NaN.  eps(u): the bound of difference u.
 template <int P, class Eps>
 __device__ __forceinline__ void gates(Eps eps, const float (&d)[P], float (&g)[P]) {
   bool odd = false;
 #pragma unroll
   for (int u = 0; u < P; ++u) {
     const float num = eps(u) - fabsf(d[u]);
-    odd |= !(fabsf(num) <= 1.2f);
-    const float x = -div_gate_scale(num);
-    const float m = __builtin_rintf(x * 0x1.715476p0f);
-    const float r = (x - m * 0x1.62e4p-1f) - m * 0x1.7f7d1cp-20f;
-    float q = 0x1.a01a02p-13f;
-    q = 0x1.6c16c2p-10f + q * r;
-    q = 0x1.111112p-7f + q * r;
-    q = 0x1.555556p-5f + q * r;
-    q = 0x1.555556p-3f + q * r;
-    q = 0.5f + q * r;
-    const float p = 1.0f + (r + (r * r) * q);
-    g[u] = inv_rounded(1.0f + __builtin_ldexpf(p, (int)m));  // exact: no subnormal here
+    odd |= !(fabsf(num) <= kGateShort);
+    // within 1 ulp, and rounded where inv_rounded asks for it
+    g[u] = gate_short(num, [](float x) { return __builtin_amdgcn_rcpf(x); });
   }
   if (__ballot(odd)) {
 #pragma unroll

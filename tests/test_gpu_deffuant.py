@@ -311,3 +311,50 @@ def test_forward_is_refused_under_capture(dm):
 def test_column_run_equals_step_kernels_where_few_instances_leave_it(dm, monkeypatch, n, B, steps,
                                                                      k):
     test_column_run_equals_step_kernels(dm, monkeypatch, n, B, steps, k)
+
+
+@pytest.mark.parametrize("beyond", [False, True])
+@pytest.mark.parametrize("odd", [0, 1])
+def test_step_kernel_gates_have_the_bits_of_ieee_operations(dm, beyond, odd):
+    """One pair an instance, x_a = 0 and x_c = d a power of two, mu = 1, so that
+    the step gives g d exactly, with eps - d exactly the argument: over the short
+    form's range, where 1 + exp(-z) has all mantissa bits set (the reciprocal's
+    hardest divisor), at its end, and (beyond) mixed with arguments past it,
+    infinities and NaN."""
+    import torch
+
+    from jaxabm_amd._lib import check, lib, ptr, stream_handle
+
+    rs = np.random.default_rng(4)
+    f32 = np.float32
+    num = np.concatenate([
+        rs.uniform(-1.2, 1.2, 1 << 20), np.exp(rs.uniform(np.log(1e-20), np.log(1.2), 1 << 20)),
+        -np.exp(rs.uniform(np.log(1e-20), np.log(1.2), 1 << 20)),
+        np.linspace(1.7e-9, 5.7e-9, 1 << 18),   # 1 + exp(-z) = 0x1.fffffep+0 for most
+        [float.fromhex("-0x1.3ed162p-5"), float.fromhex("-0x1.194feep-4"), 1.2, -1.2]]).astype(f32)
+    num = num[np.abs(num) <= f32(1.2)]
+    if beyond:
+        num[::7] = rs.uniform(-3.0, 3.0, len(num[::7])).astype(f32)
+        num[5::64] = np.nextafter(f32(1.2), f32(2))
+        num[11::640] = [np.inf, -np.inf, np.nan, 100.0, -100.0][0]
+        num[12::640], num[13::640], num[14::640] = -np.inf, np.nan, -2.0
+    num = num[: len(num) // 4 * 4 - odd]
+    k = np.frexp(np.where(np.isfinite(num), num, f32(1)))[1]   # |num| in [2^(k-1), 2^k)
+    d = np.where(num > 0, np.ldexp(f32(1), k - 24), np.ldexp(f32(1), k)).astype(f32)
+    eps = (num + d).astype(f32)
+    fin = np.isfinite(num)
+    assert (eps - d == num)[fin].all()
+    B = len(num)
+    x = torch.from_numpy(np.stack([np.zeros(B, f32), d])).cuda()
+    perm = torch.arange(2, dtype=torch.int32, device="cuda")
+    mu = torch.ones(B, device="cuda")
+    e = torch.from_numpy(eps).cuda()
+    check(lib().abm_deffuant_step(ptr(x), ptr(x), 2, B, ptr(perm), ptr(e), ptr(mu), 1,
+                                  stream_handle()), "step")
+    with np.errstate(all="ignore"):
+        z = (eps - d) / f32(0.02)
+        want = (f32(1) / (f32(1) + O.math_f32("exp", -z))) * d
+    got = x[0].cpu().numpy()
+    bad = np.flatnonzero(~((got == want) | (np.isnan(got) & np.isnan(want))))
+    assert len(bad) == 0, [(float(num[i]).hex(), float(got[i] / d[i]).hex(),
+                            float(want[i] / d[i]).hex()) for i in bad[:5]] + [len(bad)]
