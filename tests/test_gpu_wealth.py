@@ -73,7 +73,8 @@ def _run_raw(wealth, eng, steps, max_n, draws=False):
                                      (300, 100)])
 def test_wealth_lds_and_global_paths_agree(wealth, n, max_n, draws):
     """Every path gives identical records and state: draws computed in the
-    run or grid-wide before it; small instances with state in registers;
+    run or grid-wide before it; with a draw buffer, the exchange apart from walk
+    and records, or the whole instance in one workgroup above the table's limit;
     LDS-resident runs (n <= max_n <= 8000) and global-buffer runs (max_n = 0,
     or an instance above max_n)."""
     steps = 40
@@ -88,11 +89,12 @@ def test_wealth_lds_and_global_paths_agree(wealth, n, max_n, draws):
 
 
 def test_wealth_global_path_matches_oracle(wealth):
-    """An instance above the LDS capacity runs on its global buffers."""
+    """An instance above the LDS capacity, without a draw buffer, runs on its
+    global buffers."""
     n, steps = 9000, 8
     eng = wealth.WealthEngine(n, seed=11)
     x, y, w, rng = O.wealth_init(n, 11, eng.mode)
-    mean, gini = eng.run(steps)
+    mean, gini = _run_raw(wealth, eng, steps, n)
     om, og = O.wealth_run(x, y, w, rng, steps, eng.mode)
     np.testing.assert_array_equal(eng.w.cpu().numpy(), w)
     np.testing.assert_array_equal(mean, om)
@@ -100,12 +102,13 @@ def test_wealth_global_path_matches_oracle(wealth):
 
 
 @pytest.mark.parametrize("n,steps,seed", [(8001, 30, 1), (50_000, 40, 2), (300_000, 12, 3)])
-def test_grid_path_matches_oracle_and_one_workgroup_run(wealth, n, steps, seed):
-    """Above 8,000 agents WealthEngine.run spreads each step over the GPU
-    (abm_wealth_run_grid): the oracle's records and state, and the same bits
-    as the one-workgroup run of the batch entry point on global buffers."""
+def test_grid_path_matches_oracle_and_one_workgroup_run(wealth, monkeypatch, n, steps, seed):
+    """WealthEngine.run with each step spread over the GPU (abm_wealth_run_grid),
+    from the smallest size that may take it: the oracle's records and state, and
+    the same bits as the one-workgroup run of the batch entry point."""
     import os
 
+    monkeypatch.setattr(wealth, "EXCHANGE_MAX_AGENTS", wealth.GRID_MIN_AGENTS)
     eng = wealth.WealthEngine(n, seed=seed)
     assert n > wealth.GRID_MIN_AGENTS
     mean, gini = eng.run(steps)
@@ -123,7 +126,7 @@ def test_grid_path_matches_oracle_and_one_workgroup_run(wealth, n, steps, seed):
     np.testing.assert_array_equal(g2, gini)
 
 
-def test_grid_path_wealth_above_the_lds_bins(wealth):
+def test_grid_path_wealth_above_the_lds_bins(wealth, monkeypatch):
     """A state where one agent holds 5,000 units (total wealth 15,000 <= n,
     the histogram's range): wealth values past the grid path's per-workgroup
     LDS bins go to the global histogram directly; the records and state equal
@@ -133,6 +136,7 @@ def test_grid_path_wealth_above_the_lds_bins(wealth):
     import torch
 
     n, steps, seed = 20_000, 25, 5
+    monkeypatch.setattr(wealth, "EXCHANGE_MAX_AGENTS", wealth.GRID_MIN_AGENTS)
     eng = wealth.WealthEngine(n, seed=seed)
     x, y, w, rng = O.wealth_init(n, seed, O.MODE_PARTITIONABLE)
     w[:] = 0
