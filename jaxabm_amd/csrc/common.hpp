@@ -34,6 +34,15 @@ __device__ __forceinline__ T *in_global(T *p) {
   return (T *)g;
 }
 
+// Workgroup barrier that orders LDS only: for exchanges through LDS, where the
+// global stores in flight (and loads issued ahead) need not have arrived, which
+// __syncthreads() would wait for.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Integer threshold for `uniform < p` on [0,1): with m = bits >> 9,
 // u = m * 2^-23 exactly, so u < p  <=>  m < ceil(p * 2^23) (p in (0, 1]).
 // Computed on the host in double: exact for float p.

@@ -285,8 +285,8 @@ __device__ __forceinline__ double inv_one_plus(double t) {
 // sigmoid(128 (x - k/32)) = 1 / (1 + t e^(4k)) with t = e^(-128 x).
 // A workgroup is `cols` columns (a power of two, up to its threads) by
 // kDefThreads / cols chunks, so that a small batch fills its lanes too.  What
-// a chunk is and how the chunks are summed depends on n alone: an instance's
-// statistics do not depend on the batch it runs in.  Bound by the 33
+// a chunk is and how the chunks are summed depends on n and the caller's number
+// of chunks alone, not on the batch an instance runs in.  Bound by the 33
 // reciprocals an opinion (float64 VALU).
 __global__ void __launch_bounds__(kDefThreads)
     k_deffuant_stats(const float *__restrict__ x, int64_t n, int32_t B, int32_t cols,
@@ -459,13 +459,6 @@ __device__ __forceinline__ int32_t column_of(int32_t blk, int32_t B) {
   return base + 256 <= B ? base + (r & 7) * 32 + (r >> 3) : blk;
 }
 
-__device__ __forceinline__ void column_barrier() {
-  // orders LDS only: the tape and the next pairings may stay in flight
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Accesses below go through raw buffers of one row: a pair past the end loads
 // pair (0, 0) and stores nothing, without a branch around the access (which
 // would make every later wait a full one).
@@ -542,7 +535,7 @@ __device__ __forceinline__ void column_steps(const ColumnRun &a, float *x, int32
       }
       pr = nx;
     }
-    column_barrier();
+    lds_barrier();
     after(t);
   }
 }
@@ -559,7 +552,7 @@ __global__ void __launch_bounds__(kColThreads) k_deffuant_column_forward(ColumnR
   const int32_t b = column_of(blockIdx.x, a.B), tid = threadIdx.x, T = col_threads<P>();
   const int64_t nB = (int64_t)a.n * a.B, half = a.n >> 1;
   for (int32_t i = tid; i < a.n; i += T) col_x[i] = a.ckpt[(int64_t)i * a.B + b];
-  column_barrier();
+  lds_barrier();
   const int32_t t_last = (a.steps - 1) / a.k * a.k;
   int32_t next = a.k;  // steps done at the next checkpoint
   auto tape = [&](int32_t t) -> float * {
@@ -571,7 +564,7 @@ __global__ void __launch_bounds__(kColThreads) k_deffuant_column_forward(ColumnR
     float *c = a.ckpt + (int64_t)((t + 1) / a.k) * nB + (int64_t)b * a.n;
     for (int32_t i = tid; i < a.n; i += T) c[i] = col_x[i];
     next += a.k;
-    column_barrier();  // before the next step writes
+    lds_barrier();  // before the next step writes
   };
   column_steps<P>(a, col_x, 0, a.steps, a.eps[b], a.mu[b], tape, after);
   for (int32_t i = tid; i < a.n; i += T) a.work[(int64_t)i * a.B + b] = col_x[i];
@@ -624,7 +617,7 @@ __device__ __forceinline__ void column_sweep(const ColumnRun &a, float *l, int32
       }
       pr = nx;
     }
-    column_barrier();
+    lds_barrier();
   }
 }
 
@@ -656,12 +649,12 @@ __global__ void __launch_bounds__(kColThreads) k_deffuant_column_backward(Column
         const float *c = a.ckpt + j * nB + (int64_t)b * a.n;
         for (int32_t i = tid; i < a.n; i += T) x[i] = c[i];
       }
-      column_barrier();
+      lds_barrier();
       column_steps<P>(a, x, t0, t1, eps, mu, tape, [](int32_t) {});
     }
     if (!kBoth || j == nseg - 1) {
       for (int32_t i = tid; i < a.n; i += T) l[i] = column[i];
-      column_barrier();
+      lds_barrier();
     }
     column_sweep<P>(a, l, t0, t1, eps, mu, tape, ge, gm);
     if (!kBoth && j > 0) {

@@ -97,21 +97,10 @@ struct SirStep {
   const int32_t *prev2_slots; // the step before that, or null
   const uint32_t *keys;
   uint32_t thr_beta, thr_gamma;
-  int mode;
   int32_t *slots;
   int32_t *watch;  // host memory, or null: [0] steps begun, [1] 1 once one was the identity
   int32_t begun;   // value for watch[0], or 0: this step does not tell
 };
-
-// Workgroup barrier that orders LDS only.  Every intra-block exchange in the
-// step kernel goes through LDS (state, marks and bitmaps are never read back
-// by another thread of the block in the same step), so the barrier need not
-// wait for outstanding global stores the way __syncthreads() does.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 __device__ __forceinline__ bool infected(const uint32_t *__restrict__ bm, int32_t u) {
   return (bm[u >> 5] >> (u & 31)) & 1u;
@@ -351,6 +340,9 @@ __device__ __forceinline__ void scan_items(const SirStep &a, const uint32_t *__r
   }
 }
 
+// Every exchange between the threads of a block goes through LDS (state, marks
+// and bitmaps are never read back by another thread of the block in the same
+// step), so its barriers are lds_barrier().
 template <bool kLds, int kMode>
 __global__ void __launch_bounds__(kSirThreads) k_sir_step(SirStep a) {
   extern __shared__ uint4 lds_bm4[];  // kLds: the bitmap words
@@ -739,11 +731,10 @@ int launch_step(const abm_sir_graph *g, uint8_t *state, uint16_t *mark,
   a.keys = keys4;
   a.thr_beta = tb;
   a.thr_gamma = tg;
-  a.mode = mode;
   a.slots = slots;
   const unsigned blocks = (unsigned)(g->n_chunks < kSirBlocks ? g->n_chunks : kSirBlocks);
   // one instantiation per stream layout: each carries one copy of the draw
-  const bool part = a.mode == kModePartitionable;
+  const bool part = mode == kModePartitionable;
   if (a.words <= kLdsBitmapWords) {
     auto *kp = k_sir_step<true, kModePartitionable>;
     auto *ko = k_sir_step<true, kModeOriginal>;

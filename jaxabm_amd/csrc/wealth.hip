@@ -1,5 +1,5 @@
-// wealth.hip -- wealth-exchange random walk: one workgroup runs a whole
-// simulation of one instance; a launch runs a batch of instances.
+// wealth.hip -- wealth-exchange random walk: batches of instances, and one large
+// instance over the whole GPU.
 //
 // Program (reference API, jaxabm/model.py:118-216, jaxabm/agent.py:92-177):
 //  init   agent keys = split(init_key, n); kx, ky = split(agent_key);
@@ -233,14 +233,6 @@ __host__ __device__ inline bool wealth_split_run(const abm_wealth_inst &in, int6
   return in.draws != nullptr && in.n <= cap;
 }
 
-// Barrier that orders LDS only: what a step reads back goes through LDS, so
-// the wealth rows in flight to memory need not have arrived.
-__device__ __forceinline__ void wealth_lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Words of one increment array: every thread's A agents, or pairs of them.
 constexpr int32_t exchange_words(int A, bool packed) {
   return A * kWealthThreads / (packed ? 2 : 1);
@@ -312,7 +304,7 @@ __device__ __forceinline__ void exchange_steps(const abm_wealth_inst &in, uint32
       const RowBuffer next = row_buffer(targets + (t + P < steps ? t + P : steps - 1) * row, n);
 #pragma unroll
       for (int a = 0; a < A; ++a) target[p][a] = load(next, a);
-      wealth_lds_barrier();
+      lds_barrier();  // what a step reads back goes through LDS
       const RowBuffer now = row_buffer(targets + t * row, n);
 #pragma unroll
       for (int a = 0; a < A; ++a) {
@@ -514,18 +506,19 @@ __global__ void __launch_bounds__(kWealthThreads)
   }
 }
 
-// ---- one large instance across the whole GPU (abm_wealth_run_grid): two
-// launches per step.  K1(t): every workgroup draws step t for its agents and
-// applies the draws (positions; one exchange atomic per giving agent), and
-// workgroup 0 first records step t-1 from the histogram.  K2(t): the
-// exchange is applied and the wealth histogram built.  Wealth stays bunched
-// on a few small values, so the histogram is gathered without hot words:
-// per-workgroup LDS bins, flushed with one atomic per bin in use, the
-// values below kGridHot into one of kGridCopies copies (chosen by workgroup)
-// and the rest into the instance's histogram.  The total T is conserved, so
-// it is summed once, at step 0; the record stops once it has counted all n
-// agents, so no running maximum is kept.  The same integer and IEEE float
-// operations as the one-workgroup run, so the same bits.
+// ---- one large instance across the whole GPU (abm_wealth_run_grid): one launch
+// per step with scratch for second copies (k_wealth_grid_step, below), two
+// without.  K1(t): every workgroup draws step t for its agents and applies the
+// draws (positions; one exchange atomic per giving agent), and workgroup 0 first
+// records step t-1 from the histogram.  K2(t): the exchange is applied and the
+// wealth histogram built.  Either way wealth stays bunched on a few small values,
+// so the histogram is gathered without hot words: per-workgroup LDS bins, flushed
+// with one atomic per bin in use, the values below kGridHot into one of
+// kGridCopies copies (chosen by workgroup) and the rest into the instance's
+// histogram.  The total T is conserved, so it is summed once, at step 0; the
+// record stops once it has counted all n agents, so no running maximum is kept.
+// The same integer and IEEE float operations as the one-workgroup run, so the
+// same bits.
 constexpr int kGridThreads = 256;
 constexpr int kGridBins = 1024;     // LDS histogram bins per workgroup
 constexpr int64_t kGridMaxBlocks = 1024;
@@ -539,19 +532,14 @@ constexpr int kGridCopies = 16;
 static_assert(ABM_WEALTH_GRID_ACC_WORDS == 2 + kGridCopies * kGridHot,
               "acc layout: T, a spare word, then the hot-bin copies");
 
-// Mean and Gini of step t from the histogram and the total; clears the bins
-// it reads (one workgroup).  Bins are read 256 a round until all n agents
-// are counted, which covers every nonzero bin.
-__device__ void wealth_grid_record(const abm_wealth_inst &in, int32_t t, uint32_t *acc,
-                                   uint32_t *red) {
+// Mean and Gini of step t from a histogram set and the total; clears the bins it
+// reads (one workgroup).  Bins are read 256 a round until all n agents are
+// counted, which covers every nonzero bin.
+__device__ void wealth_grid_rank(const abm_wealth_inst &in, int32_t t, uint32_t T, uint32_t *hot,
+                                 uint32_t *hist, uint32_t *red) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t n = in.n;
-  const uint32_t T = acc[0];
-  uint32_t *hot = acc + 2;
-  __shared__ uint32_t carry;
-  if (tid == 0) carry = 0;
-  __syncthreads();
-  uint32_t S_part = 0;
+  uint32_t S_part = 0, counted = 0;
   for (int64_t base = 0; base <= n; base += kGridThreads) {
     const int64_t w = base + tid;
     uint32_t c = 0;
@@ -565,8 +553,8 @@ __device__ void wealth_grid_record(const abm_wealth_inst &in, int32_t t, uint32_
         if (v[k]) hot[k * kGridHot + w] = 0;
       }
     } else if (w <= n) {
-      c = (uint32_t)in.hist[w];
-      if (c) in.hist[w] = 0;
+      c = hist[w];
+      if (c) hist[w] = 0;
     }
     uint32_t inc = c;
 #pragma unroll
@@ -576,38 +564,27 @@ __device__ void wealth_grid_record(const abm_wealth_inst &in, int32_t t, uint32_
     }
     if (lane == 63) red[wave] = inc;
     __syncthreads();
-    uint32_t wave_off = 0;
-    for (int q = 0; q < wave; ++q) wave_off += red[q];
-    const uint32_t before = carry + wave_off + inc - c;
+    uint32_t before = counted + inc - c;
+    for (int q = 0; q < kGridThreads / 64; ++q) {
+      if (q < wave) before += red[q];
+      counted += red[q];
+    }
     if (c) {
       const uint64_t ranksum = (uint64_t)c * before + (uint64_t)c * (c + 1) / 2;
       S_part += (uint32_t)w * (uint32_t)ranksum;
     }
-    __syncthreads();
-    if (tid == kGridThreads - 1) carry = before + c;
-    __syncthreads();
-    if ((int64_t)carry >= n) break;  // block-uniform
+    __syncthreads();  // red is rewritten
+    if ((int64_t)counted >= n) break;  // block-uniform
   }
   const uint32_t S = block_sum_u32(S_part, red);
-  if (tid == 0) {
-    in.mean_out[t] = (float)(int32_t)T / (float)n;
-    const int32_t Ti = (int32_t)T;
-    float g = 0.0f;
-    if ((float)Ti > 1e-6f) {
-      const int32_t num = (int32_t)(2u * S);
-      const int32_t den = (int32_t)((uint32_t)n * T);
-      const float q = (float)num / (float)den;
-      const float cst = (float)((double)(n + 1) / (double)n);
-      g = q - cst;
-    }
-    in.gini_out[t] = g;
-  }
+  if (tid == 0) wealth_write_record(in, t, T, S);
 }
 
 __global__ void __launch_bounds__(kGridThreads)
     k_wealth_grid_agents(abm_wealth_inst in, int32_t t, uint32_t *acc, int mode) {
   __shared__ uint32_t red[kGridThreads / 64];
-  if (blockIdx.x == 0 && t > 0) wealth_grid_record(in, t - 1, acc, red);
+  if (blockIdx.x == 0 && t > 0)
+    wealth_grid_rank(in, t - 1, acc[0], acc + 2, (uint32_t *)in.hist, red);
   if (t >= in.steps) return;
   const int64_t n = in.n;
   const int64_t stride = (int64_t)gridDim.x * kGridThreads;
@@ -689,52 +666,6 @@ __device__ __forceinline__ void wealth_shared_keys(const abm_wealth_inst &in, ui
   out[1] = kk1.k1;
   out[2] = kk2.k0;
   out[3] = kk2.k1;
-}
-
-// Mean and Gini of step t from a histogram set; clears the bins it reads.
-__device__ void wealth_grid_rank(const abm_wealth_inst &in, int32_t t, uint32_t T, uint32_t *hot,
-                                 uint32_t *hist, uint32_t *red) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t n = in.n;
-  uint32_t S_part = 0, counted = 0;
-  for (int64_t base = 0; base <= n; base += kGridThreads) {
-    const int64_t w = base + tid;
-    uint32_t c = 0;
-    if (w < kGridHot) {
-      uint32_t v[kGridCopies];
-#pragma unroll
-      for (int k = 0; k < kGridCopies; ++k) v[k] = hot[k * kGridHot + w];
-#pragma unroll
-      for (int k = 0; k < kGridCopies; ++k) {
-        c += v[k];
-        if (v[k]) hot[k * kGridHot + w] = 0;
-      }
-    } else if (w <= n) {
-      c = hist[w];
-      if (c) hist[w] = 0;
-    }
-    uint32_t inc = c;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t y = __shfl_up(inc, off);
-      if (lane >= off) inc += y;
-    }
-    if (lane == 63) red[wave] = inc;
-    __syncthreads();
-    uint32_t before = counted + inc - c;
-    for (int q = 0; q < kGridThreads / 64; ++q) {
-      if (q < wave) before += red[q];
-      counted += red[q];
-    }
-    if (c) {
-      const uint64_t ranksum = (uint64_t)c * before + (uint64_t)c * (c + 1) / 2;
-      S_part += (uint32_t)w * (uint32_t)ranksum;
-    }
-    __syncthreads();  // red is rewritten
-    if ((int64_t)counted >= n) break;  // block-uniform
-  }
-  const uint32_t S = block_sum_u32(S_part, red);
-  if (tid == 0) wealth_write_record(in, t, T, S);
 }
 
 template <int kMode>

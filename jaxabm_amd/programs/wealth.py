@@ -1,5 +1,4 @@
-"""Wealth-exchange random walk on the HIP engine (one workgroup per instance,
-whole run in one launch).
+"""Wealth-exchange random walk on the HIP engine: single instances and batches.
 
 Program (written against the reference API, jaxabm/model.py:118-216,
 jaxabm/agent.py:92-177; Gini after examples/models/advanced_economic_model.py:
@@ -121,8 +120,8 @@ class WealthEngine:
 
 
 def run_batch(engines: list[WealthEngine], steps: list[int], stream=None):
-    """Run several instances in one launch (one workgroup each); returns a list
-    of (mean, gini) host arrays."""
+    """Run several instances together (abm_wealth_run_batch); returns a list of
+    (mean, gini) host arrays."""
     if not engines:
         return []
     mode = engines[0].mode
