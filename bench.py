@@ -400,7 +400,7 @@ def _trader_cpu(n, steps, runs):
 
 def bench_wealth(args) -> dict:
     """Wealth exchange, 1,000 agents, 100 steps, seed 0: one bench step = one
-    whole simulation (state init + one single-workgroup launch)."""
+    whole simulation (state init, then draws, exchange and records)."""
     import numpy as np
     import torch
 
@@ -546,8 +546,8 @@ def bench_generic(args) -> dict:
 def bench_schelling(args) -> dict:
     """Schelling, 512 x 512 torus, 200 steps: one bench step = one whole
     simulation from the seeded grid (the seeded grid, agent ids and positions
-    restored by device copies, then the 200 steps), replayed as one hipGraph
-    like the SIR line."""
+    restored by device copies, then SchellingEngine.run), and the same steps
+    replayed as one hipGraph like the SIR line."""
     import numpy as np
     import torch
 
@@ -559,6 +559,7 @@ def bench_schelling(args) -> dict:
     stream = torch.cuda.Stream()
     with torch.cuda.stream(stream):
         eng = SchellingEngine(H, W, seed=0)
+        rng0 = eng.rng.copy()
         keys = eng.key_table(S)
         counters = torch.empty((S, 2), dtype=torch.int32, device="cuda")
         happy = torch.empty(S, dtype=torch.float32, device="cuda")
@@ -592,40 +593,21 @@ def bench_schelling(args) -> dict:
                 np.array_equal(moves.cpu().numpy(), ref[1]))
     check(lib().abm_graph_destroy(g), "graph_destroy")
 
-    # the measured run: launches of 16 steps, each replayed as its own graph
-    # (the state restore in the first), stopped once the grid has settled
-    chunk = SchellingEngine.SETTLE_CHUNK
-    graphs = []
-    for s0 in range(0, S, chunk):
-        s1 = min(s0 + chunk, S)
-        gi = C.c_void_p()
-        check(lib().abm_graph_begin(sh), "graph_begin")
-        if s0 == 0:
-            for k, t0 in init.items():
-                check(lib().abm_memcpy_d2d(ptr(getattr(eng, k)), ptr(t0),
-                                           C.c_size_t(t0.numel() * t0.element_size()), sh),
-                      "reset")
-        eng.launch(keys[s0:], s1 - s0, counters[s0:], happy[s0:], moves[s0:], stream=stream,
-                   prev=counters[s0 - 1] if s0 else None)
-        check(lib().abm_graph_end(sh, C.byref(gi)), "graph_end")
-        graphs.append(gi)
-    launched = []
+    # the measured run: the engine's own, which launches ahead of the GPU until
+    # the grid has settled and reads the records back
+    got = []
 
     def run():
-        launched.append(eng.run_settling(
-            keys, S, counters, happy, moves, chunk, stream,
-            launch=lambda i, s0, s1: check(lib().abm_graph_launch(graphs[i], sh), "graph_launch")))
+        with torch.cuda.stream(stream):
+            for k, t in init.items():
+                getattr(eng, k).copy_(t)
+            eng.rng = rng0.copy()
+            got[:] = eng.run(S)
 
-    with torch.cuda.stream(stream):
-        happy.fill_(-1.0)   # the measured runs must write every record again
-        moves.fill_(-1)
     for _ in range(args.warmup):
         run()
     t = _timed(stream, run, args.steps)
-    same = same and bool(np.array_equal(happy.cpu().numpy(), ref[0]) and
-                         np.array_equal(moves.cpu().numpy(), ref[1]))
-    for gi in graphs:
-        check(lib().abm_graph_destroy(gi), "graph_destroy")
+    same = same and all(np.array_equal(a, b) for a, b in zip(got, ref))
     # identity steps (the previous step found every agent happy) read one
     # count and move nothing: only computed steps are charged the 10.8 B
     hf = np.asarray(ref[0])
@@ -638,15 +620,14 @@ def bench_schelling(args) -> dict:
         "ms_per_step": t * 1e3, "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": "i8", "data": "synthetic (seeded grid)",
         "config": {"workload": "schelling_512x512_200steps", "cells": H * W, "sim_steps": S,
-                   "hipgraph": True,
+                   "hipgraph": False,
                    "bench_step": "one full simulation from the seeded grid (state restored "
-                                 "by device copies, then 200 steps)",
-                   "launch": f"{chunk} steps per graph replay; after each the host reads the "
-                             "last step's happy count back, and once a launch ends with every "
-                             "agent happy the steps after the one queued behind it are "
-                             "recorded as identity steps without a launch"},
+                                 "by device copies, then SchellingEngine.run: 200 steps, "
+                                 "records on the host)",
+                   "launch": "a few steps ahead of the GPU; launching stops once a step "
+                             "reports that every agent was happy before it"},
         "replays_identical": same,
-        "steps_launched": launched[-1],
+        "steps_launched": eng.steps_launched,
         "one_graph_ms_per_run": t_one * 1e3,
         "one_graph_note": "all 200 steps as one graph replay (identity steps launched, each "
                           "exiting after reading the previous step's count)",
