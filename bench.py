@@ -439,8 +439,8 @@ def bench_wealth(args) -> dict:
         "cpu_baseline": _wealth_cpu(n, S, args.cpu_runs),
         "roofline": {"bound": "latency", "achieved": None, "peak": None, "unit": None,
                      "frac": None, "traffic": None,
-                     "note": "one workgroup holds the 32 KB/step working set; launch- and "
-                             "barrier-bound, a bandwidth roofline does not apply"},
+                     "note": "100 dependent exchanges in one workgroup's LDS, and four launches; "
+                             "a bandwidth roofline does not apply"},
     }
 
 
