@@ -26,9 +26,9 @@ graph=True)`` turns that loop into graph replays:
    step from a device counter.  It writes agent and env state back into the
    same buffers, and its metrics into row t of a device history.  So a graph
    that holds the captured one several times in a row replays several steps:
-   a run of at least BATCH_MIN_STEPS steps makes one of STEPS_PER_LAUNCH and
-   replays it while that many steps are left (then the one-step graph),
-   which saves most of a graph launch per step.
+   a run of enough steps for its nodes (BATCH_MIN_STEPS, BATCH_NODE_STEPS)
+   makes one of STEPS_PER_LAUNCH and replays it while that many steps are left
+   (then the one-step graph), which saves most of a graph launch per step.
 
 Results are those of the eager loop bit for bit (same kernels, same order).
 Env values that are Python scalars become 0-d device tensors (int32,
@@ -52,12 +52,17 @@ from . import reductions
 from ._lib import MAX_COPY_ITEMS, REDUCE_BATCH_MAX, CopyItem, check, lib, stream_handle
 
 _SCALARS = (bool, int, float)
-# steps per graph launch in runs of at least BATCH_MIN_STEPS steps.  Measured on
-# a 10,000-agent model: 21.5 us a replayed step one a launch, 18.3 eight a launch,
-# 17.7 thirty-two; making the graph of eight costs about 60 us, of thirty-two 200,
-# so that a run of 50 steps gains nothing from eight and one of 100 steps 7%
+# steps per graph launch in runs of at least BATCH_MIN_STEPS steps, and of
+# BATCH_NODE_STEPS for each node of the step.  Measured on a 10,000-agent model of
+# 3 nodes: 21.5 us a replayed step one a launch, 18.3 eight a launch, 17.7
+# thirty-two; making the graph of eight costs about 60 us, of thirty-two 200, so
+# that a run of 50 steps gains nothing from eight and one of 100 steps 7%.  Making
+# it costs some 11 us for each node of the step and saves 3 us a step whatever they
+# are: eight a launch gain or lose at 33 nodes -0.3 ms in 64 steps and 0.4 in 256,
+# at 123 nodes -1.0 in 128 and 0.6 in 512, at 243 -2.3 in 128 and 1.5 in 1,024
 STEPS_PER_LAUNCH = 8
 BATCH_MIN_STEPS = 64
+BATCH_NODE_STEPS = 4
 
 
 class NotReplayable(Exception):
@@ -379,8 +384,8 @@ def _needs_grad(model) -> bool:
 
 def run_graph(model, n: int, between=None) -> Dict[str, Any]:
     """Run up to ``n`` steps of ``model``: steps 1 and 2 eagerly, steps
-    3..n as replays of the captured step (STEPS_PER_LAUNCH a launch in runs of
-    at least BATCH_MIN_STEPS steps while that many are left, else one).  Returns the run's info
+    3..n as replays of the captured step (STEPS_PER_LAUNCH a launch in runs long
+    enough while that many are left, else one).  Returns the run's info
     (``steps_done``: 0 when step 1 fails, 1 when step 2 cannot be replayed,
     2 when the capture is refused, n otherwise; ``mode``, ``reason``, node
     counts).  The model's state, env, keys and history end as after
@@ -411,11 +416,12 @@ def run_graph(model, n: int, between=None) -> Dict[str, Any]:
     if n == 2:
         r.finish(2)
         return {"mode": "eager", "steps": n, "steps_done": 2, "reason": "two steps"}
-    k = STEPS_PER_LAUNCH if n >= BATCH_MIN_STEPS and STEPS_PER_LAUNCH > 1 else 1
-    gk = C.c_void_p()
+    k, gk = 1, C.c_void_p()
     try:
         g = r.capture()
-        if k > 1:
+        nodes = sum(r.info[k] for k in ("kernel_nodes", "memcpy_nodes", "memsets_replaced"))
+        if STEPS_PER_LAUNCH > 1 and n >= max(BATCH_MIN_STEPS, BATCH_NODE_STEPS * nodes):
+            k = STEPS_PER_LAUNCH
             check(lib().abm_graph_repeat(C.c_void_p(g.raw_cuda_graph()), k, C.byref(gk)),
                   "graph_repeat")
     except Exception as e:  # noqa: BLE001

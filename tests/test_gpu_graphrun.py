@@ -575,3 +575,23 @@ def test_results_kept_from_a_step_that_is_not_replayed(J, refused):
     values = [float(v) for v in kept]
     assert values[refused - 1] == values[refused]   # the same step, twice
     assert [float(v) for v in hist["m"]] == values[:refused - 1] + values[refused:]
+
+
+@pytest.mark.parametrize("steps,per_launch", [(127, 1), (128, 8)])
+def test_steps_a_launch_follow_the_nodes_of_the_step(J, monkeypatch, steps, per_launch):
+    """A step of many nodes (the vmapped update) is replayed eight times a launch
+    from BATCH_NODE_STEPS steps a node on; either way the eager loop's results."""
+    from jaxabm_amd import fuse, graphrun
+
+    fuse.enable(False)
+    try:
+        a, b = make_trader(J, n=500), make_trader(J, n=500)
+        assert_same_run(a, b, a.run(5), b.run(5, graph=True))
+        info = b.last_run_info
+        nodes = info["kernel_nodes"] + info["memcpy_nodes"] + info["memsets_replaced"]
+        assert nodes > 16   # above BATCH_MIN_STEPS at the usual 4 steps a node
+        monkeypatch.setattr(graphrun, "BATCH_NODE_STEPS", 128 / nodes)
+        assert_same_run(a, b, a.run(steps), b.run(steps, graph=True))
+        assert b.last_run_info["steps_per_launch"] == per_launch
+    finally:
+        fuse.enable(True)
