@@ -777,6 +777,12 @@ void launch_loss(const abm_deffuant_problem *p, const float *x, hipStream_t s) {
 // as long as 64: 4 of 40,000, 1,366 and 2,567.
 constexpr int64_t kColFewAgents = 3 * 2 * 4 * kColThreads;
 constexpr int32_t kColFewInstances = 16;
+// Populations of a few pairs leave a column's lanes idle, which tells where the
+// instances fill the chip many times over: 64,000 instances of 8 agents, 60 steps,
+// 966 us in columns and 892 in step kernels, of 2 agents 933 and 757, of 32 agents
+// 1,033 and 1,773; 16,000 of 8, 337 and 722.
+constexpr int64_t kColPairAgents = 16;
+constexpr int32_t kColManyInstances = 32768;
 
 // Whether a flagged descriptor takes the column run; the same answer in the
 // forward and the backward of one descriptor.  Either way the same opinions,
@@ -784,7 +790,8 @@ constexpr int32_t kColFewInstances = 16;
 bool column_run(const abm_deffuant_problem *p) {
   if (!(p->flags & ABM_DEFFUANT_COLUMNS) || p->n > kColAgents || p->steps < 1) return false;
   if (p->ckpt_every == 1 ? p->steps < 2 : !p->traj) return false;
-  return !(p->n > kColFewAgents && p->batch <= kColFewInstances && p->batch % 4 != 0);
+  if (p->n > kColFewAgents && p->batch <= kColFewInstances && p->batch % 4 != 0) return false;
+  return p->n > kColPairAgents || p->batch <= kColManyInstances;
 }
 
 ColumnRun column_args(const abm_deffuant_problem *p) {

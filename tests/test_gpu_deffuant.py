@@ -304,11 +304,13 @@ def test_forward_is_refused_under_capture(dm):
 
 
 # the largest population that few instances run in columns and the next, the
-# most instances that count as few, and multiples of four, which never do
+# most instances that count as few, and multiples of four, which never do; the
+# most instances of a few pairs that do
 @pytest.mark.parametrize("n,B,steps,k", [(24576, 2, 5, 2), (24577, 2, 5, 2), (24577, 1, 4, 1),
                                          (24577, 15, 3, 2), (24577, 17, 3, 2), (24577, 4, 3, 2),
-                                         (40832, 17, 4, 2), (40832, 4, 4, 1)])
-def test_column_run_equals_step_kernels_where_few_instances_leave_it(dm, monkeypatch, n, B, steps,
+                                         (40832, 17, 4, 2), (40832, 4, 4, 1), (16, 32768, 3, 2),
+                                         (16, 32769, 3, 2), (17, 32769, 3, 2)])
+def test_column_run_equals_step_kernels_at_its_limits(dm, monkeypatch, n, B, steps,
                                                                      k):
     test_column_run_equals_step_kernels(dm, monkeypatch, n, B, steps, k)
 
