@@ -783,12 +783,12 @@ void launch_loss(const abm_deffuant_problem *p, const float *x, hipStream_t s) {
 // as long as 64: 4 of 40,000, 1,366 and 2,567.
 constexpr int64_t kColFewAgents = 3 * 2 * 4 * kColThreads;
 constexpr int32_t kColFewInstances = 16;
-// Populations of a few pairs leave a column's lanes idle, which tells where the
-// instances fill the chip many times over: 64,000 instances of 8 agents, 60 steps,
-// 966 us in columns and 892 in step kernels, of 2 agents 933 and 757, of 32 agents
-// 1,033 and 1,773; 16,000 of 8, 337 and 722.
-constexpr int64_t kColPairAgents = 16;
-constexpr int32_t kColManyInstances = 32768;
+// Populations of up to four pairs leave a column's lanes idle, which tells once
+// the instances fill the chip seven times over (8,192 wavefronts): 64,000 instances
+// of 8 agents, 60 steps, 914 us in columns and 811 in step kernels, of 2 agents 884
+// and 669, of 32 agents 963 and 1,719; 32,000 of 8, 538 and 835.
+constexpr int64_t kColPairAgents = 8;
+constexpr int32_t kColManyInstances = 7 * 8192;
 
 // Whether a flagged descriptor takes the column run; the same answer in the
 // forward and the backward of one descriptor.  Either way the same opinions,

@@ -308,10 +308,9 @@ def test_forward_is_refused_under_capture(dm):
 # most instances of a few pairs that do
 @pytest.mark.parametrize("n,B,steps,k", [(24576, 2, 5, 2), (24577, 2, 5, 2), (24577, 1, 4, 1),
                                          (24577, 15, 3, 2), (24577, 17, 3, 2), (24577, 4, 3, 2),
-                                         (40832, 17, 4, 2), (40832, 4, 4, 1), (16, 32768, 3, 2),
-                                         (16, 32769, 3, 2), (17, 32769, 3, 2)])
-def test_column_run_equals_step_kernels_at_its_limits(dm, monkeypatch, n, B, steps,
-                                                                     k):
+                                         (40832, 17, 4, 2), (40832, 4, 4, 1), (8, 57344, 3, 2),
+                                         (8, 57345, 3, 2), (9, 57345, 3, 2)])
+def test_column_run_equals_step_kernels_at_its_limits(dm, monkeypatch, n, B, steps, k):
     test_column_run_equals_step_kernels(dm, monkeypatch, n, B, steps, k)
 
 
