@@ -262,13 +262,12 @@ int abm_wealth_init_host_key(const uint32_t init_key[2], int64_t n, float *x, fl
                              int mode, void *stream);
 /* Runs every instance of the device array insts[count] for its steps.  max_n:
  * the largest n in the table (0 if unknown).  With draws, an instance's draws
- * are computed first by a grid-wide kernel; if n <= max_n
- * <= 40,000 (or n <= 1,024), one workgroup then runs the exchange out of LDS
- * (leaving each step's wealth in place of its targets in draws) while others
- * walk the positions, and the records of all steps are taken at the end.
- * Otherwise one workgroup runs the whole instance, out of LDS when 0 < n <=
- * max_n <= 8000 (20 bytes per agent of dynamic LDS), else on its global
- * buffers.  Same results either way. */
+ * are computed first by a grid-wide kernel; if n <= max_n <= 40,000 (or n <=
+ * 1,024), one workgroup then runs the exchange out of LDS (leaving each step's
+ * wealth in place of its targets in draws) while others walk the positions, and
+ * the records of all steps are taken at the end.  Otherwise one workgroup runs
+ * the whole instance, out of LDS when 0 < n <= max_n <= 8000 (20 bytes per agent
+ * of dynamic LDS), else on its global buffers.  Same results either way. */
 int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t max_n, int mode,
                          void *stream);
 /* One instance across the whole GPU, for large n.  inst: the descriptor in
@@ -277,10 +276,10 @@ int abm_wealth_run_batch(const abm_wealth_inst *insts, int32_t count, int64_t ma
  * applies the previous step's exchange to its agents, then draws and applies
  * this step's walk and gives its units, while one workgroup records the step
  * before.  Otherwise two launches per step (draws, walk and exchange atomics
- * with the previous step recorded; then the exchange applied and counted).  acc: device scratch uint32[ABM_WEALTH_GRID_ACC_WORDS]
- * (the total and 16 copies of the 64 smallest histogram bins, so that no
- * word takes an atomic from every workgroup).  Same results as
- * abm_wealth_run_batch. */
+ * with the previous step recorded; then the exchange applied and counted).
+ * acc: device scratch uint32[ABM_WEALTH_GRID_ACC_WORDS] (the total and 16 copies
+ * of the 64 smallest histogram bins, so that no word takes an atomic from every
+ * workgroup).  Same results as abm_wealth_run_batch. */
 #define ABM_WEALTH_GRID_ACC_WORDS 1026
 int abm_wealth_run_grid(const abm_wealth_inst *inst, uint32_t *acc, int mode, void *stream);
 
@@ -571,7 +570,8 @@ typedef struct abm_reduce_item {
 int abm_reduce_batch(const abm_reduce_item *items, int32_t count, void *stream);
 /* abm_reduce_batch and abm_commit_step in one launch.  Items from n_early on
  * (of n_items) copy results: their src is the out of a reduction.  No item's
- * destination may overlap a reduction's input.  One node of a replayed step of JaxModel.run(graph=True). */
+ * destination may overlap a reduction's input.  One node of a replayed step of
+ * JaxModel.run(graph=True). */
 int abm_reduce_commit_step(const abm_reduce_item *red, int32_t n_red, const abm_copy_item *items,
                            int32_t n_early, int32_t n_items, int64_t *row, int32_t *ts,
                            uint32_t *done, const uint32_t *key_table, int64_t key_rows,

@@ -948,8 +948,9 @@ int abm_deffuant_backward(const abm_deffuant_problem *p, void *stream) {
     if (int rc = column_lds_attr()) return rc;
     const bool wide = nblocks(n, 64) * (int64_t)nblocks(p->batch, 16) >= 1024;
     hipLaunchKernelGGL(wide ? k_deffuant_lambda_columns<64> : k_deffuant_lambda_columns<16>,
-                       dim3(nblocks(n, wide ? 64 : 16), nblocks(p->batch, 16)), dim3(256), 0, s, final_x, n, p->batch, (const double *)p->stats,
-                       (const double *)p->coef, p->lam);
+                       dim3(nblocks(n, wide ? 64 : 16), nblocks(p->batch, 16)), dim3(256), 0, s,
+                       final_x, n, p->batch, (const double *)p->stats, (const double *)p->coef,
+                       p->lam);
     hipLaunchKernelGGL(column_backward(n), dim3((unsigned)p->batch), dim3(column_threads(n)),
                        (size_t)n * (column_both(n) ? 8 : 4), s, column_args(p));
     ABM_LAUNCH_CHECK("abm_deffuant_backward");

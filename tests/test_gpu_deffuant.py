@@ -248,7 +248,8 @@ def test_batch_size_does_not_change_an_instance(dm):
 
 # Column runs against the step kernels: pairs per thread 1 and 4 (1,024 and
 # 1,025 pairs), opinions and adjoints both in LDS or in turn (20,416 agents and
-# above), the largest column and the next size (step kernels on both sides),
+# above), the largest column's size and the next (step kernels on both sides for
+# these two instances; in columns below, at the limits),
 # whole lines of instances and a rest, every tape layout (k = 1, 2, one
 # segment, a last segment of one step), one step.
 @pytest.mark.parametrize("n,B,steps,k", [(2, 1, 5, 2), (3, 2, 4, 1), (65, 5, 7, 3),
